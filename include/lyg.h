@@ -234,7 +234,7 @@ int32_t lyg_fill_batch(lyg_ctx* ctx, const lyg_batch_in* in, const lyg_fill_opti
  * its half width is line_width * attributes[width_attribute] * 0.5; curves interpolate the
  * widths of their endpoints.  Positions agree with lyon's within float rounding of asin /
  * cos / sin; status as lyg_stroke_path / lyg_stroke_batch, plus LYG_ERR_NO_SPACE for a path
- * with a curve of more than 4,194,304 flattened points.  One GPU lane strokes one path.
+ * with a curve of more than 4,194,304 flattened points.
  * out_attributes (optional, n_attributes floats per output vertex, vertex_capacity rows):
  * StrokeVertex::interpolated_attributes (stroke.rs:2728-2746) of every vertex — its
  * source endpoint's row, or on a curve a*(1-t) + b*t of the curve's two endpoint rows. */

@@ -51,6 +51,9 @@ struct lyg_ctx {
     uint64_t last_stroke_items = 0;       // items of the last split stroke batch
     uint32_t last_stroke_again = 0;       // its paths walked again whole
     DevBuf st_items, st_heads, st_spec, st_end, st_parts, st_parts_off;
+    // variable-width stroke: per-path plan, kept points, their flags and vertex sources, side
+    // lines, windows, sub-path ends, candidate lists
+    DevBuf vw_path, vw_rec, vw_flags, vw_src, vw_att, vw_win, vw_tails, vw_lists;
     // fill: one stream per size class of a round, and the events that join them
     hipStream_t class_stream[8] = {};
     hipEvent_t class_ev[25] = {};  // one per fill launch (size class x form) + 1

@@ -196,6 +196,62 @@ struct StrokeVWLaunch {
     const float* attrs;
     uint32_t n_attrs;
     float* out_attrs;
+    // the paths to walk: list[0 .. *n_list) (null: all)
+    const uint32_t* list;
+    const uint32_t* n_list;
+};
+
+// Joins per window of the parallel variable-width stroke.
+static constexpr uint32_t VW_WINDOW = 63u;
+// The end of a sub-path of the parallel variable-width stroke.
+struct VWTail {
+    uint32_t path, first, count;  // its points: first .. first + count of the path's kept ones
+    uint32_t flags;               // 1: closed, 2: a point was dropped after the first
+    uint32_t nv, nt;              // what its end emits
+    // set by the emit pass, in vertices / triangles of the path: where its end starts, the
+    // first vertices of the joins at its second and at its last but one buffered point
+    uint32_t v_at, t_at, f1_base, p_base;
+};
+// Parallel variable-width stroke (stroke_vw.hip).
+struct VWPar {
+    PathBatchDev in;
+    const lyg_stroke_options* opts;
+    uint32_t opts_stride;
+    const float* widths;
+    uint32_t widths_stride;
+    const float* attrs;
+    uint32_t n_attrs;
+    float* out_attrs;
+    // per path: the plan's counts and their offsets (n + 1), the kept points, 0 parallel /
+    // 1 serial / 2 nothing to walk, and the results
+    uint32_t *raw_n, *win_n, *tail_n, *att_cap_n;
+    const uint32_t *raw_off, *win_off, *tail_off, *att_off;
+    uint32_t *kept_n, *path_mode, *path_status, *path_nv, *path_ni;
+    // per kept point (a path's at raw_off): x, y, half width, running length; flags; vertex
+    // source (null without vertex attributes)
+    float* rec;
+    uint8_t* pflags;
+    float* src_t;
+    uint32_t* src_id;
+    // edges with side lines: (slot, point) pairs in any order, four floats per slot
+    uint32_t* att_pair;
+    float* att_n;
+    // per window
+    uint32_t *win_att, *win_nv, *win_ni;
+    const uint32_t *win_voff, *win_ioff;
+    uint32_t n_windows;
+    VWTail* tails;
+    uint32_t n_tails;
+    uint32_t *slow_list, *cands, *dirty;
+    uint32_t cand_cap, dirty_cap;
+    // [0] edges with side lines, [1] serial paths, [2] candidates, [3] windows to count
+    // again, [4] a list overflowed
+    uint32_t* ctr;
+    const uint32_t *vtx_off, *idx_off;
+    float* out_vertices;
+    uint32_t* out_indices;
+    uint32_t vertex_offset;
+    uint32_t* err;
 };
 
 struct FlattenLaunch {

@@ -375,7 +375,7 @@ struct ArcJob {
     uint32_t va, vb, n, first_id;
     uint32_t* tri;   // index slots of the arc's first triangle
     uint32_t ileft;  // index slots left in the path from `tri`
-    uint32_t pad;
+    float hw;        // the join's half width
 };
 struct ArcJobs {  // at most one arc per side of a lane's join
     ArcJob sp, sn;
@@ -407,7 +407,7 @@ __device__ __forceinline__ void round_join_side(const JInfo& J, const SParams& p
         a.first_id = s.vid;
         a.tri = s.iout + 3u * s.ni;
         a.ileft = s.ileft > 3u * s.ni ? s.ileft - 3u * s.ni : 0u;
-        a.pad = 0;
+        a.hw = p.hw;
         if (side == SP) {
             jobs->sp = a;
             jobs->has_sp = true;
@@ -660,6 +660,8 @@ __device__ __forceinline__ void join_emit(JInfo& J, const EPD& prev, bool with_e
 // its upper half): the same midpoints, ids first_id + p and triangles (va, id, vb) as
 // the serial recursion.  `jl` (128 jobs) and `xl`, `cl` (64 each) are the wave's LDS;
 // `s` is the calling lane's sink (every lane of the wave writes into the same path).
+// JOB_HW: the arcs' half widths are their own (variable width), else the path's `hw`.
+template <bool JOB_HW = false>
 __device__ __forceinline__ void emit_arcs(const ArcJobs& aj, const Sink& s, float hw, ArcJob* jl,
                                           uint32_t* xl, uint32_t* cl) {
     const int l = lane_id();
@@ -711,7 +713,8 @@ __device__ __forceinline__ void emit_arcs(const ArcJobs& aj, const Sink& s, floa
         }
         Sink w = s;  // this lane's copy of the path's sink, placed at the node
         w.vid = a.first_id + p;
-        const uint32_t id = sink_sv(w, mk(a.cx, a.cy), mk(t_cos(mid), t_sin(mid)), hw);
+        const uint32_t id = sink_sv(w, mk(a.cx, a.cy), mk(t_cos(mid), t_sin(mid)),
+                                    JOB_HW ? a.hw : hw);
         if (3u * p + 3u <= a.ileft) {
             uint32_t* o = a.tri + 3u * p;
             o[0] = va;

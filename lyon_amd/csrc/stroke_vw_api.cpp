@@ -1,5 +1,6 @@
-// Host side of the variable-width stroke (StrokeOptions::variable_line_width): a count
-// launch (one lane per path), the two offset scans, the output check, an emit launch.
+// Host side of the variable-width stroke (StrokeOptions::variable_line_width): the plan and
+// its scans, the count, the offset scans, the output check, the emit launches; the serial
+// kernel (one lane per path) for the paths the parallel form leaves out.
 #include <algorithm>
 #include <vector>
 
@@ -10,6 +11,11 @@
 extern "C" {
 hipError_t lyg_launch_stroke_vw(const lyg::StrokeVWLaunch* L, int emit, int grid,
                                 hipStream_t s);
+hipError_t lyg_launch_vw_plan(const lyg::VWPar* P, int grid, hipStream_t s);
+hipError_t lyg_launch_vw_count(const lyg::VWPar* P, int grid_paths, int grid_win, uint32_t chunk,
+                               hipStream_t s);
+hipError_t lyg_launch_vw_totals(const lyg::VWPar* P, hipStream_t s);
+hipError_t lyg_launch_vw_emit(const lyg::VWPar* P, int grid_win, uint32_t chunk, hipStream_t s);
 hipError_t lyg_launch_fill_u32(uint32_t* p, uint32_t n, uint32_t v, hipStream_t s);
 }
 
@@ -19,12 +25,131 @@ bool valid_opts(const lyg_stroke_options& o) {
     return o.start_cap <= 2 && o.end_cap <= 2 && o.line_join <= 3;
 }
 
+// Launch shape of the window kernels.
+struct VWShape {
+    int grid_paths, grid;
+    uint32_t chunk;  // consecutive windows per wave and turn
+};
+
+// Points of a batch beyond which it goes to the serial kernel (the parallel form keeps 17
+// bytes per flattened point, the output takes about 40).
+constexpr uint64_t VW_MAX_POINTS = 1ull << 30;
+
+// The plan and the parallel form's memory.  LYG_ERR_NO_SPACE: the batch goes to the serial
+// kernel (too many points, or no device memory for them).
+int32_t vw_plan(lyg_ctx* c, const lyg::StrokeVWLaunch& L, uint32_t n, bool want_attrs,
+                lyg::VWPar* out, VWShape* sh) {
+    hipStream_t s = c->stream;
+    lyg::VWPar P{};
+    P.in = L.in;
+    P.opts = L.opts;
+    P.opts_stride = L.opts_stride;
+    P.widths = L.widths;
+    P.widths_stride = L.widths_stride;
+    P.attrs = L.attrs;
+    P.n_attrs = L.n_attrs;
+    P.path_status = L.path_status;
+    P.path_nv = L.path_nv;
+    P.path_ni = L.path_ni;
+    P.err = L.err;
+    if (!ensure(c, c->vw_path, 4ull * (11ull * n + 4) + 64)) return LYG_ERR_DEVICE;
+    uint32_t* u = as<uint32_t>(c->vw_path);
+    auto take = [&](size_t k) {
+        uint32_t* p = u;
+        u += k;
+        return p;
+    };
+    P.ctr = take(16);
+    P.raw_n = take(n);
+    P.win_n = take(n);
+    P.tail_n = take(n);
+    P.att_cap_n = take(n);
+    P.kept_n = take(n);
+    P.path_mode = take(n);
+    P.slow_list = take(n);
+    uint32_t* off[4];
+    for (uint32_t*& o : off) o = take((size_t)n + 1);
+    P.raw_off = off[0];
+    P.win_off = off[1];
+    P.tail_off = off[2];
+    P.att_off = off[3];
+    const uint32_t* cnt[4] = {P.raw_n, P.win_n, P.tail_n, P.att_cap_n};
+    sh->grid_paths = (int)std::min<uint32_t>(n, (uint32_t)std::max(1, c->cu_count) * 32u);
+    if (!check(c, lyg_launch_fill_u32(P.ctr, 16, 0, s), "reset") ||
+        !check(c, lyg_launch_vw_plan(&P, sh->grid_paths, s), "stroke vw plan"))
+        return LYG_ERR_DEVICE;
+    for (int k = 0; k < 4; ++k)
+        if (!check(c, ctx_scan(c, cnt[k], n, off[k], c->d_totals + 2 + k, P.ctr + 8, s), "scan"))
+            return LYG_ERR_DEVICE;
+    uint64_t* h = reinterpret_cast<uint64_t*>(c->h_pinned);
+    if (!check(c, hipMemcpyAsync(h, c->d_totals + 2, 32, hipMemcpyDeviceToHost, s), "D2H") ||
+        !check(c, hipStreamSynchronize(s), "sync"))
+        return LYG_ERR_DEVICE;
+    const uint64_t raw = h[0], win = h[1], tails = h[2], att = h[3];
+    if (raw > VW_MAX_POINTS || tails > VW_MAX_POINTS || att > VW_MAX_POINTS)
+        return LYG_ERR_NO_SPACE;
+    P.n_windows = (uint32_t)win;
+    P.n_tails = (uint32_t)tails;
+    P.cand_cap = (uint32_t)std::max<uint64_t>(4096, win);
+    P.dirty_cap = 4u * P.cand_cap;
+    const bool src = want_attrs;
+    if (!ensure(c, c->vw_rec, 16 * raw) || !ensure(c, c->vw_flags, raw) ||
+        (src && !ensure(c, c->vw_src, 12 * raw)) || !ensure(c, c->vw_att, 24 * att) ||
+        !ensure(c, c->vw_win, 4 * (5 * win + 2)) ||
+        !ensure(c, c->vw_tails, sizeof(lyg::VWTail) * tails) ||
+        !ensure(c, c->vw_lists, 4ull * (2ull * P.cand_cap + P.dirty_cap))) {
+        (void)hipGetLastError();  // the serial kernel needs none of it
+        return LYG_ERR_NO_SPACE;
+    }
+    P.rec = as<float>(c->vw_rec);
+    P.pflags = as<uint8_t>(c->vw_flags);
+    if (src) {
+        P.src_t = as<float>(c->vw_src);
+        P.src_id = as<uint32_t>(c->vw_src) + raw;
+    }
+    P.att_n = as<float>(c->vw_att);
+    P.att_pair = as<uint32_t>(c->vw_att) + 4 * att;
+    u = as<uint32_t>(c->vw_win);
+    P.win_att = take(win);
+    P.win_nv = take(win);
+    P.win_ni = take(win);
+    P.win_voff = take(win + 1);
+    P.win_ioff = take(win + 1);
+    P.tails = as<lyg::VWTail>(c->vw_tails);
+    P.cands = as<uint32_t>(c->vw_lists);
+    P.dirty = P.cands + 2ull * P.cand_cap;
+    // windows: 8 resident blocks of four waves per CU, a few consecutive windows per wave and
+    // turn (they share the search for their path)
+    const uint32_t blocks = (uint32_t)std::max(1, c->cu_count) * 8u;
+    sh->chunk = std::min<uint32_t>(16u, std::max<uint32_t>(1u, P.n_windows / (blocks * 16u)));
+    const uint64_t turns = (win + 4ull * sh->chunk - 1) / (4ull * sh->chunk);
+    sh->grid = (int)std::max<uint64_t>(1, std::min<uint64_t>(turns, blocks));
+    *out = P;
+    return LYG_OK;
+}
+
+// Counts of the planned batch into path_nv / path_ni (of the paths not left to the serial
+// kernel).
+int32_t vw_count(lyg_ctx* c, lyg::VWPar& P, const VWShape& sh) {
+    hipStream_t s = c->stream;
+    uint32_t* wv = const_cast<uint32_t*>(P.win_voff);
+    uint32_t* wi = const_cast<uint32_t*>(P.win_ioff);
+    if (!check(c, lyg_launch_vw_count(&P, sh.grid_paths, sh.grid, sh.chunk, s),
+               "stroke vw count") ||
+        !check(c, ctx_scan(c, P.win_nv, P.n_windows, wv, c->d_totals + 6, P.ctr + 8, s), "scan") ||
+        !check(c, ctx_scan(c, P.win_ni, P.n_windows, wi, c->d_totals + 7, P.ctr + 8, s), "scan") ||
+        !check(c, lyg_launch_vw_totals(&P, s), "stroke vw totals"))
+        return LYG_ERR_DEVICE;
+    return LYG_OK;
+}
+
 // Runs the batch `L` (inputs, options, widths set); offsets go to vtx_off / idx_off (n + 1
-// each), per-path statuses to c->f_status; `alloc` sets the output arrays once the totals
+// each), per-path statuses to c->f_status; want_attrs: vertex attributes will be asked for
+// (L.out_attrs is set by then); `alloc` sets the output arrays once the totals
 // are known.
-int32_t stroke_vw_run(lyg_ctx* c, lyg::StrokeVWLaunch& L, uint32_t* vtx_off, uint32_t* idx_off,
-                      uint32_t vertex_offset, const lygi::OutAlloc& alloc, uint64_t* tv,
-                      uint64_t* ti, std::vector<uint32_t>* status) {
+int32_t stroke_vw_run(lyg_ctx* c, lyg::StrokeVWLaunch& L, bool want_attrs, uint32_t* vtx_off,
+                      uint32_t* idx_off, uint32_t vertex_offset, const lygi::OutAlloc& alloc,
+                      uint64_t* tv, uint64_t* ti, std::vector<uint32_t>* status) {
     const uint32_t n = L.in.n_paths;
     hipStream_t s = c->stream;
     if (!ensure(c, c->counts_v, 4ull * n) || !ensure(c, c->counts_i, 4ull * n) ||
@@ -35,28 +160,46 @@ int32_t stroke_vw_run(lyg_ctx* c, lyg::StrokeVWLaunch& L, uint32_t* vtx_off, uin
     L.path_status = as<uint32_t>(c->f_status);
     L.vertex_offset = vertex_offset;
     L.err = c->d_counters + 5;
-    // about six resident waves per SIMD (four SIMDs per CU), each with as few paths as
-    // fill them
+    lyg::VWPar P{};
+    VWShape sh{};
+    int32_t st = vw_plan(c, L, n, want_attrs, &P, &sh);
+    if (st == LYG_OK) st = vw_count(c, P, sh);
+    if (st == LYG_ERR_DEVICE) return st;
+    bool par = st == LYG_OK;
+    // The serial kernel over all paths: about six resident waves per SIMD (four SIMDs per
+    // CU), each with as few paths as fill them; over the paths left to it: one path a wave.
     const uint32_t slots = (uint32_t)std::max(1, c->cu_count) * 4u * 6u;
-    L.paths_per_wave = std::min<uint32_t>(64u, std::max<uint32_t>(1u, (n + slots - 1) / slots));
-    const int grid =
-        (int)std::min<uint32_t>((n + L.paths_per_wave - 1) / L.paths_per_wave, 1u << 20);
-    if (!check(c, lyg_launch_fill_u32(c->d_counters + 4, 2, 0, s), "reset") ||
-        !check(c, lyg_launch_stroke_vw(&L, 0, grid, s), "stroke vw count") ||
-        !check(c, ctx_scan(c, L.path_nv, n, vtx_off, c->d_totals + 0, c->d_counters + 4, s),
-               "scan") ||
-        !check(c, ctx_scan(c, L.path_ni, n, idx_off, c->d_totals + 1, c->d_counters + 4, s),
-               "scan"))
-        return LYG_ERR_DEVICE;
+    int grid = 0;
     uint64_t* h = reinterpret_cast<uint64_t*>(c->h_pinned);
     status->assign(n, 0);
-    if (!check(c, hipMemcpyAsync(h, c->d_totals, 16, hipMemcpyDeviceToHost, s), "D2H") ||
-        !check(c, hipMemcpyAsync(h + 2, c->d_counters + 4, 4, hipMemcpyDeviceToHost, s), "D2H") ||
-        !check(c, hipMemcpyAsync(status->data(), L.path_status, 4ull * n, hipMemcpyDeviceToHost,
-                                 s),
-               "D2H") ||
-        !check(c, hipStreamSynchronize(s), "sync"))
-        return LYG_ERR_DEVICE;
+    for (;;) {
+        L.list = par ? P.slow_list : nullptr;
+        L.n_list = par ? P.ctr + 1 : nullptr;
+        L.paths_per_wave =
+            par ? 1u : std::min<uint32_t>(64u, std::max<uint32_t>(1u, (n + slots - 1) / slots));
+        grid = par ? (int)std::min(n, slots)
+                   : (int)std::min<uint32_t>((n + L.paths_per_wave - 1) / L.paths_per_wave,
+                                             1u << 20);
+        h[3] = 0;
+        if (!check(c, lyg_launch_fill_u32(c->d_counters + 4, 2, 0, s), "reset") ||
+            !check(c, lyg_launch_stroke_vw(&L, 0, grid, s), "stroke vw count") ||
+            !check(c, ctx_scan(c, L.path_nv, n, vtx_off, c->d_totals + 0, c->d_counters + 4, s),
+                   "scan") ||
+            !check(c, ctx_scan(c, L.path_ni, n, idx_off, c->d_totals + 1, c->d_counters + 4, s),
+                   "scan") ||
+            !check(c, hipMemcpyAsync(h, c->d_totals, 16, hipMemcpyDeviceToHost, s), "D2H") ||
+            !check(c, hipMemcpyAsync(h + 2, c->d_counters + 4, 4, hipMemcpyDeviceToHost, s),
+                   "D2H") ||
+            (par && !check(c, hipMemcpyAsync(h + 3, P.ctr + 4, 4, hipMemcpyDeviceToHost, s),
+                           "D2H")) ||
+            !check(c, hipMemcpyAsync(status->data(), L.path_status, 4ull * n,
+                                     hipMemcpyDeviceToHost, s),
+                   "D2H") ||
+            !check(c, hipStreamSynchronize(s), "sync"))
+            return LYG_ERR_DEVICE;
+        if (!(uint32_t)h[3]) break;
+        par = false;  // more joins that may fold back than the lists hold
+    }
     *tv = h[0];
     *ti = h[1];
     if ((uint32_t)h[2]) return LYG_ERR_TOO_MANY_VERTICES;
@@ -65,12 +208,22 @@ int32_t stroke_vw_run(lyg_ctx* c, lyg::StrokeVWLaunch& L, uint32_t* vtx_off, uin
         return LYG_ERR_TOO_MANY_VERTICES;
     float* ov = nullptr;
     uint32_t* oi = nullptr;
-    int32_t st = alloc(*tv, *ti, &ov, &oi);
+    st = alloc(*tv, *ti, &ov, &oi);
     if (st != LYG_OK) return st;
     L.vtx_off = vtx_off;
     L.idx_off = idx_off;
     L.out_vertices = ov;
     L.out_indices = oi;
+    if (par) {
+        P.vtx_off = vtx_off;
+        P.idx_off = idx_off;
+        P.out_vertices = ov;
+        P.out_indices = oi;
+        P.out_attrs = L.out_attrs;
+        P.vertex_offset = vertex_offset;
+        if (!check(c, lyg_launch_vw_emit(&P, sh.grid, sh.chunk, s), "stroke vw emit"))
+            return LYG_ERR_DEVICE;
+    }
     uint32_t err = 0;
     if (!check(c, lyg_launch_stroke_vw(&L, 1, grid, s), "stroke vw emit") ||
         !check(c, hipMemcpyAsync(&err, c->d_counters + 5, 4, hipMemcpyDeviceToHost, s), "D2H") ||
@@ -121,7 +274,7 @@ int32_t lyg_stroke_batch_vw(lyg_ctx* c, const lyg_batch_in* in, const float* att
     uint64_t tv = 0, ti = 0;
     std::vector<uint32_t> status;
     int32_t st = stroke_vw_run(
-        c, L, out->path_vertex_offsets, out->path_index_offsets, out->vertex_offset,
+        c, L, out_attributes != nullptr, out->path_vertex_offsets, out->path_index_offsets, out->vertex_offset,
         [&](uint64_t nv, uint64_t ni, float** v, uint32_t** i) -> int32_t {
             if (nv > out->vertex_capacity || ni > out->index_capacity) return LYG_ERR_CAPACITY;
             *v = out->vertices;
@@ -189,7 +342,7 @@ int32_t lyg_stroke_path_vw(lyg_ctx* c, const lyg_path_view* path, const float* a
     uint64_t tv = 0, ti = 0;
     std::vector<uint32_t> status;
     int32_t st = stroke_vw_run(
-        c, L, as<uint32_t>(c->offs_v), as<uint32_t>(c->offs_i), out->vertex_offset,
+        c, L, out_attributes != nullptr, as<uint32_t>(c->offs_v), as<uint32_t>(c->offs_i), out->vertex_offset,
         [&](uint64_t nv, uint64_t ni, float** v, uint32_t** i) -> int32_t {
             if (nv > out->vertex_capacity || ni > out->index_capacity) {
                 out->n_vertices = (uint32_t)nv;

@@ -161,6 +161,44 @@ def test_batch_matches_the_oracle(seed):
     assert exact >= 0.97 * n
 
 
+@pytest.mark.parametrize("join", [LineJoin.Miter, LineJoin.MiterClip, LineJoin.Round])
+@pytest.mark.parametrize("closed", [False, True])
+def test_sub_paths_around_the_window_size(join, closed):
+    """Sub-paths of 1-5, 61-66 and 125-129 points (a window holds 63 joins and repeats the
+    one before), one per path and several in a path, with repeated points that are dropped,
+    and curves whose joins may fold back (widths that change by more than an edge)."""
+    rng = np.random.default_rng(9)
+    paths = []
+    for counts in ([1], [2], [3], [4], [5], [61], [62], [63], [64], [65], [66], [125], [126],
+                   [127], [128], [129], [62, 1, 64], [63, 63, 2], [5, 126, 3]):
+        b = PathBuilder(1)
+        for k in counts:
+            pts = rng.uniform(0, 300, (k, 2)).round(1)
+            b.begin(tuple(pts[0]), [rng.uniform(0.2, 2)])
+            for q in pts[1:]:
+                b.line_to(tuple(q), [rng.uniform(0.2, 2)])
+                if rng.random() < 0.1:
+                    b.line_to(tuple(q), [1.0])
+            b.end(closed)
+        paths.append(b.build())
+    for _ in range(60):
+        b = PathBuilder(1)
+        b.begin((0, 0), [1.0])
+        for _ in range(8):
+            b.cubic_bezier_to(*[tuple(q) for q in rng.uniform(0, 60, (3, 2))],
+                              [rng.uniform(0.2, 12)])
+        b.end(closed)
+        paths.append(b.build())
+    same = 0
+    for path in paths:
+        opts = StrokeOptions(line_width=2.0, line_join=join, start_cap=LineCap.Round,
+                             end_cap=LineCap.Square, tolerance=0.05, variable_line_width=0)
+        v, i = gpu_vw(path, opts)
+        rv, ri = ref_vw(path, opts)
+        same += np.array_equal(i, ri) and close_enough(v, rv, 300.0)
+    assert same >= 0.97 * len(paths), same
+
+
 def test_batch_equals_plain_calls():
     n = 24
     batch, opts, widths = random_batch(n, 3)
