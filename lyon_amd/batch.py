@@ -390,10 +390,11 @@ def set_stroke_split(windows_per_part: int = 64):
 
 
 def set_fill_lds_resident(enabled=True):
-    """Placement of the batched fill sweep's arrays (lyg_ctx_set_fill_lds_resident): by
-    default the first round keeps every hot array of a path that fits 150 KiB in LDS;
-    False: arrays start in LDS and move to global memory as they grow; an int > 1 divides
-    the LDS capacities by it (paths outgrow them and are swept again).  Same output."""
+    """Where the fill sweep keeps its state (lyg_ctx_set_fill_lds_resident): by default a
+    path's active edges in registers and its pending intersections in LDS, as far as they
+    are estimated to fit; False: in arrays that start in LDS and move to global memory as
+    they grow; an int > 1 divides the first's capacities by it (paths outgrow them and are
+    swept again).  Same output."""
     v = int(enabled) if not isinstance(enabled, bool) else (1 if enabled else 0)
     st = B.lib().lyg_ctx_set_fill_lds_resident(_Ctx.get(), v)
     if st != 0:

@@ -2,11 +2,12 @@
 //
 // A fill call runs in three steps on the context's stream:
 //   1. fill_bound_kernel writes an upper bound of every path's sweep events;
-//   2. rounds of fill_sweep_kernel: each path is swept by one wave into a staging area
-//      sized from its bound.  Paths are grouped into size classes so that the per-wave
-//      working memory of a launch fits its largest path; a path that outgrows its
-//      staging or working memory ends with a retry status and is swept again in the next
-//      round with four times the room;
+//   2. rounds of sweeps: each path is swept by one wave into a staging area sized from its
+//      bound, in the first round with its active edges in registers (fill_reg.hip), later or
+//      beyond 1,024 of them over arrays (fill.hip).  Paths are grouped into size classes so
+//      that the per-wave working memory of a launch fits its largest path; a path that
+//      outgrows its staging, registers or working memory ends with a retry status and is
+//      swept again in the next round with four times the room;
 //   3. an exclusive scan over the per-path vertex/index counts, then fill_copy_kernel
 //      moves every round's staged output to its final place, rebasing the indices.
 #include <algorithm>
@@ -22,10 +23,10 @@
 extern "C" {
 size_t lyg_fill_work_bytes(const lyg::fillk::FillCaps* caps, size_t hot_bytes);
 int lyg_fill_occupancy(uint32_t waves_per_block, uint32_t hot_bytes);
-int lyg_fill_occupancy_form(uint32_t waves_per_block, uint32_t hot_bytes, int form);
-size_t lyg_fill_lds_bytes(const lyg::fillk::FillCaps* lc);
+int lyg_fill_reg_occupancy(uint32_t chunks, uint32_t rows);
+hipError_t lyg_launch_fill_reg(const lyg::FillLaunch* L, int grid, hipStream_t s);
 hipError_t lyg_launch_fill_bound(const lyg::FillLaunch* L, uint32_t n, uint32_t* bound,
-                                 hipStream_t s);
+                                 uint32_t* degree, hipStream_t s);
 hipError_t lyg_launch_fill_sweep(const lyg::FillLaunch* L, int grid, hipStream_t s);
 size_t lyg_fill_box_bytes();
 hipError_t lyg_launch_fill_inter(const lyg::FillLaunch* L, uint32_t n, void* boxes, uint32_t* inter,
@@ -49,51 +50,45 @@ constexpr uint64_t MAX_PATH_EVENTS = 1ull << 27;     // larger paths: LYG_ERR_NO
 constexpr size_t WORK_BUDGET = 16ull << 30;          // working memory of one round
 constexpr size_t STAGE_BUDGET = 64ull << 30;         // staging memory of one round
 constexpr int MAX_CLASSES = 8;
-constexpr int N_FORMS = 3;  // placement forms of the sweep's hot arrays (FillLaunch::form)
-constexpr int FORM_MIGRATE = 0, FORM_LDS = 1, FORM_PART = 2;
+// How a path is swept: over arrays that start in LDS and move to global memory as they grow,
+// or with its active edges in registers (2, 5 or 16 sets of 64).
+constexpr int N_FORMS = 4;
+constexpr int FORM_ARRAYS = 0;
+constexpr uint32_t REG_CHUNKS[N_FORMS] = {0, 2, 5, 16};
+constexpr uint32_t REG_MAX_ROWS = 44;  // pending events per column: 66 KiB of LDS
 constexpr int MAX_LAUNCHES = N_FORMS * MAX_CLASSES;
+constexpr int N_GRAPH_COUNTERS = 2 * MAX_LAUNCHES;  // a launch and the sweep after it
 constexpr size_t CLASS_STREAMS = 3;
-// The first round sweeps a path with all its hot arrays in LDS when their estimate fits
-// this many bytes per wave, else with the per-event ones in LDS when those fit, else in
-// the migrating form: three waves per CU (a CU has 160 KiB; the kernel's own LDS takes
-// 4 KiB), enough to keep every large path of a launch resident at once.
-constexpr size_t LDS_WAVE_MAX = 52u * 1024u;
-constexpr size_t LDS_CU_BYTES = 156u * 1024u;
-constexpr size_t SWEEP_MAX_WAVES = 4;  // the sweep kernel's launch bound (waves per block)
 
 using lyg::fillk::FillCaps;
 
-// LDS-resident capacities for a path of at most `bound` events (two per edge): active
-// edges (and pending edges below one point) are bounded by the edges that cross one
-// sweep line, a quarter of the events plus a margin; spans by the active edges (dead
-// spans wait for the next cleanup); the pending intersections by 2.5 active edges; the
-// monotone node pool by the events.  The 513-point stars of the fill workload peak at
-// 280 active edges, 265 spans, 678 heap entries and 1,114 nodes (bound 1,044).  A path
-// that outgrows one of them is swept again in the migrating form.
-// `shrink` > 1 divides them (at least 8 each), which makes paths outgrow the LDS form on
-// purpose: the tests' way to run its fallback.
-FillCaps lds_caps(uint64_t bound, uint32_t shrink) {
-    const uint64_t d = shrink > 1 ? shrink : 1;
-    auto cap = [&](uint64_t v) {
-        return (uint32_t)std::min<uint64_t>(std::max<uint64_t>(v / d, 8), 0x7fffffffu);
-    };
-    const uint64_t act = bound / 4 + bound / 32 + 16;
-    FillCaps k;
-    k.ev = 0;
-    k.act = cap(act);
-    k.span = cap(act + 16);
-    k.heap = cap(act * 5 / 2 + 64);
-    k.node = cap(bound + bound / 4 + 64);
-    k.below = cap(act / 4 + 16);
-    return k;
+// What sizes the register sweep: a path's events and the sum of its segments' degrees (a
+// line 1, a quadratic 2, a cubic 3: how often a horizontal line can cross them).
+struct Shape {
+    uint64_t bound, degree;
+};
+// Active edges: half the crossings a line can have, with a margin.  The 513-point stars of
+// the fill workload peak at 280 (estimate 305), 64 random curves at 70 (estimate 97).
+uint64_t act_estimate(const Shape& p) { return p.degree / 2 + p.degree / 16 + 16; }
+// Pending intersections: 2.5 per active edge (the stars peak at 678), at least 512.
+uint64_t heap_estimate(const Shape& p) {
+    return std::max<uint64_t>(act_estimate(p) * 5 / 2 + 64, 512);
 }
-// The form a path starts in, and its LDS capacities (spans and nodes 0 in FORM_PART).
-int path_form(uint64_t bound, uint32_t mode, FillCaps* lc) {
-    *lc = lds_caps(bound, mode);
-    if (mode && lyg_fill_lds_bytes(lc) <= LDS_WAVE_MAX) return FORM_LDS;
-    lc->span = lc->node = 0;
-    if (mode && lyg_fill_lds_bytes(lc) <= LDS_WAVE_MAX) return FORM_PART;
-    return FORM_MIGRATE;
+
+// The form a path's first sweep takes: the fewest register sets that hold its estimate.  With
+// its active edges in registers an event takes 3.2-4.1 us (2 sets; over arrays 7.1) or 8.8 us
+// (5 sets, the 513-point stars; over arrays 18.4): one path of 64 segments (4,900 events)
+// 20.1 ms instead of 37.2, the 4,096-path workload 330 instead of 704.  Beyond 16 sets, and
+// after a retry with 16, the sweep goes over arrays.
+int path_form(const Shape& p, uint32_t mode) {
+    if (!mode) return FORM_ARRAYS;
+    const uint64_t act = act_estimate(p);
+    for (int f = 1; f < N_FORMS; ++f)
+        if (act <= 64 * REG_CHUNKS[f]) return f;
+    return FORM_ARRAYS;
+}
+uint32_t reg_rows(const Shape& p) {
+    return (uint32_t)std::min<uint64_t>((heap_estimate(p) + 63) / 64, REG_MAX_ROWS);
 }
 
 // Working-memory capacities of one wave for paths of at most `bound` events and `inter`
@@ -158,9 +153,12 @@ struct Launch {
     size_t k0, k1, blocks, stride, work_off;
     uint64_t est;   // the class's work: its largest path's events + 2 x intersections
     FillCaps cap;   // working-memory capacities
-    int form;       // placement form of the hot arrays
-    FillCaps lc;    // their LDS capacities (forms 1 and 2)
-    uint32_t wpb, hot;
+    int form;
+    uint32_t wpb, hot;                // the sweep over arrays: waves per block, LDS per wave
+    uint32_t rows, act_lim, heap_lim; // the register sweep
+    // the sweep over arrays after it (blocks 0: none)
+    size_t again_blocks, again_stride, again_off;
+    FillCaps again_cap;
 };
 
 // The paths of one round in launch order with their staging offsets, and its launches.
@@ -169,20 +167,38 @@ struct RoundPlan {
     std::vector<uint64_t> offs;  // staging offsets: vertices [0, m], triangles [m + 1, 2m + 1]
     std::vector<Launch> launches;
     size_t work_bytes = 0;       // working memory of all launches
+    uint64_t log_ops = 0;        // operations the register sweep's log holds
 };
 
-// Plans round `round` over the paths `todo`, with `scale` times the first round's room.
+// Plans round `round` over the paths `todo`, with `scale` times the first round's room.  A
+// captured graph has no second round: there every register launch is followed by a sweep over
+// arrays of the paths that outgrew it.
 int32_t plan_round(lyg_ctx* c, const std::vector<uint32_t>& todo,
-                   const std::vector<uint32_t>& bound, const std::vector<uint32_t>& inter,
-                   const std::vector<uint64_t>& need, int round, uint64_t scale, RoundPlan* P) {
-    // order by launch: size class, then the placement form (the first round picks it
-    // per path; retries migrate); then by path
+                   const std::vector<uint32_t>& bound, const std::vector<uint32_t>& degree,
+                   const std::vector<uint32_t>& inter, const std::vector<uint64_t>& need,
+                   int round, uint64_t scale, bool graph, RoundPlan* P) {
+    // the register sweep's log takes 32 bytes per staged triangle
+    uint64_t all_v = 0, all_t = 0;
+    for (uint32_t p : todo) {
+        uint64_t v, t;
+        stage_caps(bound[p], inter[p], scale, &v, &t);
+        all_v += v;
+        all_t += t;
+    }
+    const uint32_t mode = c->fill_lds_resident;
+    const bool reg = round <= (mode == 1 ? 1 : 0) && 8 * all_v + 44 * all_t <= STAGE_BUDGET;
+    auto shape = [&](uint32_t p) { return Shape{bound[p], degree[p]}; };
+    P->log_ops = reg ? all_t : 0;
+    // order by launch: size class, then the form (the first round picks it per path, the
+    // second takes all the register sets, later ones sweep over arrays); then by path
     std::vector<int> cls(todo.size());
     for (size_t k = 0; k < todo.size(); ++k) {
         const uint32_t p = todo[k];
-        FillCaps lc;
-        const int form = round == 0 ? path_form(bound[p], c->fill_lds_resident, &lc)
-                                    : FORM_MIGRATE;
+        const int form = !reg ? FORM_ARRAYS
+                         : round == 0 ? path_form(shape(p), mode)
+                         : mode && act_estimate(shape(p)) <= 64 * REG_CHUNKS[N_FORMS - 1]
+                             ? N_FORMS - 1
+                             : FORM_ARRAYS;
         cls[k] = N_FORMS * size_class(need[p]) + form;
     }
     std::vector<size_t> order(todo.size());
@@ -230,35 +246,47 @@ int32_t plan_round(lyg_ctx* c, const std::vector<uint32_t>& todo,
         for (size_t k = k0; k < k1; ++k) ln.est = std::max<uint64_t>(ln.est, need[list[k]]);
         ln.cap = class_caps(std::max<uint64_t>(maxb, 1), maxi, scale);
         ln.form = kc % N_FORMS;
-        ln.lc = FillCaps{};
         ln.wpb = wpb;
         ln.hot = hot;
+        ln.rows = ln.act_lim = ln.heap_lim = 0;
+        ln.again_blocks = 0;
         int ln_occ = occ;
-        if (ln.form != FORM_MIGRATE) {
-            // every capacity grows with the bound: the largest path's fit them all
-            (void)path_form(maxb, c->fill_lds_resident, &ln.lc);
-            if (ln.form == FORM_LDS) ln.lc = lds_caps(maxb, c->fill_lds_resident);
-            ln.hot = (uint32_t)((lyg_fill_lds_bytes(&ln.lc) + 255) & ~(size_t)255);
-            ln.wpb = (uint32_t)std::max<size_t>(
-                1, std::min<size_t>(SWEEP_MAX_WAVES, LDS_CU_BYTES / ln.hot));
-            ln_occ = lyg_fill_occupancy_form(ln.wpb, ln.hot, ln.form);
-            while (ln_occ < 1 && ln.wpb > 1)
-                ln_occ = lyg_fill_occupancy_form(--ln.wpb, ln.hot, ln.form);
-            if (ln_occ < 1) {  // cannot launch: the migrating form
-                ln.form = FORM_MIGRATE;
-                ln.wpb = wpb;
-                ln.hot = hot;
+        if (ln.form != FORM_ARRAYS) {
+            ln.rows = round ? REG_MAX_ROWS : 0;
+            for (size_t k = k0; k < k1; ++k)
+                ln.rows = std::max(ln.rows, reg_rows(shape(list[k])));
+            ln_occ = lyg_fill_reg_occupancy(REG_CHUNKS[ln.form], ln.rows);
+            if (ln_occ < 1) {  // cannot launch
+                ln.form = FORM_ARRAYS;
                 ln_occ = occ;
             }
         }
-        if (ln.form != FORM_MIGRATE) {
-            // arrays that live in LDS need no global region (their overflow retries):
-            // the heap is most of a wave's worst-case working memory
-            ln.cap.heap = 0;
-            ln.cap.below = 0;
-            if (ln.form == FORM_LDS) ln.cap.span = 0;
+        if (ln.form != FORM_ARRAYS) {
+            ln.wpb = 1;
+            ln.hot = 0;
+            ln.act_lim = ln.heap_lim = 0xffffffffu;
+            if (mode > 1) {  // the tests' way to make paths outgrow the registers
+                Shape most{0, 0};
+                for (size_t k = k0; k < k1; ++k) {
+                    most.bound = std::max<uint64_t>(most.bound, bound[list[k]]);
+                    most.degree = std::max<uint64_t>(most.degree, degree[list[k]]);
+                }
+                ln.act_lim = (uint32_t)std::max<uint64_t>(act_estimate(most) / mode, 8);
+                ln.heap_lim = (uint32_t)std::max<uint64_t>(heap_estimate(most) / mode, 8);
+            }
+            // in memory: the event arrays, and two copies of the active edges for a recovery
+            const uint32_t ev = ln.cap.ev;
+            if (graph && mode == 1) {
+                ln.again_cap = ln.cap;
+                ln.again_stride = lyg_fill_work_bytes(&ln.cap, hot);
+                ln.again_blocks = std::min<size_t>((k1 - k0 + wpb - 1) / wpb, c->cu_count);
+                want_bytes += ln.again_blocks * ln.again_stride * wpb;
+            }
+            ln.cap = FillCaps{};
+            ln.cap.ev = ev;
+            ln.cap.act = 64 * REG_CHUNKS[ln.form];
         }
-        ln.stride = lyg_fill_work_bytes(&ln.cap, ln.form != FORM_MIGRATE ? 0 : ln.hot);
+        ln.stride = lyg_fill_work_bytes(&ln.cap, ln.hot);
         size_t blocks = (k1 - k0 + ln.wpb - 1) / ln.wpb;
         ln.blocks = std::max<size_t>(1, std::min<size_t>(blocks, (size_t)c->cu_count * ln_occ));
         ln.work_off = 0;
@@ -269,12 +297,17 @@ int32_t plan_round(lyg_ctx* c, const std::vector<uint32_t>& todo,
     // over the budget: every class gives up blocks in proportion
     size_t& work_bytes = P->work_bytes;
     work_bytes = 0;
-    for (Launch& ln : launches) {
+    auto place = [&](size_t* blocks, size_t block_bytes) {
         if (want_bytes > WORK_BUDGET)
-            ln.blocks = std::max<size_t>(
-                1, (size_t)((double)ln.blocks * (double)WORK_BUDGET / (double)want_bytes));
-        ln.work_off = work_bytes;
-        work_bytes += (ln.blocks * ln.stride * ln.wpb + 255) & ~(size_t)255;
+            *blocks = std::max<size_t>(
+                1, (size_t)((double)*blocks * (double)WORK_BUDGET / (double)want_bytes));
+        const size_t at = work_bytes;
+        work_bytes += (*blocks * block_bytes + 255) & ~(size_t)255;
+        return at;
+    };
+    for (Launch& ln : launches) {
+        ln.work_off = place(&ln.blocks, ln.stride * ln.wpb);
+        if (ln.again_blocks) ln.again_off = place(&ln.again_blocks, ln.again_stride * wpb);
     }
     return LYG_OK;
 }
@@ -307,13 +340,35 @@ void set_launch(lyg::FillLaunch& L, const RoundPlan& P, size_t li, uint8_t* work
     L.caps = ln.cap;
     L.hot_bytes = ln.hot;
     L.waves_per_block = ln.wpb;
-    L.form = (uint32_t)ln.form;
-    L.lds_caps = ln.lc;
+    L.reg_chunks = REG_CHUNKS[ln.form];
+    L.heap_rows = ln.rows;
+    L.act_limit = ln.act_lim;
+    L.heap_limit = ln.heap_lim;
     L.path_list = d_list + ln.k0;
     L.n_list = (uint32_t)(ln.k1 - ln.k0);
     L.stage_v_off = d_off + ln.k0;
     L.stage_t_off = d_off + (m + 1) + ln.k0;
     L.work_counter = counters + li;  // one per launch
+    L.only_retry = 0;
+}
+
+hipError_t launch_sweep(const lyg::FillLaunch& L, const Launch& ln, hipStream_t s) {
+    return ln.form == FORM_ARRAYS ? lyg_launch_fill_sweep(&L, (int)ln.blocks, s)
+                                  : lyg_launch_fill_reg(&L, (int)ln.blocks, s);
+}
+
+// The sweep over arrays that follows launch li in a graph.
+hipError_t launch_again(lyg_ctx* c, lyg::FillLaunch L, const Launch& ln, uint8_t* work,
+                        hipStream_t s) {
+    L.work = work + ln.again_off;
+    L.work_stride = ln.again_stride;
+    L.caps = ln.again_cap;
+    L.hot_bytes = c->fill_hot_bytes;
+    L.waves_per_block = c->fill_waves_per_block;
+    L.reg_chunks = 0;
+    L.work_counter += MAX_LAUNCHES;
+    L.only_retry = 1;
+    return lyg_launch_fill_sweep(&L, (int)ln.again_blocks, s);
 }
 
 struct FillJob {
@@ -334,16 +389,21 @@ struct FillResult {
 // Step 1 and the intersection estimate, read back to the host: every path's event bound
 // and its estimated self-intersections.
 bool measure(lyg_ctx* c, const lyg::FillLaunch& L, hipStream_t s, std::vector<uint32_t>* bound_out,
-             std::vector<uint32_t>* inter_out) {
+             std::vector<uint32_t>* degree_out, std::vector<uint32_t>* inter_out) {
     const uint32_t n = L.in.n_paths;
-    if (!ensure(c, c->f_bound, 4ull * n)) return false;
+    if (!ensure(c, c->f_bound, 8ull * n)) return false;
     std::vector<uint32_t>& bound = *bound_out;
+    std::vector<uint32_t>& degree = *degree_out;
     std::vector<uint32_t>& inter = *inter_out;
     bound.assign(n, 0);
+    degree.assign(n, 0);
     inter.assign(n, 0);
     uint32_t n_verbs = 0;
-    if (!check(c, lyg_launch_fill_bound(&L, n, as<uint32_t>(c->f_bound), s), "fill bound") ||
-        !check(c, hipMemcpyAsync(bound.data(), c->f_bound.p, 4ull * n, hipMemcpyDeviceToHost, s),
+    uint32_t* d_bound = as<uint32_t>(c->f_bound);
+    if (!check(c, lyg_launch_fill_bound(&L, n, d_bound, d_bound + n, s), "fill bound") ||
+        !check(c, hipMemcpyAsync(bound.data(), d_bound, 4ull * n, hipMemcpyDeviceToHost, s),
+               "D2H") ||
+        !check(c, hipMemcpyAsync(degree.data(), d_bound + n, 4ull * n, hipMemcpyDeviceToHost, s),
                "D2H") ||
         !check(c, hipMemcpyAsync(&n_verbs, L.in.verb_off + n, 4, hipMemcpyDeviceToHost, s), "D2H") ||
         !check(c, hipStreamSynchronize(s), "sync"))
@@ -380,8 +440,8 @@ int32_t fill_sweep(lyg_ctx* c, const FillJob& J, uint32_t* vtx_off, uint32_t* id
     L.path_round = as<uint32_t>(c->f_round);
     L.path_hint = as<uint32_t>(c->f_hint);
     L.vertex_offset = J.vertex_offset;
-    std::vector<uint32_t> bound, inter;
-    if (!measure(c, L, s, &bound, &inter)) return LYG_ERR_DEVICE;
+    std::vector<uint32_t> bound, degree, inter;
+    if (!measure(c, L, s, &bound, &degree, &inter)) return LYG_ERR_DEVICE;
     // size classes go by the larger of the two room drivers
     std::vector<uint64_t> need(n);
     for (uint32_t i = 0; i < n; ++i) need[i] = (uint64_t)bound[i] + 2ull * inter[i];
@@ -404,7 +464,7 @@ int32_t fill_sweep(lyg_ctx* c, const FillJob& J, uint32_t* vtx_off, uint32_t* id
     int round = 0;
     for (; round < MAX_ROUNDS && !todo.empty(); ++round, scale = next_scale) {
         RoundPlan P;
-        const int32_t planned = plan_round(c, todo, bound, inter, need, round, scale, &P);
+        const int32_t planned = plan_round(c, todo, bound, degree, inter, need, round, scale, false, &P);
         if (planned != LYG_OK) return planned;
         const std::vector<uint32_t>& list = P.list;
         const std::vector<uint64_t>& offs = P.offs;
@@ -414,7 +474,9 @@ int32_t fill_sweep(lyg_ctx* c, const FillJob& J, uint32_t* vtx_off, uint32_t* id
         if (!ensure_at(c, c->f_list, round, 4 * m) ||
             !ensure_at(c, c->f_stage_off, round, 8 * offs.size()) ||
             !ensure_at(c, c->f_stage_v, round, 8 * sv[m]) ||
-            !ensure_at(c, c->f_stage_t, round, 12 * st[m]))
+            !ensure_at(c, c->f_stage_t, round, 12 * st[m]) ||
+            (P.log_ops && !ensure(c, c->f_ops, sizeof(lyg::FillOp) * P.log_ops)) ||
+            !ensure(c, c->f_path_ops, 4ull * n))
             return LYG_ERR_DEVICE;
         uint32_t* d_list = as<uint32_t>(c->f_list[round]);
         uint64_t* d_off = as<uint64_t>(c->f_stage_off[round]);
@@ -431,6 +493,8 @@ int32_t fill_sweep(lyg_ctx* c, const FillJob& J, uint32_t* vtx_off, uint32_t* id
         L.round = (uint32_t)round;
         L.stage_v = as<float>(c->f_stage_v[round]);
         L.stage_t = as<uint32_t>(c->f_stage_t[round]);
+        L.ops = as<lyg::FillOp>(c->f_ops);
+        L.path_ops = as<uint32_t>(c->f_path_ops);
         const std::vector<Launch>& launches = P.launches;
         if (!ensure(c, c->f_work, P.work_bytes)) return LYG_ERR_NO_SPACE;
         const auto t_round = std::chrono::steady_clock::now();
@@ -448,7 +512,7 @@ int32_t fill_sweep(lyg_ctx* c, const FillJob& J, uint32_t* vtx_off, uint32_t* id
                        as<uint32_t>(c->f_counters));
             const auto t_launch = std::chrono::steady_clock::now();
             if (!check(c, hipStreamWaitEvent(cs, c->class_ev[0], 0), "wait") ||
-                !check(c, lyg_launch_fill_sweep(&L, (int)ln.blocks, cs), "fill sweep") ||
+                !check(c, launch_sweep(L, ln, cs), "fill sweep") ||
                 !check(c, hipEventRecord(c->class_ev[1 + li], cs), "event") ||
                 !check(c, hipStreamWaitEvent(s, c->class_ev[1 + li], 0), "wait"))
                 return LYG_ERR_DEVICE;
@@ -456,11 +520,10 @@ int32_t fill_sweep(lyg_ctx* c, const FillJob& J, uint32_t* vtx_off, uint32_t* id
                 (void)hipStreamSynchronize(cs);
                 fprintf(stderr,
                         "[lyg]   class launch %zu: %zu paths, %zu blocks, %.1f KiB per wave, "
-                        "heap %u node %u act %u, %s %u waves x %u B LDS, %.2f ms\n",
+                        "heap %u node %u act %u, %u register sets x %u rows, %.2f ms\n",
                         li, ln.k1 - ln.k0, ln.blocks, ln.stride / 1024.0, ln.cap.heap, ln.cap.node,
                         ln.cap.act,
-                        ln.form == FORM_LDS ? "LDS" : ln.form == FORM_PART ? "LDS+global" : "migrating",
-                        ln.wpb, ln.hot,
+                        REG_CHUNKS[ln.form], ln.rows,
                         std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() -
                                                                   t_launch).count());
                 fflush(stderr);
@@ -609,7 +672,8 @@ struct lygi::FillGraph {
     uint32_t n = 0;
     uint32_t vertex_offset = 0;
     uint64_t vertex_capacity = 0, index_capacity = 0;
-    DevBuf status, round, nv, ni, list, off, stage_v, stage_t, work, counters, totals, tiles;
+    DevBuf status, round, nv, ni, list, off, stage_v, stage_t, ops, path_ops, work, counters,
+        totals, tiles;
     std::vector<hipGraph_t> graphs;
     hipGraphExec_t head = nullptr, tail = nullptr;
     std::vector<hipGraphExec_t> part;  // per class stream
@@ -648,12 +712,12 @@ int32_t lygi::fill_graph_capture(lyg_ctx* c, const lyg_batch_in* in, const lyg_f
     g->index_capacity = out->index_capacity;
     if (!ensure(c, g->status, 4ull * n) || !ensure(c, g->round, 4ull * n) ||
         !ensure(c, g->nv, 4ull * n) || !ensure(c, g->ni, 4ull * n) ||
-        !ensure(c, g->counters, 4ull * (MAX_LAUNCHES + 1)) || !ensure(c, g->totals, 16) ||
+        !ensure(c, g->counters, 4ull * (N_GRAPH_COUNTERS + 1)) || !ensure(c, g->totals, 16) ||
         // the scans' tile buffer is allocated before the capture, not inside it
         (n > 32768 && !ensure(c, g->tiles, lyg_scan_tiles_bytes(n))))
         return LYG_ERR_DEVICE;
     uint32_t* counters = as<uint32_t>(g->counters);
-    uint32_t* overflow = counters + MAX_LAUNCHES;  // the offset scans' 32-bit overflow flag
+    uint32_t* overflow = counters + N_GRAPH_COUNTERS;  // the offset scans' 32-bit overflow flag
     lyg::FillLaunch L{};
     L.in.verbs = in->verbs;
     L.in.points = in->points;
@@ -670,8 +734,8 @@ int32_t lygi::fill_graph_capture(lyg_ctx* c, const lyg_batch_in* in, const lyg_f
     L.vertex_offset = out->vertex_offset;
     L.round = 0;
     // the plan: lyg_fill_batch's first round over every path
-    std::vector<uint32_t> bound, inter;
-    if (!measure(c, L, s, &bound, &inter)) return LYG_ERR_DEVICE;
+    std::vector<uint32_t> bound, degree, inter;
+    if (!measure(c, L, s, &bound, &degree, &inter)) return LYG_ERR_DEVICE;
     std::vector<uint64_t> need(n);
     std::vector<uint32_t> todo(n);
     for (uint32_t i = 0; i < n; ++i) {
@@ -683,13 +747,15 @@ int32_t lygi::fill_graph_capture(lyg_ctx* c, const lyg_batch_in* in, const lyg_f
         todo[i] = i;
     }
     RoundPlan P;
-    const int32_t planned = plan_round(c, todo, bound, inter, need, 0, 1, &P);
+    const int32_t planned = plan_round(c, todo, bound, degree, inter, need, 0, 1, true, &P);
     if (planned != LYG_OK) return planned;
     const size_t m = P.list.size();
     const uint64_t* sv = P.offs.data();
     const uint64_t* st = P.offs.data() + m + 1;
     if (!ensure(c, g->list, 4 * m) || !ensure(c, g->off, 8 * P.offs.size()) ||
-        !ensure(c, g->stage_v, 8 * sv[m]) || !ensure(c, g->stage_t, 12 * st[m]))
+        !ensure(c, g->stage_v, 8 * sv[m]) || !ensure(c, g->stage_t, 12 * st[m]) ||
+        (P.log_ops && !ensure(c, g->ops, sizeof(lyg::FillOp) * P.log_ops)) ||
+        !ensure(c, g->path_ops, 4ull * n))
         return LYG_ERR_DEVICE;
     if (!ensure(c, g->work, P.work_bytes)) return LYG_ERR_NO_SPACE;
     uint32_t* d_list = as<uint32_t>(g->list);
@@ -701,6 +767,8 @@ int32_t lygi::fill_graph_capture(lyg_ctx* c, const lyg_batch_in* in, const lyg_f
         return LYG_ERR_DEVICE;
     L.stage_v = as<float>(g->stage_v);
     L.stage_t = as<uint32_t>(g->stage_t);
+    L.ops = as<lyg::FillOp>(g->ops);
+    L.path_ops = as<uint32_t>(g->path_ops);
     const size_t n_streams = std::min<size_t>(P.launches.size(), CLASS_STREAMS);
     if (!class_streams(c, n_streams, P.launches.size()) ||
         !check(c, hipEventCreateWithFlags(&g->fork, hipEventDisableTiming), "hipEventCreate"))
@@ -708,7 +776,7 @@ int32_t lygi::fill_graph_capture(lyg_ctx* c, const lyg_batch_in* in, const lyg_f
     const std::vector<size_t> stream_of = assign_streams(P, n_streams);
     // head: counters and the status a path keeps if no launch reaches it
     if (!capture_on(c, s, g, &g->head, [&]() {
-            return check(c, lyg_launch_fill_u32(counters, MAX_LAUNCHES + 1, 0, s), "reset") &&
+            return check(c, lyg_launch_fill_u32(counters, N_GRAPH_COUNTERS + 1, 0, s), "reset") &&
                    check(c, lyg_launch_fill_list_u32(L.path_status, d_list, (uint32_t)m,
                                                      ST_UNSWEPT, s),
                          "status");
@@ -727,8 +795,10 @@ int32_t lygi::fill_graph_capture(lyg_ctx* c, const lyg_batch_in* in, const lyg_f
                 const size_t li = P.launches.size() - 1 - r;
                 if (stream_of[li] != si) continue;
                 set_launch(L, P, li, as<uint8_t>(g->work), d_list, d_off, counters);
-                if (!check(c, lyg_launch_fill_sweep(&L, (int)P.launches[li].blocks, cs),
-                           "fill sweep"))
+                const Launch& ln = P.launches[li];
+                if (!check(c, launch_sweep(L, ln, cs), "fill sweep") ||
+                    (ln.again_blocks &&
+                     !check(c, launch_again(c, L, ln, as<uint8_t>(g->work), cs), "fill sweep")))
                     return false;
             }
             return true;
@@ -804,7 +874,7 @@ int32_t lygi::fill_graph_result(FillGraph* g, uint64_t* n_vertices, uint64_t* n_
     std::vector<uint32_t> st(g->n);
     if (!check(c, hipStreamSynchronize(s), "sync") ||
         !check(c, hipMemcpy(tot, g->totals.p, 16, hipMemcpyDeviceToHost), "D2H") ||
-        !check(c, hipMemcpy(&ovf, as<uint32_t>(g->counters) + MAX_LAUNCHES, 4,
+        !check(c, hipMemcpy(&ovf, as<uint32_t>(g->counters) + N_GRAPH_COUNTERS, 4,
                             hipMemcpyDeviceToHost),
                "D2H") ||
         !check(c, hipMemcpy(st.data(), g->status.p, 4ull * g->n, hipMemcpyDeviceToHost), "D2H"))
@@ -834,7 +904,7 @@ void lygi::fill_graph_destroy(FillGraph* g) {
     if (g->fork) (void)hipEventDestroy(g->fork);
     for (hipEvent_t e : g->join) (void)hipEventDestroy(e);
     for (DevBuf* b : {&g->status, &g->round, &g->nv, &g->ni, &g->list, &g->off, &g->stage_v,
-                      &g->stage_t, &g->work, &g->counters, &g->totals, &g->tiles})
+                      &g->stage_t, &g->ops, &g->path_ops, &g->work, &g->counters, &g->totals, &g->tiles})
         free_buf(*b);
     delete g;
 }

@@ -134,6 +134,15 @@ struct FillCaps {
 };
 }  // namespace fillk
 
+// A span operation of the register sweep's log (fill_reg.hip).
+struct FillOp {
+    float x, y;
+    uint32_t id, kind;             // vertex id; left / right vertex, begin, end
+    uint32_t next;                 // the span's next operation
+    uint32_t link_side, link_stack;
+    uint32_t tris;                 // its triangles, then their offset in the path's
+};
+
 struct FillLaunch {
     PathBatchDev in;
     const lyg_fill_options* opts;  // per path (opts_stride 1) or shared (stride 0)
@@ -143,12 +152,6 @@ struct FillLaunch {
     fillk::FillCaps caps;          // capacities of the per-wave arrays
     uint32_t hot_bytes;            // per-wave dynamic LDS for the hot arrays (0: none)
     uint32_t waves_per_block;
-    // placement form of the hot arrays: 0 they start in LDS and move to global memory when
-    // they outgrow it; 1 all in LDS; 2 the arrays touched on every event in LDS, spans and
-    // nodes in global memory.  Forms 1 and 2 use the lds_caps capacities (act, span, node,
-    // heap, below) and stop a path that outgrows one with the retry status.
-    uint32_t form;
-    fillk::FillCaps lds_caps;
     float* stage_v;                // per-path staging, path i at stage_v_off[i] (vertices)
     uint32_t* stage_t;             // and stage_t_off[i] (triangles)
     const uint64_t* stage_v_off;
@@ -162,6 +165,14 @@ struct FillLaunch {
     const uint32_t* path_list;     // paths to process (nullptr: 0..n_list)
     uint32_t n_list;
     uint32_t* work_counter;
+    uint32_t only_retry;           // only the paths whose status is retry
+    // register sweep (reg_chunks 0: the sweep over arrays): sets of 64 active edges, pending
+    // events per LDS column, limits below those, the log (path i's operations at
+    // stage_t_off[i]) and its length per path
+    uint32_t reg_chunks, heap_rows;
+    uint32_t act_limit, heap_limit;
+    FillOp* ops;
+    uint32_t* path_ops;
     // copy pass
     const uint32_t* vtx_off;
     const uint32_t* idx_off;

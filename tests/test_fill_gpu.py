@@ -216,6 +216,60 @@ def test_many_launches_in_one_round():
     assert np.array_equal(i1, i0)
 
 
+def zigzag(edges):
+    """A closed comb: a horizontal line crosses up to `edges` of its edges."""
+    n = edges // 2
+    pts = []
+    for i in range(n):
+        pts += [(float(4 * i), 0.25 * (i % 7)), (float(4 * i + 1), 1000.0 + 0.5 * (i % 5))]
+    return polygon(pts + [(4.0 * n, 0.0), (4.0 * n, 1010.0), (-2.0, 1010.0), (-2.0, 0.0)])
+
+
+def fan(edges):
+    """Thin triangles with one apex on top: `edges` edges start at one point."""
+    b = PathBuilder()
+    for i in range(edges // 2):
+        b.begin((0.0, 0.0))
+        b.line_to((20.0 * i - 300.0, 500.0))
+        b.line_to((20.0 * i - 290.0, 500.0 + i % 3))
+        b.end(True)
+    return b.build()
+
+
+@pytest.mark.parametrize("shape,sizes", [
+    (zigzag, (118, 122, 124, 126, 128, 130)),          # 2 sets of 64 active edges
+    (zigzag, (310, 314, 316, 318, 320, 322)),          # 5 sets
+    (zigzag, (1014, 1018, 1020, 1022, 1024, 1026, 1830, 1900, 2100)),  # 16 sets; beyond
+    (fan, (60, 62, 64, 66, 126, 128, 130)),            # 64 edges below one event
+], ids=["two_sets", "five_sets", "sixteen_sets", "edges_below"])
+def test_active_edges_around_the_register_sets(shape, sizes):
+    """Paths whose active edges, or edges below one event, just fit the register sweep or
+    just outgrow it: plain calls, a batch and a captured batch all give the oracle's
+    vertices and triangles."""
+    from lyon_amd.batch import DeviceBatch, FillBatcher, FillGraph, synchronize
+    from lyon_amd.path import PathBatch
+    paths = [shape(k) for k in sizes]
+    o = FillOptions(tolerance=0.05)
+    refs = [ref_fill(p, o) for p in paths]
+    for k, p in zip(sizes, paths):
+        check(p, o, f"{shape.__name__} {k}", coverage=False)
+    opts = workloads.fill_options(len(paths), tolerance=0.05)
+    opts["fill_rule"] = int(o.fill_rule)
+    db = DeviceBatch(PathBatch.from_paths(paths), opts)
+    res = FillBatcher().run(db)
+    synchronize()
+    graph = FillGraph(db, int(res.n_vertices), int(res.n_indices))
+    graph.launch()
+    for r in (res, graph.result()):
+        v, i, vo, io = r.all_vertices(), r.all_indices(), r.vertex_offsets, r.index_offsets
+        for k, (st, rv, ri) in enumerate(refs):
+            assert r.status[k] == st == 0
+            assert np.array_equal(v[vo[k]:vo[k + 1]].view(np.uint32),
+                                  np.asarray(rv, np.float32).view(np.uint32)), sizes[k]
+            assert np.array_equal(canon(i[io[k]:io[k + 1]]),
+                                  canon(np.asarray(ri, np.int64) + int(vo[k]))), sizes[k]
+
+
 def test_very_large_path():
     """fill_tests.rs:2140-2166: a path of 1,000,000 endpoints (two wiggling sides of a long
     band) fills without error; the same vertices and triangle count as the oracle and the
