@@ -86,6 +86,50 @@ def test_winding_grid_matches_oracle(tol):
             assert np.array_equal(ins, want)
 
 
+@pytest.mark.parametrize("n", [1, 65, 8192, 8193, 40001])
+def test_queries_beside_curves_and_around_a_waves_share(n):
+    """Query points left of, right of and at the ends of the curves' x ranges (where a curve
+    is counted without being flattened, or just has to be), in numbers around one and
+    several queries per wave; curves of a pixel and of a million, quadratics and cubics."""
+    rng = np.random.default_rng(n)
+    b = PathBuilder()
+    curves = []
+    for k in range(150):
+        scale = float(10.0 ** rng.uniform(0, 6) if k % 5 == 0 else 10.0 ** rng.uniform(0, 3))
+        p = (rng.random((4, 2)) * scale).astype(np.float32)
+        if k % 10 == 0:
+            b.begin(tuple(p[0]))
+        else:
+            p[0] = curves[-1][-1]
+        if k % 2:
+            b.quadratic_bezier_to(tuple(p[1]), tuple(p[2]))
+            p = p[:3]
+        else:
+            b.cubic_bezier_to(tuple(p[1]), tuple(p[2]), tuple(p[3]))
+        curves.append(p)
+        if k % 10 == 9:
+            b.end(bool(k % 20 == 9))
+    path = b.build()
+    at = []
+    for c in curves:
+        lo, hi = c.min(axis=0).astype(np.float64), c.max(axis=0).astype(np.float64)
+        for x in (lo[0], hi[0]):
+            for d in (0.0, 1e-7, 2e-5, 0.0099, 0.0101):
+                for sgn in (-1.0, 1.0):
+                    at.append((x + sgn * (d * (hi[0] - lo[0]) + 1e-6 * d * x),
+                               lo[1] + rng.random() * (hi[1] - lo[1])))
+        at += [(x, c[0][1]) for x in (lo[0] - 1.0, hi[0] + 1.0)]
+        at.append((float("nan"), c[0][1]))
+        at.append((c[0][0], float("nan")))
+    at = np.asarray(at, np.float32)
+    xy = np.concatenate([at] * (n // len(at) + 1))[rng.permutation(n) if n < len(at)
+                                                   else np.arange(n)]
+    w, _ = A.path_winding_numbers(xy, path, 0.05, FillRule.NonZero)
+    ref = O.winding_numbers(path, xy, 0.05)
+    bad = np.nonzero(w != ref)[0]
+    assert len(bad) == 0, (len(bad), xy[bad[0]], w[bad[0]], ref[bad[0]])
+
+
 def test_area_matches_oracle_bit_exact():
     for tol in (0.01, 0.05, 1.0):
         for k, p in enumerate(_paths()):
