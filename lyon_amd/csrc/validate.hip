@@ -284,26 +284,47 @@ __global__ void __launch_bounds__(WAVE* VAL_WAVES) winding_kernel(ValidateLaunch
 
 // approximate_signed_area with one wave per path.  lyon's result is a serial f32 sum in
 // event order, so the additions stay serial, but everything before them is spread over the
-// lanes: the verbs are read 64 at a time; between two boundary verbs (Begin, End, Close) the
-// flattened points of a run of segments are computed 1,024 at a time, 16 consecutive ones
-// per lane (t from the closed form once, then lyon's serial sum), each lane forms the cross
-// products of its points with the points before them, and the terms are added to the
-// running sum in point order through readlane.  Begin / End / Close
-// are applied in order between the runs, with area.rs's rules for ill-formed paths.
+// lanes: the verbs are read 64 at a time, a lane sets one up (polynomial form, and lyon's
+// serial t at every 16th point of the run, one addition per point); then the flattened
+// points of a run of segments between two boundary verbs are computed 1,024 at a time, 16
+// consecutive ones per lane, and each lane forms the cross products of its points with the
+// points before them.  For the sum the running value goes from lane to lane, each adding its
+// 16 terms.  Begin / End / Close are applied in order between the runs, with area.rs's rules
+// for ill-formed paths.
+//
+// Bound by VALU issue, about two instructions per point, one of them the serial addition.
+// 10,000 paths, 81 M points: 1,575 us when every lane set its curve up by itself (Wang's
+// count, t in closed form) and terms were read lane by lane; 385 us now.
 constexpr int AREA_WAVES = 4;
-constexpr int AREA_RUN = 16;  // consecutive points per lane
+constexpr int AREA_RUN = 16;              // consecutive points per lane
+constexpr uint32_t AREA_TABLE = 512;      // every 16th point's t: 8,192 points at once
+
+struct AreaPoly {
+    float4 a01;   // a0, a1
+    float4 a23;   // a2, a3 (0 for a quadratic)
+    float4 rest;  // to, step, points
+};
+struct AreaShared {
+    AreaPoly poly[WAVE];
+    uint32_t pre[WAVE + 1];  // term prefix of the window's verbs
+    uint32_t pis[WAVE];      // first point of each verb
+    uint32_t vbs[WAVE];      // verb codes
+    float t[AREA_TABLE];     // t of the run's points 0, 16, 32, ...
+};
+
+// The running value, from the lane before each lane (lane 0 takes `carry`).
+__device__ __forceinline__ float from_lane_before(float v, float carry) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(
+        __builtin_bit_cast(int, carry), __builtin_bit_cast(int, v), 0x138, 0xf, 0xf, false));  // wave_shr:1
+}
 
 __global__ void __launch_bounds__(WAVE* AREA_WAVES) signed_area_kernel(ValidateLaunch L) {
-    __shared__ uint32_t pre_all[AREA_WAVES][WAVE + 1];  // term prefix of the window's verbs
-    __shared__ uint32_t pi_all[AREA_WAVES][WAVE];       // first point of each verb
-    __shared__ uint32_t vb_all[AREA_WAVES][WAVE];       // verb codes
+    __shared__ AreaShared shared[AREA_WAVES];
     const int l = lane_id();
-    const uint32_t w = threadIdx.x / WAVE;
-    uint32_t* pre = pre_all[w];
-    uint32_t* pis = pi_all[w];
-    uint32_t* vbs = vb_all[w];
+    AreaShared& S = shared[threadIdx.x / WAVE];
     const uint32_t stride = gridDim.x * AREA_WAVES;
-    for (uint32_t pid = blockIdx.x * AREA_WAVES + w; pid < L.n_paths; pid += stride) {
+    for (uint32_t pid = blockIdx.x * AREA_WAVES + threadIdx.x / WAVE; pid < L.n_paths;
+         pid += stride) {
         const uint32_t vb = L.verb_off[pid], nv = L.verb_off[pid + 1] - vb;
         const uint32_t pb = L.point_off[pid];
         const PathPts pts{L.points + 2ull * pb, L.point_off[pid + 1] - pb};
@@ -317,28 +338,49 @@ __global__ void __launch_bounds__(WAVE* AREA_WAVES) signed_area_kernel(ValidateL
             const uint32_t cons = points_of(verb);
             const uint32_t incl = incl_scan(cons);
             const uint32_t pi = pc + incl - cons;
-            // flattened points of each segment verb (Line 1, curves Wang's count)
+            // polynomial form and flattened points (Line 1, curves Wang's count)
             uint32_t cnt = 0;
-            if (verb == 0u) {
+            vec2 a0 = mk(0.0f, 0.0f), a1 = a0, a2 = a0, a3 = a0, to = a0;
+            float step = 1.0f;
+            if (verb <= 2u) {
+                const vec2 c1 = pts.at(pi);
+                to = c1;
                 cnt = 1;
-            } else if (verb == 1u) {
-                cnt = seg_count(quad_wang(pts.at(pi - 1u), pts.at(pi), pts.at(pi + 1u), L.tolerance));
-            } else if (verb == 2u) {
-                cnt = seg_count(cubic_wang(pts.at(pi - 1u), pts.at(pi), pts.at(pi + 1u),
-                                           pts.at(pi + 2u), L.tolerance));
+                if (verb != 0u) {
+                    a0 = pts.at(pi - 1u);
+                    const vec2 c2 = pts.at(pi + 1u);
+                    float n;
+                    if (verb == 1u) {
+                        n = quad_wang(a0, c1, c2, L.tolerance);
+                        a1 = mul(sub(c1, a0), 2.0f);
+                        a2 = sub(add(a0, c2), mul(c1, 2.0f));
+                        to = c2;
+                    } else {
+                        const vec2 c3 = pts.at(pi + 2u);
+                        n = cubic_wang(a0, c1, c2, c3, L.tolerance);
+                        a1 = mul(sub(c1, a0), 3.0f);
+                        a2 = add(sub(mul(a0, 3.0f), mul(c1, 6.0f)), mul(c2, 3.0f));
+                        a3 = add(sub(c3, a0), mul(sub(c1, c2), 3.0f));
+                        to = c3;
+                    }
+                    step = 1.0f / n;
+                    cnt = seg_count(n);
+                }
             }
             const uint32_t tincl = incl_scan(cnt);
-            __builtin_amdgcn_wave_barrier();
-            pre[l + 1] = tincl;
-            if (l == 0) pre[0] = 0;
-            pis[l] = pi;
-            vbs[l] = verb;
-            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
-            __builtin_amdgcn_wave_barrier();
+            wave_sync();
+            S.poly[l].a01 = make_float4(a0.x, a0.y, a1.x, a1.y);
+            S.poly[l].a23 = make_float4(a2.x, a2.y, a3.x, a3.y);
+            S.poly[l].rest = make_float4(to.x, to.y, step, u2f(cnt));
+            S.pre[l + 1] = tincl;
+            if (l == 0) S.pre[0] = 0;
+            S.pis[l] = pi;
+            S.vbs[l] = verb;
+            wave_sync();
             const uint64_t bmask = ballot(verb >= 3u);  // boundaries and lanes past the path
             int j = 0;
             while (j < WAVE && !stop) {
-                const uint32_t vj = vbs[j];
+                const uint32_t vj = readlane_u(verb, j);
                 if (vj >= 3u) {
                     if (vj == 0xffu) break;
                     if (vj == 3u) {
@@ -347,7 +389,7 @@ __global__ void __launch_bounds__(WAVE* AREA_WAVES) signed_area_kernel(ValidateL
                             stop = true;
                             break;
                         }
-                        first = pts.at(pis[j]);
+                        first = pts.at(readlane_u(pi, j));
                         cur = first;
                         da = 0.0f;
                         v0c = mk(0.0f, 0.0f);
@@ -365,134 +407,111 @@ __global__ void __launch_bounds__(WAVE* AREA_WAVES) signed_area_kernel(ValidateL
                     ++j;
                     continue;
                 }
-                // a run of segment verbs j .. j2 - 1
-                const uint64_t rest = bmask & ~mask_lt(j);
-                const int j2 = rest ? __builtin_ctzll(rest) : WAVE;
+                // a run of segment verbs j .. j2 - 1, as many as the table holds (one verb
+                // with more points than that takes t in closed form)
                 if (!in_sub) {
                     stop = true;
                     break;
                 }
-                const uint32_t r0 = pre[j], r1 = pre[j2];
-                for (uint32_t q0 = r0; q0 < r1; q0 += WAVE * AREA_RUN) {
-                    // lane l: points [g0, gend) of the run, in order
-                    const uint32_t g0 = q0 + (uint32_t)l * AREA_RUN;
-                    const uint32_t gend = g0 < r1 ? (g0 + AREA_RUN < r1 ? g0 + AREA_RUN : r1) : g0;
-                    vec2 v1s[AREA_RUN];
-                    vec2 p_last = cur, v1_last = mk(0.0f, 0.0f);
+                const uint64_t rest = bmask & ~mask_lt(j);
+                const uint32_t r0 = readlane_u(tincl - cnt, j);
+                const uint64_t over =
+                    (rest | ballot(tincl - r0 > AREA_TABLE * AREA_RUN)) & ~mask_lt(j);
+                int j2 = over ? __builtin_ctzll(over) : WAVE;
+                const bool fits = j2 > j;
+                j2 = fits ? j2 : j + 1;
+                const uint32_t r1 = readlane_u(tincl, j2 - 1);
+                if (fits && l >= j && l < j2) {
+                    uint32_t g = tincl - cnt - r0;
+                    uint32_t k = (AREA_RUN - (g & (AREA_RUN - 1))) & (AREA_RUN - 1);
+                    if (k < cnt) {
+                        float t = 0.0f;
+                        for (uint32_t q = 0; q <= k; ++q) t = t + step;
+                        for (g += k; k < cnt; k += AREA_RUN, g += AREA_RUN) {
+                            S.t[g / AREA_RUN] = t;
 #pragma unroll
-                    for (int u = 0; u < AREA_RUN; ++u) v1s[u] = mk(0.0f, 0.0f);
-                    if (g0 < gend) {
+                            for (int q = 0; q < AREA_RUN; ++q) t = t + step;
+                        }
+                    }
+                }
+                wave_sync();
+                for (uint32_t q0 = r0; q0 < r1; q0 += WAVE * AREA_RUN) {
+                    // lane l: points g0 .. g0 + 15 of the run (those past its end are not used)
+                    const uint32_t m = r1 - q0 < (uint32_t)(WAVE * AREA_RUN)
+                                           ? r1 - q0
+                                           : (uint32_t)(WAVE * AREA_RUN);
+                    const uint32_t g0 = q0 + (uint32_t)l * AREA_RUN;
+                    float terms[AREA_RUN];
+                    vec2 v1_first = mk(0.0f, 0.0f), v0 = v1_first, p = v1_first;
+                    if ((uint32_t)l * AREA_RUN < m) {
                         int lo = j, hi = j2 - 1;  // last verb of the run with pre <= g0
                         while (lo < hi) {
                             const int mid = (lo + hi + 1) >> 1;
-                            if (pre[mid] <= g0) lo = mid;
+                            if (S.pre[mid] <= g0) lo = mid;
                             else hi = mid - 1;
                         }
                         int my = lo;
-                        int kind = 0;
-                        vec2 a0 = mk(0.0f, 0.0f), a1 = a0, a2 = a0, a3 = a0, to = a0;
-                        float step = 1.0f, t = 0.0f;
-                        uint32_t n_pts = 1, k = 0;
-                        auto setup = [&](int v, uint32_t kk) {
-                            const uint32_t sp = pis[v];
-                            kind = (int)vbs[v];
-                            k = kk;
-                            if (kind == 0) {
-                                to = pts.at(sp);
-                                n_pts = 1;
-                                return;
-                            }
-                            const vec2 f = pts.at(sp - 1u), c1 = pts.at(sp), c2 = pts.at(sp + 1u);
-                            float nf;
-                            if (kind == 1) {
-                                nf = quad_wang(f, c1, c2, L.tolerance);
-                                a1 = mul(sub(c1, f), 2.0f);
-                                a2 = sub(add(f, c2), mul(c1, 2.0f));
-                                to = c2;
-                            } else {
-                                const vec2 c3 = pts.at(sp + 2u);
-                                nf = cubic_wang(f, c1, c2, c3, L.tolerance);
-                                a1 = mul(sub(c1, f), 3.0f);
-                                a2 = add(sub(mul(f, 3.0f), mul(c1, 6.0f)), mul(c2, 3.0f));
-                                a3 = add(sub(c3, f), mul(sub(c1, c2), 3.0f));
-                                to = c3;
-                            }
-                            a0 = f;
-                            step = 1.0f / nf;
-                            n_pts = seg_count(nf);
-                            // t of point kk + 1: lyon's serial sum (closed form deep inside)
-                            t = 0.0f;
-                            if (kk + 1 < n_pts) {
-                                if (kk + 1 <= (uint32_t)WAVE) {
-                                    for (uint32_t q = 0; q <= kk; ++q) t = t + step;
-                                } else {
-                                    t = tchain(step, kk + 1);
-                                }
-                            }
-                        };
-                        setup(my, g0 - pre[my]);
+                        float4 a01 = S.poly[my].a01, a23 = S.poly[my].a23, re = S.poly[my].rest;
+                        uint32_t end = S.pre[my + 1];
+                        bool cubic = S.vbs[my] == 2u;
+                        float t = fits ? S.t[(g0 - r0) / AREA_RUN]
+                                       : tchain(re.z, g0 - S.pre[my] + 1u);
 #pragma unroll
                         for (int u = 0; u < AREA_RUN; ++u) {
                             const uint32_t g = g0 + (uint32_t)u;
-                            if (g < gend) {
-                                if (g >= pre[my + 1]) {
-                                    ++my;
-                                    setup(my, 0);
-                                }
-                                vec2 p;
-                                if (k + 1 >= n_pts) {
-                                    p = to;
-                                } else {
-                                    vec2 v = a0;
-                                    float tt = t;
-                                    v = add(v, mul(a1, tt));
-                                    tt = tt * t;
-                                    v = add(v, mul(a2, tt));
-                                    if (kind == 2) {
-                                        tt = tt * t;
-                                        v = add(v, mul(a3, tt));
-                                    }
-                                    p = v;
-                                }
-                                ++k;
-                                t = t + step;
-                                v1s[u] = sub(p, first);
-                                v1_last = v1s[u];
-                                p_last = p;
+                            if (u && g >= end && my + 1 < j2) {
+                                ++my;
+                                a01 = S.poly[my].a01;
+                                a23 = S.poly[my].a23;
+                                re = S.poly[my].rest;
+                                end = S.pre[my + 1];
+                                cubic = S.vbs[my] == 2u;
+                                t = 0.0f + re.z;
                             }
+                            vec2 v = mk(a01.x, a01.y);
+                            float tt = t;
+                            v = add(v, mul(mk(a01.z, a01.w), tt));
+                            tt = tt * t;
+                            v = add(v, mul(mk(a23.x, a23.y), tt));
+                            tt = tt * t;
+                            const vec2 v3 = add(v, mul(mk(a23.z, a23.w), tt));
+                            v = cubic ? v3 : v;
+                            p = g + 1u >= end ? mk(re.x, re.y) : v;
+                            t = t + re.z;
+                            const vec2 v1 = sub(p, first);
+                            if (u == 0) v1_first = v1;
+                            else terms[u] = cross(v0, v1);
+                            v0 = v1;
                         }
                     }
-                    // the point before the lane's first: the previous lane's last (its run is
-                    // full whenever this one has points), or the carry for lane 0
-                    vec2 v0 = shfl_v(v1s[AREA_RUN - 1], l == 0 ? 0 : l - 1);
-                    if (l == 0) v0 = v0c;
-                    float terms[AREA_RUN];
-#pragma unroll
-                    for (int u = 0; u < AREA_RUN; ++u) {
-                        terms[u] = cross(v0, v1s[u]);
-                        v0 = v1s[u];
-                    }
-                    // lyon's serial sum, in point order
-                    const uint32_t m = r1 - q0 < (uint32_t)(WAVE * AREA_RUN) ? r1 - q0
-                                                                             : (uint32_t)(WAVE * AREA_RUN);
-                    const uint32_t full = m / AREA_RUN, rem = m % AREA_RUN;
+                    // the point before the lane's first: the previous lane's last, or the
+                    // carry for lane 0
+                    terms[0] = cross(mk(from_lane_before(v0.x, v0c.x), from_lane_before(v0.y, v0c.y)),
+                                     v1_first);
+                    // lyon's serial sum: after turn ln, lane ln holds the sum up to its end
+                    const uint32_t full = m / AREA_RUN, left = m % AREA_RUN;
+                    float sum = da;
                     for (uint32_t ln = 0; ln < full; ++ln) {
+                        sum = from_lane_before(sum, da);
 #pragma unroll
-                        for (int u = 0; u < AREA_RUN; ++u) da = da + readlane_f(terms[u], (int)ln);
+                        for (int u = 0; u < AREA_RUN; ++u) sum = sum + terms[u];
                     }
-                    if (rem) {
+                    if (left) {
+                        sum = from_lane_before(sum, da);
 #pragma unroll
                         for (int u = 0; u < AREA_RUN; ++u)
-                            if ((uint32_t)u < rem) da = da + readlane_f(terms[u], (int)full);
+                            if ((uint32_t)u < left) sum = sum + terms[u];
                     }
-                    const int last_lane = (int)((m - 1) / AREA_RUN);
-                    v0c = readlane_v(v1_last, last_lane);
-                    cur = readlane_v(p_last, last_lane);
+                    da = readlane_f(sum, (int)((m - 1) / AREA_RUN));
+                    v0c = readlane_v(v0, WAVE - 1);  // of a full chunk
                 }
+                // a run ends at its last segment's end
+                cur = readlane_v(to, j2 - 1);
+                v0c = sub(cur, first);
                 j = j2;
             }
             pc += readlane_u(incl, WAVE - 1);
-            __builtin_amdgcn_wave_barrier();
+            wave_sync();
         }
         if (l == 0) L.areas[pid] = area;
     }

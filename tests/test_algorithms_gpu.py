@@ -138,6 +138,39 @@ def test_area_matches_oracle_bit_exact():
             assert np.float32(a).view(np.uint32) == np.float32(r).view(np.uint32), (k, tol, a, r)
 
 
+@pytest.mark.parametrize("curve_points", [1, 15, 16, 17, 130, 1024, 8192, 20000])
+def test_areas_around_the_points_computed_at_once(curve_points):
+    """Runs of segments whose flattened points just fit, fill or exceed a lane's 16, a
+    wave's 1,024 and the table's 8,192 at once (one curve of more takes t in closed form),
+    and of 1 to 130 verbs; bit-exact."""
+    rng = np.random.default_rng(curve_points)
+    tol = 1e-3
+    paths = []
+    for verbs in (1, 3, 62, 63, 64, 130):
+        if curve_points * verbs > 400000:
+            continue
+        b = PathBuilder()
+        b.begin((0.0, 0.0))
+        for k in range(verbs):
+            # Wang: n = sqrt(6 d / (8 tol)) for a second difference d of the control points
+            d = (curve_points * (1.0 - 0.02 * rng.random())) ** 2 * 8.0 * tol / 6.0
+            x, y = rng.random(2) * 100.0
+            if k % 7 == 3:
+                b.line_to((x, y))
+            elif k % 2:
+                b.quadratic_bezier_to((x + 1.5 * d, y), (x, y + 3.0))
+            else:
+                b.cubic_bezier_to((x, y + d), (x - d, y), (x + 5.0, y - 2.0))
+        b.end(verbs % 2 == 1)
+        paths.append(b.build())
+    db = DeviceBatch(PathBatch.from_paths(paths))
+    da = DeviceBuffer(4 * len(paths))
+    A.signed_areas_device(db, tol, da)
+    a = da.download(np.float32, len(paths))
+    r = np.array([O.signed_area(p, tol) for p in paths], np.float32)
+    assert np.array_equal(a.view(np.uint32), r.view(np.uint32)), (a, r)
+
+
 def test_batched_forms_match_oracle():
     """Batched winding numbers and areas over device-resident paths, with ragged inputs:
     empty paths, a path of one Begin/End, and a query naming a path past the batch."""
