@@ -403,8 +403,9 @@ int32_t lyg_ctx_set_stroke_staging(lyg_ctx* ctx, int enabled, float room_scale);
  * by different waves at once; each part first re-walks the window before it to rebuild
  * the walk's state, and a check per path confirms it matches the state the previous part
  * ended in (else the path is walked again whole).  The output is the same bytes as the
- * whole-path walk.  Default 64 (parts of 4,096 steps); 0: every path is walked by one
- * wave. */
+ * whole-path walk.  0: every path is walked by one wave.  Until this is called (or the
+ * autotuner), the parts go by the batch's paths: 2 windows for a path or few, up to 64 (parts
+ * of 4,096 steps) for thousands. */
 int32_t lyg_ctx_set_stroke_split(lyg_ctx* ctx, uint32_t windows_per_part);
 /* Where the fill sweep keeps its state (no lyon counterpart).  enabled (default): each path
  * of at most 1,024 estimated active edges is swept with those in registers and its pending

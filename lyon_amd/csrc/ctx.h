@@ -48,6 +48,7 @@ struct lyg_ctx {
     DevBuf scan_tiles;               // tile sums of scans over more than 32768 counts
     DevBuf st_cap_v, st_cap_i, st_off_v, st_off_i, st_v, st_i, st_fallback;
     // stroke: long paths split into parts of this many 64-step windows (0: whole paths)
+    bool stroke_split_auto = true;  // until set or tuned: fewer windows for few paths
     uint32_t stroke_split_windows = 64;
     uint64_t last_stroke_items = 0;       // items of the last split stroke batch
     uint32_t last_stroke_again = 0;       // its paths walked again whole

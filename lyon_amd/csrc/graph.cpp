@@ -29,10 +29,10 @@ hipError_t lyg_launch_scan(const uint32_t* counts, uint32_t n, uint32_t* offsets
 hipError_t lyg_launch_fill_u32(uint32_t* p, uint32_t n, uint32_t v, hipStream_t s);
 int lyg_fill_occupancy(uint32_t waves_per_block, uint32_t hot_bytes);
 hipError_t lyg_launch_stroke_plan(const lyg::StrokeLaunch* L, uint32_t n_paths,
-                                  uint32_t split_windows, float room_scale, uint32_t* extra,
+                                  uint32_t split_windows, uint32_t max_parts, float room_scale, uint32_t* extra,
                                   uint32_t* rv, uint32_t* ri, int grid, hipStream_t s);
 hipError_t lyg_launch_stroke_cut(const lyg::StrokeLaunch* L, uint32_t n_paths,
-                                 uint32_t split_windows, float room_scale, const uint32_t* extra,
+                                 uint32_t split_windows, uint32_t max_parts, float room_scale, const uint32_t* extra,
                                  const uint32_t* extra_off, const uint32_t* rv,
                                  const uint32_t* ri, const uint32_t* v_off, const uint32_t* i_off,
                                  uint32_t cap_extra, uint32_t* err, int grid, hipStream_t s);
@@ -150,14 +150,14 @@ bool capture_stroke_items(lyg_ctx* c, lyg_graph* g, const lyg_batch_in* in,
     uint32_t* voff = as<uint32_t>(g->voff);
     uint32_t* ioff = as<uint32_t>(g->ioff);
     const int pgrid = (int)std::min<uint32_t>(n, (uint32_t)std::max(1, c->cu_count) * 32u);
-    const uint32_t W = c->stroke_split_windows;
+    const lygi::Cutting cutting = lygi::stroke_cutting(c, n);
     const float room = c->stroke_room_scale;
     auto scan = [&](const uint32_t* counts, uint32_t* offsets, uint64_t* total) {
         return check(c, scan_with(c, g->scan_tiles, counts, n, offsets, total, g->counters + 4, s),
                      "scan");
     };
     auto plan_and_scans = [&]() {
-        return check(c, lyg_launch_stroke_plan(&L, n, W, room, parts, rv, ri, pgrid, s), "plan") &&
+        return check(c, lyg_launch_stroke_plan(&L, n, cutting.windows, cutting.max_parts, room, parts, rv, ri, pgrid, s), "plan") &&
                scan(parts, parts_off, g->totals + 2) && scan(rv, voff, g->totals + 0) &&
                scan(ri, ioff, g->totals + 1);
     };
@@ -233,7 +233,7 @@ bool capture_stroke_items(lyg_ctx* c, lyg_graph* g, const lyg_batch_in* in,
     if (!check(c, hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal), "begin capture"))
         return false;
     bool ok = check(c, lyg_launch_fill_u32(g->counters, 8, 0, s), "reset") && plan_and_scans();
-    ok = ok && check(c, lyg_launch_stroke_cut(&L, n, W, room, parts, parts_off, rv, ri, voff, ioff,
+    ok = ok && check(c, lyg_launch_stroke_cut(&L, n, cutting.windows, cutting.max_parts, room, parts, parts_off, rv, ri, voff, ioff,
                                               g->cap_extra, g->counters + 6, pgrid, s), "cut");
     ok = ok && check(c, lyg_launch_stroke_heads(&L, n, pgrid, s), "heads");
     ok = ok && check(c, lyg_launch_stroke(&E, 1, egrid, s), "stroke emit (items)");
@@ -396,6 +396,7 @@ int32_t lyg_ctx_set_fill_lds_resident(lyg_ctx* c, int enabled) {
 int32_t lyg_ctx_set_stroke_split(lyg_ctx* c, uint32_t windows_per_part) {
     if (!c || windows_per_part > (1u << 20)) return LYG_ERR_INVALID_ARGUMENT;
     c->stroke_split_windows = windows_per_part;
+    c->stroke_split_auto = false;
     return LYG_OK;
 }
 
@@ -428,8 +429,10 @@ int32_t lyg_autotune_stroke(lyg_ctx* c, const lyg_batch_in* in, const lyg_stroke
     }
     c->stroke_blocks_per_cu = st == LYG_OK ? best_b : keep;
     // then the parts long paths are cut into (0: whole paths)
-    static const uint32_t split_cand[] = {0, 16, 32, 64, 128};
+    static const uint32_t split_cand[] = {0, 2, 4, 8, 16, 32, 64, 128};
     const uint32_t keep_w = c->stroke_split_windows;
+    const bool keep_auto = c->stroke_split_auto;
+    c->stroke_split_auto = false;
     uint32_t best_w = keep_w;
     float best_split = 1e30f;
     for (uint32_t w : split_cand) {
@@ -451,6 +454,7 @@ int32_t lyg_autotune_stroke(lyg_ctx* c, const lyg_batch_in* in, const lyg_stroke
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     c->stroke_split_windows = st == LYG_OK ? best_w : keep_w;
+    c->stroke_split_auto = st == LYG_OK ? false : keep_auto;
     if (chosen) {
         chosen->blocks_per_cu = c->stroke_blocks_per_cu;
         chosen->waves_per_block = 4;

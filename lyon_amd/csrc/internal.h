@@ -24,6 +24,12 @@ struct BatchSpec {
     uint32_t* idx_off;       // device, n + 1
 };
 
+// How a batched stroke cuts its long paths: parts of `windows` windows (0: whole paths), or of
+// as many more as make max_parts parts of a path (0: any number).
+struct Cutting {
+    uint32_t windows, max_parts;
+};
+Cutting stroke_cutting(const lyg_ctx* c, uint32_t n_paths);
 // Batched stroke; *tv / *ti get the totals (also on a capacity error).
 int32_t stroke_batch(lyg_ctx* c, const BatchSpec& b, const OutAlloc& alloc, uint64_t* tv,
                      uint64_t* ti);

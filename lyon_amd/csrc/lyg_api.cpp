@@ -14,6 +14,7 @@
 #include <vector>
 
 #include "../../include/lyg.h"
+#include "lyg_math.h"
 #include "lyg_types.h"
 
 extern "C" {
@@ -22,10 +23,10 @@ hipError_t lyg_launch_stroke_stage_caps(const lyg::StrokeLaunch* L, uint32_t n, 
                                         uint32_t* cap_v, uint32_t* cap_i, hipStream_t s);
 hipError_t lyg_launch_stroke_compact(const lyg::StrokeCompact* C, int grid, hipStream_t s);
 hipError_t lyg_launch_stroke_plan(const lyg::StrokeLaunch* L, uint32_t n_paths,
-                                  uint32_t split_windows, float room_scale, uint32_t* extra,
+                                  uint32_t split_windows, uint32_t max_parts, float room_scale, uint32_t* extra,
                                   uint32_t* rv, uint32_t* ri, int grid, hipStream_t s);
 hipError_t lyg_launch_stroke_cut(const lyg::StrokeLaunch* L, uint32_t n_paths,
-                                 uint32_t split_windows, float room_scale, const uint32_t* extra,
+                                 uint32_t split_windows, uint32_t max_parts, float room_scale, const uint32_t* extra,
                                  const uint32_t* extra_off, const uint32_t* rv,
                                  const uint32_t* ri, const uint32_t* v_off, const uint32_t* i_off,
                                  uint32_t cap_extra, uint32_t* err, int grid, hipStream_t s);
@@ -283,6 +284,7 @@ int32_t stroke_batch_items(lyg_ctx* c, const lygi::BatchSpec& b, const lygi::Out
         !ensure(c, c->st_fallback, 4ull * n + 4))
         return LYG_ERR_DEVICE;
     L.heads = as<lyg::StrokeHeads>(c->st_heads);
+    const lygi::Cutting cutting = lygi::stroke_cutting(c, n);
     uint64_t* h = reinterpret_cast<uint64_t*>(c->h_pinned);
     const int pgrid = (int)std::min<uint32_t>(n, (uint32_t)std::max(1, c->cu_count) * 32u);
     uint32_t* parts = as<uint32_t>(c->st_parts);
@@ -294,7 +296,7 @@ int32_t stroke_batch_items(lyg_ctx* c, const lygi::BatchSpec& b, const lygi::Out
     // 1. the plan of every path (parts beyond the first, staging rooms), its offsets
     if (c->timing) (void)hipEventRecord(c->ev[0], s);
     if (!check(c, lyg_launch_fill_u32(c->d_counters, 8, 0, s), "reset") ||
-        !check(c, lyg_launch_stroke_plan(&L, n, c->stroke_split_windows, c->stroke_room_scale,
+        !check(c, lyg_launch_stroke_plan(&L, n, cutting.windows, cutting.max_parts, c->stroke_room_scale,
                                          parts, rv, ri, pgrid, s),
                "stroke plan") ||
         !check(c, ctx_scan(c, parts, n, parts_off, c->d_totals + 2, c->d_counters + 4, s), "scan") ||
@@ -318,7 +320,7 @@ int32_t stroke_batch_items(lyg_ctx* c, const lygi::BatchSpec& b, const lygi::Out
     L.item_spec = as<lyg::CarryRec>(c->st_spec);
     L.item_end = as<lyg::CarryRec>(c->st_end);
     // the items, and the first points of split paths
-    if (!check(c, lyg_launch_stroke_cut(&L, n, c->stroke_split_windows, c->stroke_room_scale,
+    if (!check(c, lyg_launch_stroke_cut(&L, n, cutting.windows, cutting.max_parts, c->stroke_room_scale,
                                         parts, parts_off, rv, ri, voff, ioff,
                                         (uint32_t)n_extra, nullptr, pgrid, s),
                "stroke cut") ||
@@ -440,6 +442,23 @@ int32_t stroke_batch_items(lyg_ctx* c, const lygi::BatchSpec& b, const lygi::Out
 
 }  // namespace
 
+// A part is a wave of its own, with a window of prologue, and the GPU holds 2,048 of them at
+// once: few paths are cut finer, down to where the prologues cost more than the waves give.
+// us per batch of paths of 4-64 segments (8-110 windows each) at 2 / 4 / 8 / 16 / 32 / 64
+// windows: 8 paths 267 251 267 357 499 912; 64: 344 316 343 409 614 1,024; 512: 718 588 500
+// 514 736 1,141; 2,000: 1,792 1,347 1,124 1,055 1,029 1,424; 4,000: 3,130 2,298 1,857 1,672
+// 1,626 1,988.  Very long paths get longer parts instead of more than 64 K of them in all.
+lygi::Cutting lygi::stroke_cutting(const lyg_ctx* c, uint32_t n_paths) {
+    if (!c->stroke_split_auto) return {c->stroke_split_windows, 0};
+    const uint32_t windows = n_paths <= 4      ? 2
+                             : n_paths <= 128  ? 4
+                             : n_paths <= 512  ? 8
+                             : n_paths <= 1536 ? 16
+                             : n_paths <= 6144 ? 32
+                                               : 64;
+    return {windows, std::max(1u, 65536u / std::max(n_paths, 1u))};
+}
+
 int32_t lygi::stroke_batch(lyg_ctx* c, const lygi::BatchSpec& b, const lygi::OutAlloc& alloc,
                            uint64_t* tv_out, uint64_t* ti_out) {
     const uint32_t n = b.in.n_paths;
@@ -487,6 +506,70 @@ int32_t lygi::stroke_batch(lyg_ctx* c, const lygi::BatchSpec& b, const lygi::Out
 }
 
 namespace {
+
+// Whether a path flattens to at least LONG_PATH_STEPS points (estimated): it is then cut into
+// parts like a path of a batch, ten more launches but no second pass and no lone wave.
+// Closed paths of 4 / 8 / 16 / 64 / 256 cubics (140, 430, 1,000, 3,800, 16,000 points), us a
+// call by one wave in two passes: 174 332 487 1,242 4,455, and first sized right 174 219 323
+// 837 -; cut into parts: 219 220 230 251 392.
+constexpr uint64_t LONG_PATH_STEPS = 512;
+bool long_path(const lyg_path_view& p, float tol) {
+    uint64_t steps = 0;
+    uint32_t at = 0;
+    auto pt = [&](uint32_t i) {
+        return i < p.n_points ? lyg::mk(p.points[2ull * i], p.points[2ull * i + 1]) : lyg::mk(0, 0);
+    };
+    for (uint32_t v = 0; v < p.n_verbs && steps < LONG_PATH_STEPS; ++v) {
+        const uint8_t verb = p.verbs[v];
+        const uint32_t cur = at ? at - 1 : 0;
+        if (verb == LYG_VERB_QUADRATIC) {
+            steps += lyg::seg_count(lyg::quad_wang(pt(cur), pt(at), pt(at + 1), tol));
+            at += 2;
+        } else if (verb == LYG_VERB_CUBIC) {
+            steps += lyg::seg_count(lyg::cubic_wang(pt(cur), pt(at), pt(at + 1), pt(at + 2), tol));
+            at += 3;
+        } else {
+            steps += 1;
+            at += verb != LYG_VERB_END;
+        }
+    }
+    return steps >= LONG_PATH_STEPS;
+}
+
+// One uploaded path (options in in_opts) as a batch of one, into the caller's host arrays.
+int32_t stroke_path_items(lyg_ctx* c, const lyg::PathBatchDev& in, lyg_output* out) {
+    lygi::BatchSpec b{};
+    b.in = in;
+    b.opts = c->in_opts.p;
+    b.vertex_offset = out->vertex_offset;
+    b.vtx_off = as<uint32_t>(c->offs_v);
+    b.idx_off = as<uint32_t>(c->offs_i);
+    uint64_t tv = 0, ti = 0;
+    const int32_t st = lygi::stroke_batch(
+        c, b,
+        [&](uint64_t nv, uint64_t ni, float** v, uint32_t** i) -> int32_t {
+            if (nv > out->vertex_capacity || ni > out->index_capacity) return LYG_ERR_CAPACITY;
+            if (!ensure(c, c->out_v, 8 * nv + 8) || !ensure(c, c->out_i, 4 * ni + 4))
+                return LYG_ERR_DEVICE;
+            *v = as<float>(c->out_v);
+            *i = as<uint32_t>(c->out_i);
+            return LYG_OK;
+        },
+        &tv, &ti);
+    if (st == LYG_OK || st == LYG_ERR_CAPACITY) {
+        out->n_vertices = (uint32_t)tv;
+        out->n_indices = (uint32_t)ti;
+    }
+    if (st != LYG_OK || (tv == 0 && ti == 0)) return st;
+    hipStream_t s = c->stream;
+    if (!check(c, hipMemcpyAsync(out->vertices, c->out_v.p, 8 * tv, hipMemcpyDeviceToHost, s), "D2H") ||
+        (ti && !check(c, hipMemcpyAsync(out->indices, c->out_i.p, 4 * ti, hipMemcpyDeviceToHost, s), "D2H")) ||
+        !check(c, hipStreamSynchronize(s), "sync")) {
+        out->n_vertices = out->n_indices = 0;
+        return LYG_ERR_DEVICE;
+    }
+    return LYG_OK;
+}
 
 bool valid_stroke_opts(const lyg_stroke_options& o) {
     return o.start_cap <= 2 && o.end_cap <= 2 && o.line_join <= 3;
@@ -714,6 +797,9 @@ int32_t lyg_stroke_path(lyg_ctx* c, const lyg_path_view* path, const lyg_stroke_
     L.in.point_off = as<uint32_t>(c->in_offs) + 2;
     L.in.n_paths = 1;
     L.in.first_path = 0;
+    if (c->stroke_staged && lygi::stroke_cutting(c, 1).windows &&
+        long_path(*path, opts->tolerance))
+        return stroke_path_items(c, L.in, out);
     L.opts = as<lyg_stroke_options>(c->in_opts);
     L.opts_stride = 0;
     L.path_nv = as<uint32_t>(c->counts_v);

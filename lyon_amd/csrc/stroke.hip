@@ -885,14 +885,14 @@ __device__ __forceinline__ void item_room(uint64_t steps, uint64_t verbs, uint64
 
 // The cutting of one path into items.  A path of one sub-path with at least
 // 2 * split_windows windows is cut into parts of split_windows windows (part j starts at
-// window j * split_windows of the path; its prologue is the window before it); every
-// other path is one item.  PLAN: counts the parts beyond the first and the staging room
+// window j * split_windows of the path; its prologue is the window before it), or of as many
+// more as make max_parts parts of it (0: any number); every other path is one item.  PLAN: counts the parts beyond the first and the staging room
 // of all of them (*extra, *rv, *ri).  Otherwise: writes the items, item 0 at index
 // `path`, parts 1.. from extra_first, staging rooms from v_base / i_base on (the rooms
 // are recomputed exactly as planned).  One wave.
 template <bool PLAN>
 __device__ void cut_path(const StrokeLaunch& L, uint32_t path, uint32_t split_windows,
-                         float room_scale, uint32_t* extra, uint32_t* rv, uint32_t* ri,
+                         uint32_t max_parts, float room_scale, uint32_t* extra, uint32_t* rv, uint32_t* ri,
                          uint32_t n_extra_planned, uint32_t extra_first, uint32_t v_base,
                          uint32_t i_base) {
     const int l = lane_id();
@@ -911,6 +911,18 @@ __device__ void cut_path(const StrokeLaunch& L, uint32_t path, uint32_t split_wi
         A = arc_count(arc_subdivisions(2.0f * 3.14159265358979323846f, hw, tol));
     // parts of split_windows windows; with PLAN the eligibility is decided at the end
     const bool cut = PLAN ? split_windows > 0 : n_extra_planned > 0;
+    if (cut && max_parts) {
+        uint64_t all = 0;
+        uint32_t pts_before = 0;
+        for (uint32_t v0 = 0; v0 < nverbs; v0 += WAVE) {
+            uint8_t mv;
+            uint32_t off, cnt;
+            all += (chunk_steps(verbs, nverbs, v0, pts, npts, &pts_before, tol, &mv, &off, &cnt) +
+                    WAVE - 1) / WAVE;
+        }
+        const uint64_t most = (all + max_parts - 1) / max_parts;
+        if (most > split_windows) split_windows = (uint32_t)min<uint64_t>(most, 1u << 30);
+    }
     uint64_t steps = 0, windows = 0, sum_v = 0, sum_i = 0;
     uint32_t n_begin = 0, n_end = 0, pt_carry = 0, open_j = 0;
     bool end_last = false;
@@ -924,6 +936,7 @@ __device__ void cut_path(const StrokeLaunch& L, uint32_t path, uint32_t split_wi
     StrokeItem cur{};
     cur.path = path;
     cur.flags = ITEM_FIRST | ITEM_SPLIT;
+    uint64_t next_cut = split_windows;  // the window the next part starts at
     uint64_t cur_steps = 0, cur_verbs = 0;
     auto close_item = [&]() {
         // joins: the verbs that start in the part, the one in progress at its start, and
@@ -957,35 +970,41 @@ __device__ void cut_path(const StrokeLaunch& L, uint32_t path, uint32_t split_wi
             if (!cut) continue;
             const uint32_t nw = (ns + WAVE - 1) / WAVE;
             uint32_t part_s = 0;  // first step of the open part in this chunk
-            for (uint32_t w = 0; w < nw; ++w) {
-                const uint64_t gw = windows + w;
-                if (gw > 0 && gw % split_windows == 0) {
-                    // the open part ends here; the next starts with its prologue
-                    const uint32_t s0 = w * WAVE;
-                    cur_verbs += __popcll(ballot(has && off >= part_s && off < s0));
-                    cur.k1 = k;
-                    cur.w1 = s0;
-                    close_item();
-                    ++open_j;
-                    // the prologue: back over the windows seen until PRO_STEPS steps
+            for (; next_cut < windows + nw; next_cut += split_windows) {
+                // the open part ends here; the next starts with its prologue
+                const uint32_t w = (uint32_t)(next_cut - windows), s0 = w * WAVE;
+                cur_steps += s0 - part_s;
+                cur_verbs += __popcll(ballot(has && off >= part_s && off < s0));
+                cur.k1 = k;
+                cur.w1 = s0;
+                close_item();
+                ++open_j;
+                cur = StrokeItem{};
+                cur.path = path;
+                cur.flags = ITEM_SPLIT;
+                if (w > 0) {
+                    // the window before is a full one of this chunk
+                    cur.k0 = k;
+                    cur.w0 = s0 - WAVE;
+                    cur.pt0 = pt_k;
+                } else {
+                    // back over the windows seen until PRO_STEPS steps
                     uint32_t q = 0, got = 0;
                     const uint32_t avail = n_seen < 4 ? n_seen : 4u;
                     for (; q + 1 < avail && got + rn[q] < PRO_STEPS; ++q) got += rn[q];
-                    cur = StrokeItem{};
-                    cur.path = path;
-                    cur.flags = ITEM_SPLIT;
                     cur.k0 = rk[q];
                     cur.w0 = rw[q];
                     cur.pt0 = rp[q];
-                    cur.ke = k;
-                    cur.we = s0;
-                    cur_steps = 0;
-                    cur_verbs = 0;
-                    part_s = s0;
                 }
-                const uint32_t wn = min((uint32_t)WAVE, ns - w * WAVE);
-                cur_steps += wn;
-                // newest window first in the ring
+                cur.ke = k;
+                cur.we = s0;
+                cur_steps = 0;
+                cur_verbs = 0;
+                part_s = s0;
+            }
+            cur_steps += ns - part_s;
+            // the chunk's last four windows, newest first in the ring
+            for (uint32_t w = nw > 4 ? nw - 4 : 0; w < nw; ++w) {
                 for (int r = 3; r > 0; --r) {
                     rk[r] = rk[r - 1];
                     rw[r] = rw[r - 1];
@@ -995,7 +1014,7 @@ __device__ void cut_path(const StrokeLaunch& L, uint32_t path, uint32_t split_wi
                 rk[0] = k;
                 rw[0] = w * WAVE;
                 rp[0] = pt_k;
-                rn[0] = wn;
+                rn[0] = min((uint32_t)WAVE, ns - w * WAVE);
                 ++n_seen;
             }
             cur_verbs += __popcll(ballot(has && off >= part_s));
@@ -1033,11 +1052,12 @@ __device__ void cut_path(const StrokeLaunch& L, uint32_t path, uint32_t split_wi
 // arrays, which scans turn into item and staging offsets.
 __global__ void __launch_bounds__(WAVE) stroke_plan_kernel(StrokeLaunch L, uint32_t n_paths,
                                                            uint32_t split_windows,
-                                                           float room_scale, uint32_t* extra,
+                                                           uint32_t max_parts, float room_scale,
+                                                           uint32_t* extra,
                                                            uint32_t* rv, uint32_t* ri) {
     for (uint32_t path = blockIdx.x; path < n_paths; path += gridDim.x) {
         uint32_t e, v, i;
-        cut_path<true>(L, path, split_windows, room_scale, &e, &v, &i, 0, 0, 0, 0);
+        cut_path<true>(L, path, split_windows, max_parts, room_scale, &e, &v, &i, 0, 0, 0, 0);
         if (lane_id() == 0) {
             extra[path] = e;
             rv[path] = v;
@@ -1050,7 +1070,7 @@ __global__ void __launch_bounds__(WAVE) stroke_plan_kernel(StrokeLaunch L, uint3
 // the first of the paths before; v_off / i_off: staging), and the path's item range.
 __global__ void __launch_bounds__(WAVE) stroke_cut_kernel(StrokeLaunch L, uint32_t n_paths,
                                                           uint32_t split_windows,
-                                                          float room_scale,
+                                                          uint32_t max_parts, float room_scale,
                                                           const uint32_t* extra,
                                                           const uint32_t* extra_off,
                                                           const uint32_t* rv, const uint32_t* ri,
@@ -1067,8 +1087,8 @@ __global__ void __launch_bounds__(WAVE) stroke_cut_kernel(StrokeLaunch L, uint32
             e = 0;
         }
         uint32_t v = rv[path], i = ri[path];
-        cut_path<false>(L, path, split_windows, room_scale, nullptr, &v, &i, e, ef, v_off[path],
-                        i_off[path]);
+        cut_path<false>(L, path, split_windows, max_parts, room_scale, nullptr, &v, &i, e, ef,
+                        v_off[path], i_off[path]);
         if (lane_id() == 0) {
             StrokeHeads H;
             H.f0 = H.f1 = H.f2 = F2{0.0f, 0.0f};
@@ -1291,21 +1311,21 @@ hipError_t lyg_launch_stroke_compact(const lyg::StrokeCompact* C, int grid, hipS
     return hipGetLastError();
 }
 hipError_t lyg_launch_stroke_plan(const lyg::StrokeLaunch* L, uint32_t n_paths,
-                                  uint32_t split_windows, float room_scale, uint32_t* extra,
+                                  uint32_t split_windows, uint32_t max_parts, float room_scale, uint32_t* extra,
                                   uint32_t* rv, uint32_t* ri, int grid, hipStream_t s) {
     if (n_paths == 0) return hipSuccess;
     hipLaunchKernelGGL(lyg::stroke_plan_kernel, dim3(grid), dim3(lyg::WAVE), 0, s, *L, n_paths,
-                       split_windows, room_scale, extra, rv, ri);
+                       split_windows, max_parts, room_scale, extra, rv, ri);
     return hipGetLastError();
 }
 hipError_t lyg_launch_stroke_cut(const lyg::StrokeLaunch* L, uint32_t n_paths,
-                                 uint32_t split_windows, float room_scale, const uint32_t* extra,
+                                 uint32_t split_windows, uint32_t max_parts, float room_scale, const uint32_t* extra,
                                  const uint32_t* extra_off, const uint32_t* rv,
                                  const uint32_t* ri, const uint32_t* v_off, const uint32_t* i_off,
                                  uint32_t cap_extra, uint32_t* err, int grid, hipStream_t s) {
     if (n_paths == 0) return hipSuccess;
     hipLaunchKernelGGL(lyg::stroke_cut_kernel, dim3(grid), dim3(lyg::WAVE), 0, s, *L, n_paths,
-                       split_windows, room_scale, extra, extra_off, rv, ri, v_off, i_off,
+                       split_windows, max_parts, room_scale, extra, extra_off, rv, ri, v_off, i_off,
                        cap_extra, err);
     return hipGetLastError();
 }

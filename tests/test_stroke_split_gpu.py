@@ -49,6 +49,52 @@ def test_split_matches_whole_walk(closed):
         assert LAST["items"] > len(batch), "no path was split"
 
 
+@pytest.mark.parametrize("n", [1, 4, 5, 128, 129, 512, 513, 1537])
+def test_cutting_by_the_number_of_paths(n):
+    """A context whose cutting was never set picks it by the number of paths: at and around
+    the numbers where it changes the bytes are those of the whole walk.  Plain calls around
+    512 points, where they start to be cut, equal the oracle."""
+    import threading
+
+    from lyon_amd import BuffersBuilder, StrokeOptions, StrokeTessellator, VertexBuffers
+    from lyon_amd.batch import DeviceBatch, StrokeBatcher
+    from oracle import pyoracle as O
+    batch = workloads.stroke_batch(n, 1, 32 if n > 128 else 128, 2048.0, seed=n, closed=n % 2 == 1)
+    opts = workloads.stroke_options(n, tolerance=0.05, seed=n)
+    ref = run(DeviceBatch(batch, opts), 0, vertex_offset=3)
+    paths = []
+    for segs in (510, 511, 512, 513, 640):
+        b = PathBuilder()
+        b.begin((0.0, 0.0))
+        for k in range(segs):
+            b.line_to((3.0 * k, 10.0 * (k % (2 + n % 5))))
+        b.end(n % 2 == 0)
+        paths.append(b.build())
+    got, plain = [], []
+
+    def fresh():  # a context of its own
+        r = StrokeBatcher().run(DeviceBatch(batch, opts), vertex_offset=3)
+        got.append((r.vertex_offsets.copy(), r.index_offsets.copy(),
+                    r.all_vertices().view(np.uint32).copy(), r.all_indices().copy()))
+        for p in paths:
+            buf = VertexBuffers()
+            StrokeTessellator().tessellate_path(p, StrokeOptions(line_width=2.0, tolerance=0.05),
+                                                BuffersBuilder(buf).with_vertex_offset(7))
+            plain.append((buf.vertices, buf.indices))
+
+    t = threading.Thread(target=fresh)
+    t.start()
+    t.join()
+    assert got and len(plain) == len(paths)
+    same(ref, got[0], f"{n} paths")
+    for p, (v, i) in zip(paths, plain):
+        st, rv, ri = O.stroke(p, line_width=2.0, tolerance=0.05, vertex_offset=7)
+        assert st == 0
+        assert np.array_equal(np.asarray(v, np.float32).view(np.uint32),
+                              np.asarray(rv, np.float32).view(np.uint32))
+        assert np.array_equal(np.asarray(i), np.asarray(ri))
+
+
 def test_split_with_short_paths_mixed_in():
     """The 10,000-path batched stroke workload's first 2,000 paths (8-256 segments), most
     of them too short to split, with a few long ones."""
