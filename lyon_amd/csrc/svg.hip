@@ -1,8 +1,10 @@
 // SVG path data on the device: lyon_extra's PathParser (crates/extra/src/parser.rs:140-462)
-// writing into lyon_path's Path layout (BuilderImpl, crates/path/src/path.rs:516-611), one
-// lane per path string.  The parse is a serial state machine over the characters, so a
-// lane walks one string, writing into a staging room sized by the string's length; scans
-// of the counts place the paths end to end and a copy kernel moves them there.
+// writing into lyon_path's Path layout (BuilderImpl, crates/path/src/path.rs:516-611).  The
+// parse is a serial state machine over the characters; a wave per string finds the numbers
+// and commands of a well-formed one in parallel, and a lane walks each string that is not, or
+// that uses what the wave does not handle.  Both write into a staging room sized by the
+// string's length; scans of the counts place the paths end to end and a copy kernel moves
+// them there.
 //
 // Numbers: the parser collects `-? digits* (. digits*)? ([eE] -? digits*)?` and converts it
 // with Rust's `str::parse::<f32>`, which is correctly rounded (round half to even) for
@@ -22,6 +24,7 @@
 #include "arc_core.h"
 #include "lyg_math.h"
 #include "lyg_types.h"
+#include "wave.h"
 
 namespace lyg {
 
@@ -682,16 +685,320 @@ __device__ void parse_svg(const uint8_t* s, uint32_t a, uint32_t b, int nattr, i
     if (S.non_ascii) E = PErr{LYG_SVG_ERR_NON_ASCII, S.na_line, S.na_col, 0u};
 }
 
+// ---- a wave per string ------------------------------------------------------------------
+// A string the parser accepts from beginning to end, without arcs and smooth quadratics, is a
+// sequence of numbers and command letters that can be found without walking it: 64
+// characters at a time, ballots tell the classes apart, and a character starts a number by
+// itself, the one before it and the last one before it that is no digit.  Lanes then convert
+// a number each, and a lane applies one command (or one repetition of it) each; only the
+// current point goes from lane to lane, as relative commands add to it in order.  Whatever
+// does not fit (errors, non-ASCII text, arcs, digits or exponents beyond the one-operation
+// conversion, letters that start no command) is noticed, and the string is left to the serial
+// parser below, which reports errors where they are.  That a lane's numbers are the ones the
+// serial parser reads: they do not overlap, and their lengths add up to all the characters of
+// numbers, so what lies between two of them is separators and command letters.
+//
+// Bound by VALU issue and the latency of a wave's ~90 instructions per 64 characters.  4,096
+// strings of 8-64 segments (1.1 KB on average): 2,368 us with a lane per string, the text read
+// byte by byte (now only for the strings left over); 72 us so.
+constexpr uint32_t SVG_CHARS = 1024;  // characters looked at together
+constexpr uint32_t SVG_AHEAD = 64;    // and beyond, for a number that ends there
+constexpr int SVG_WAVES = 4;
+
+struct SvgText {
+    uint8_t text[SVG_CHARS + SVG_AHEAD];
+    uint16_t start[SVG_CHARS + WAVE];  // where the numbers start
+};
+
+// The number at t[p], read as the serial parser would; its end in *end.  False when it is not
+// one, or not one that a double operation converts.
+__device__ __forceinline__ bool wave_number(const uint8_t* t, uint32_t p, uint32_t* end, float* out) {
+    const uint32_t lim = SVG_CHARS + SVG_AHEAD - 1;  // t[lim] is never part of a number read here
+    uint32_t ch = t[p];
+    const bool neg = ch == '-';
+    if (neg) ch = t[++p];
+    uint64_t w = 0;
+    int kept = 0, mant = 0, shift = 0;
+    bool frac = false;
+    for (;;) {
+        if (is_digit(ch)) {
+            const uint32_t d = ch - '0';
+            ++mant;
+            kept += (kept != 0) | (d != 0);
+            w = w * 10 + d;
+            shift -= frac;
+        } else if (ch == '.' && !frac) {
+            frac = true;
+        } else {
+            break;
+        }
+        if (p >= lim) return false;
+        ch = t[++p];
+    }
+    int ex = 0;
+    if (ch == 'e' || ch == 'E') {
+        if (p >= lim) return false;
+        ch = t[++p];
+        const bool eneg = ch == '-';
+        if (eneg && p < lim) ch = t[++p];
+        int ed = 0;
+        while (is_digit(ch) && p < lim) {
+            ex = ex < 100000 ? ex * 10 + (int)(ch - '0') : ex;
+            ++ed;
+            ch = t[++p];
+        }
+        if (ed == 0) return false;
+        if (eneg) ex = -ex;
+    }
+    *end = p;
+    if (mant == 0 || kept > 19 || p >= lim) return false;
+    const int e = ex + shift;
+    uint32_t bits;
+    if (w == 0 || e + kept <= -46) bits = 0;
+    else if (e + kept > 39) bits = 0x7f800000u;
+    else if (!fast_round(w, e, &bits)) return false;
+    *out = __uint_as_float(bits | (neg ? 0x80000000u : 0u));
+    return true;
+}
+
+// Parses the string if it can; false leaves it to the serial parser.  vals, cmds: room for as
+// many numbers and command words as the string has characters.
+__device__ bool wave_svg(const uint8_t* s, uint32_t len, SvgText& T, float* vals, uint32_t* cmds,
+                         Out<true>& O) {
+    const int l = lane_id();
+    if (len >= 1u << 24) return false;  // a command word holds its first number in 24 bits
+    uint32_t n_num = 0, n_cmd = 0, in_numbers = 0, covered = 0, prev_end = 0;
+    uint32_t last_c = ' ';
+    // the last character that is no digit: 0 closes a number before a '.', 1 a sign that starts
+    // one, 2 a separator or command
+    uint32_t last_kind = 2;
+    for (uint32_t base = 0; base < len; base += SVG_CHARS) {
+        wave_sync();
+        const uint32_t here = len - base < SVG_CHARS ? len - base : SVG_CHARS;
+        uint32_t c[SVG_CHARS / WAVE + 1];
+#pragma unroll
+        for (uint32_t r = 0; r <= SVG_CHARS / WAVE; ++r) {
+            const uint32_t i = base + r * WAVE + (uint32_t)l;
+            c[r] = i < len ? (uint32_t)s[i] : 0u;
+        }
+#pragma unroll
+        for (uint32_t r = 0; r <= SVG_CHARS / WAVE; ++r) T.text[r * WAVE + l] = (uint8_t)c[r];
+        wave_sync();
+        uint32_t n_here = 0;
+        for (uint32_t r = 0; r * WAVE < here; ++r) {
+            uint32_t ch = T.text[r * WAVE + l];
+            if (r * WAVE + (uint32_t)l >= here) ch = ' ';
+            const uint32_t lower = ch | 0x20u;
+            const bool digit = is_digit(ch), dot = ch == '.', minus = ch == '-';
+            const uint32_t before = from_lane_before(ch, last_c);
+            const bool expo = lower == 'e' && (is_digit(before) || before == '.');
+            const bool sep = is_ws(ch) || ch == ',';
+            const bool cmd = lower == 'm' || lower == 'l' || lower == 'h' || lower == 'v' ||
+                             lower == 'q' || lower == 's' || lower == 'c' || lower == 'z';
+            if (ballot(!(digit || dot || minus || expo || sep || cmd)) != 0) return false;
+            const uint64_t dm = ballot(digit), xm = ballot(expo);
+            const bool exp_sign = minus && (before | 0x20u) == 'e';
+            const uint64_t closing = ballot(dot || exp_sign) | xm;
+            const uint64_t sign = ballot(minus && !exp_sign);
+            const uint64_t below = ~dm & mask_lt(l);
+            uint32_t kind = last_kind;
+            if (below) {
+                const int q = highest_bit(below);
+                kind = (closing >> q & 1u) ? 0u : (sign >> q & 1u) ? 1u : 2u;
+            }
+            const bool after_sep = is_ws(before) || before == ',' ||
+                                   ((before | 0x20u) >= 'a' && (before | 0x20u) <= 'z' &&
+                                    (before | 0x20u) != 'e');
+            const bool starts = (digit && after_sep) || (minus && !exp_sign) ||
+                                (dot && (kind == 0u || (kind == 2u && !is_digit(before))));
+            const uint64_t sm = ballot(starts), cm = ballot(cmd);
+            const uint32_t nb = (uint32_t)__builtin_popcountll(sm & mask_lt(l));
+            if (starts) T.start[n_here + nb] = (uint16_t)(r * WAVE + l);
+            if (cmd)
+                cmds[n_cmd + (uint32_t)__builtin_popcountll(cm & mask_lt(l))] =
+                    ch << 24 | (n_num + n_here + nb);
+            in_numbers += (uint32_t)__builtin_popcountll(dm | closing | sign);
+            n_here += (uint32_t)__builtin_popcountll(sm);
+            n_cmd += (uint32_t)__builtin_popcountll(cm);
+            last_c = readlane_u(ch, WAVE - 1);
+            const uint64_t other = ~dm;
+            if (other) {
+                const int q = highest_bit(other);
+                last_kind = (closing >> q & 1u) ? 0u : (sign >> q & 1u) ? 1u : 2u;
+            }
+        }
+        wave_sync();
+        for (uint32_t k0 = 0; k0 < n_here; k0 += WAVE) {
+            const uint32_t k = k0 + (uint32_t)l;
+            bool bad = false;
+            uint32_t n = 0, end = 0;
+            if (k < n_here) {
+                const uint32_t p = T.start[k];
+                float v = 0.0f;
+                end = p;
+                bad = !wave_number(T.text, p, &end, &v);
+                vals[n_num + k] = v;
+                n = end - p;
+                bad |= k + 1 < n_here && end > T.start[k + 1];
+                bad |= k == 0 && base + p < prev_end;
+            }
+            if (ballot(bad) != 0) return false;
+            covered += readlane_u(incl_scan(n), WAVE - 1);
+            const uint32_t lastk = n_here - 1 - k0;
+            if (lastk < (uint32_t)WAVE) prev_end = base + readlane_u(end, (int)lastk);
+        }
+        n_num += n_here;
+    }
+    if (covered != in_numbers) return false;
+    if (n_cmd == 0) return n_num == 0;
+    wave_sync();
+    vec2 cur = mk(0.0f, 0.0f), first = cur, pc = cur;
+    uint32_t has_pc = 0, last_cmd = 0;
+    for (uint32_t g = 0; g < n_cmd; g += WAVE) {
+        // a lane per command: its repetitions
+        const uint32_t m = g + (uint32_t)l;
+        const uint32_t word = m < n_cmd ? cmds[m] : 0u;
+        const uint32_t letter = word >> 24, at = word & 0xffffffu;
+        const uint32_t upto = m + 1 < n_cmd ? cmds[m + 1] & 0xffffffu : n_num;
+        const uint32_t cnt = upto - at, lc = letter | 0x20u;
+        const uint32_t args = lc == 'c' ? 6u : lc == 'q' || lc == 's' ? 4u
+                            : lc == 'm' || lc == 'l' ? 2u : lc == 'z' ? 0u : 1u;
+        uint32_t reps = 0;
+        bool bad = false;
+        const uint32_t before = from_lane_before(letter, last_cmd);
+        if (m < n_cmd) {
+            reps = args == 6u ? cnt / 6u : args == 4u ? cnt / 4u : args == 2u ? cnt / 2u : cnt;
+            bad = reps * args != cnt || reps == 0u;
+            if (args == 0u) {
+                bad = cnt != 0u;
+                reps = 1u;
+            }
+            // the first command, and the one after a Close, begin a sub-path; no numbers
+            // come before the first
+            if (m == 0) bad |= lc != 'm' || at != 0u;
+            else bad |= (before | 0x20u) == 'z' && lc != 'm';
+        }
+        if (ballot(bad) != 0) return false;
+        const uint32_t incl = incl_scan(reps), excl = incl - reps;
+        const uint32_t total = readlane_u(incl, WAVE - 1);
+        const uint32_t n_lanes = n_cmd - g < (uint32_t)WAVE ? n_cmd - g : (uint32_t)WAVE;
+        for (uint32_t s0 = 0; s0 < total; s0 += WAVE) {
+            // a lane per repetition: the last command whose first one is not past it
+            const uint32_t n = total - s0 < (uint32_t)WAVE ? total - s0 : (uint32_t)WAVE;
+            const uint32_t rep = s0 + (uint32_t)l;
+            uint32_t j = 0;
+#pragma unroll
+            for (uint32_t step = 32; step; step >>= 1) {
+                const uint32_t e = shfl_u(excl, (int)(j + step < 63u ? j + step : 63u));
+                if (j + step < n_lanes && e <= rep) j += step;
+            }
+            const uint32_t L0 = shfl_u(letter, (int)j), nth = rep - shfl_u(excl, (int)j);
+            const uint32_t na = shfl_u(args, (int)j);
+            const uint32_t arg0 = shfl_u(at, (int)j) + nth * na;
+            const uint32_t bl = shfl_u(before, (int)j);
+            const bool on = (uint32_t)l < n;
+            uint32_t op = L0 | 0x20u;
+            const bool rel = L0 >= 'a';
+            const bool move = op == 'm' && nth == 0u;
+            if (op == 'm' && nth != 0u) op = 'l';
+            float a[6];
+#pragma unroll
+            for (uint32_t q = 0; q < 6; ++q) a[q] = on && q < na ? vals[arg0 + q] : 0.0f;
+            // the current point, lane to lane: set, moved, kept or back at the first point
+            const vec2 v = op == 'c' ? mk(a[4], a[5])
+                         : op == 'q' || op == 's' ? mk(a[2], a[3])
+                         : op == 'v' ? mk(0.0f, a[0]) : mk(a[0], a[1]);
+            vec2 end = v, fst = v;
+            for (uint32_t q = 0; q < n; ++q) {
+                const vec2 p = from_lane_before(end, cur), f = from_lane_before(fst, first);
+                end.x = op == 'z' ? f.x : op == 'v' ? p.x : rel ? v.x + p.x : v.x;
+                end.y = op == 'z' ? f.y : op == 'h' ? p.y : rel ? v.y + p.y : v.y;
+                fst = move ? end : f;
+            }
+            const vec2 from = from_lane_before(end, cur);
+            auto P = [&](float x, float y) { return rel ? mk(x + from.x, y + from.y) : mk(x, y); };
+            const vec2 p0 = P(a[0], a[1]), p1 = P(a[2], a[3]);
+            const vec2 c2 = op == 'c' ? p1 : p0;  // of a cubic
+            const bool is_c = op == 'c' || op == 's';
+            const vec2 pcb = from_lane_before(c2, pc);
+            const bool hpc = from_lane_before(is_c ? 1u : 0u, has_pc) != 0u;
+            const vec2 smooth = hpc ? add(from, sub(from, pcb)) : from;
+            const bool close_before = move && (bl | 0x20u) != 'z' && bl != 0u;
+            const uint32_t nv = !on ? 0u : close_before ? 2u : 1u;
+            const uint32_t np = !on ? 0u : is_c ? 3u : op == 'q' ? 2u : 1u;
+            const uint32_t vi = incl_scan(nv), pi = incl_scan(np);
+            uint32_t ov = O.nv + vi - nv, op_ = O.np + pi - np;
+            auto verb = [&](uint32_t x) {
+                if (ov < O.cap_v) O.verbs[ov] = (uint8_t)x;
+                ++ov;
+            };
+            auto point = [&](vec2 x) {
+                if (op_ < O.cap_p) O.points[op_] = make_float2(x.x, x.y);
+                ++op_;
+            };
+            if (on) {
+                if (close_before) verb(5);
+                verb(move ? 3u : is_c ? 2u : op == 'q' ? 1u : op == 'z' ? 4u : 0u);
+                if (is_c) point(op == 'c' ? p0 : smooth);
+                if (is_c) point(c2);
+                if (op == 'q') point(p0);
+                point(end);
+            }
+            O.nv += readlane_u(vi, WAVE - 1);
+            O.np += readlane_u(pi, WAVE - 1);
+            const int last = (int)n - 1;
+            cur = readlane_v(end, last);
+            first = readlane_v(fst, last);
+            pc = readlane_v(c2, last);
+            has_pc = readlane_u(is_c ? 1u : 0u, last);
+        }
+        last_cmd = readlane_u(letter, (int)n_lanes - 1);
+    }
+    if ((last_cmd | 0x20u) != 'z') {
+        if (l == 0 && O.nv < O.cap_v) O.verbs[O.nv] = 5;
+        ++O.nv;
+    }
+    return true;
+}
+
 }  // namespace
 
+// A wave per string; the staging rooms as svg_parse_kernel's.  The upper half of a string's
+// points room (twice as many as its characters; a point takes at least one) holds its numbers
+// and command words meanwhile.
+__global__ void __launch_bounds__(WAVE* SVG_WAVES) svg_wave_kernel(SvgLaunch L) {
+    __shared__ SvgText texts[SVG_WAVES];
+    const uint32_t w = readlane_u(threadIdx.x / WAVE, 0);
+    const uint32_t i = blockIdx.x * SVG_WAVES + w;
+    if (i >= L.n) return;
+    const uint32_t a = L.text_off[i], len = L.text_off[i + 1] - a;
+    float2* pts = reinterpret_cast<float2*>(L.points) + 2ull * a + 2ull * i;
+    float* vals = reinterpret_cast<float*>(pts + len + 2u);
+    Out<true> O{L.verbs + a + 2ull * i, pts, 0, 0, mk(0.0f, 0.0f), len + 2, 2 * len + 2};
+    const bool done = wave_svg(L.text + a, len, texts[w], vals,
+                               reinterpret_cast<uint32_t*>(vals) + len, O);
+    if (lane_id() != 0) return;
+    if (!done) {
+        L.serial[atomicAdd(L.n_serial, 1u)] = i;
+        return;
+    }
+    L.counts_v[i] = O.nv;
+    L.counts_p[i] = O.np;
+    if (O.nv > O.cap_v || O.np > len + 2u) atomicAdd(L.n_errors + 1, 1u);
+    if (L.errors)
+        for (int k = 0; k < 4; ++k) L.errors[4ull * i + k] = 0;
+}
+
+// The serial parser, a lane per string.
 // Parses string i into its staging room: verbs at text_off[i] + 2 i (room: its bytes + 2),
 // points at 2 text_off[i] + 2 i (room: twice its bytes + 2).  Every command consumes at
 // least one character and makes at most one verb and two points per character (an arc's
 // eight quadratics need eleven), plus the End of the last sub-path; a string whose output
 // would not fit anyway raises the overflow counter instead of writing past its room.
 __global__ void __launch_bounds__(256) svg_parse_kernel(SvgLaunch L) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= L.n) return;
+    uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= (L.serial ? *L.n_serial : L.n)) return;
+    if (L.serial) i = L.serial[i];
     const uint32_t a = L.text_off[i], b = L.text_off[i + 1];
     PErr E;
     Out<true> O{L.verbs + a + 2ull * i, reinterpret_cast<float2*>(L.points) + 2ull * a + 2ull * i,
@@ -732,6 +1039,9 @@ extern "C" {
 
 hipError_t lyg_launch_svg_parse(const lyg::SvgLaunch* L, hipStream_t s) {
     if (L->n == 0) return hipSuccess;
+    if (L->serial)
+        hipLaunchKernelGGL(lyg::svg_wave_kernel, dim3((L->n - 1) / lyg::SVG_WAVES + 1),
+                           dim3(lyg::WAVE * lyg::SVG_WAVES), 0, s, *L);
     hipLaunchKernelGGL(lyg::svg_parse_kernel, dim3((L->n + 255) / 256), dim3(256), 0, s, *L);
     return hipGetLastError();
 }

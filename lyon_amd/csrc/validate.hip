@@ -312,12 +312,6 @@ struct AreaShared {
     float t[AREA_TABLE];     // t of the run's points 0, 16, 32, ...
 };
 
-// The running value, from the lane before each lane (lane 0 takes `carry`).
-__device__ __forceinline__ float from_lane_before(float v, float carry) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(
-        __builtin_bit_cast(int, carry), __builtin_bit_cast(int, v), 0x138, 0xf, 0xf, false));  // wave_shr:1
-}
-
 __global__ void __launch_bounds__(WAVE* AREA_WAVES) signed_area_kernel(ValidateLaunch L) {
     __shared__ AreaShared shared[AREA_WAVES];
     const int l = lane_id();

@@ -90,6 +90,17 @@ __device__ __forceinline__ uint32_t incl_max_u32(uint32_t v) {
     x = x > t ? x : t;
     return x;
 }
+// v of the lane before each lane; lane 0 takes `carry`.
+__device__ __forceinline__ uint32_t from_lane_before(uint32_t v, uint32_t carry) {
+    return (uint32_t)__builtin_amdgcn_update_dpp((int)carry, (int)v, 0x138, 0xf, 0xf, false);  // wave_shr:1
+}
+__device__ __forceinline__ float from_lane_before(float v, float carry) {
+    return __builtin_bit_cast(float, from_lane_before(__builtin_bit_cast(uint32_t, v),
+                                                      __builtin_bit_cast(uint32_t, carry)));
+}
+__device__ __forceinline__ vec2 from_lane_before(vec2 v, vec2 carry) {
+    return mk(from_lane_before(v.x, carry.x), from_lane_before(v.y, carry.y));
+}
 __device__ __forceinline__ int highest_bit(uint64_t m) { return m ? 63 - __builtin_clzll(m) : -1; }
 // Last index i in [0, n) with a[i] <= key, for a non-decreasing `a` with a[0] <= key (0
 // when n == 0), searched by the whole wave: each round probes 64 evenly spaced entries at

@@ -152,6 +152,60 @@ def test_random_svg_matches_oracle(arcs):
     assert 0 < n_err < len(strings)
 
 
+@pytest.mark.parametrize("length", [1, 63, 64, 65, 1000, 1023, 1024, 1025, 2048, 5000])
+def test_strings_around_what_a_wave_looks_at(length):
+    """Well-formed strings (no arcs, no smooth quadratics, so that a wave parses each) whose
+    lengths and tokens lie around 64 and 1,024 characters: glued numbers, exponents, relative
+    and repeated commands, Close and the commands after it, paddings of every kind; and the
+    same strings with one thing the wave leaves to the serial parser."""
+    rng = np.random.default_rng(length)
+    nums = ["1.5.25", "-.5-3", "2e1.5", "1.e1-7", "-0", "0.000", "00012.5", "16777217", "-1E-2",
+            ".1", "123456.789", "3.4028235677973366e38", "1e-46", "9007199254740993"]
+    args = {"M": 2, "L": 2, "H": 1, "V": 1, "Q": 4, "C": 6, "S": 4}
+    strings = []
+    for k in range(40):
+        out = ["M", "1", "2"] if k % 4 else ["m", "-1", "-2"]
+        size = 5
+        while size < length:
+            c = "MLHVQCS"[int(rng.integers(0, 7))]
+            letter = c if rng.random() < 0.5 else c.lower()
+            need = args[c] * int(rng.integers(1, 4))
+            word = letter
+            while need > 0:
+                if rng.random() < 0.3:
+                    t = nums[int(rng.integers(0, len(nums)))]
+                    n = {"1.5.25": 2, "-.5-3": 2, "2e1.5": 2, "1.e1-7": 2}.get(t, 1)
+                    if n > need:
+                        continue
+                else:
+                    t, n = "%.*f" % (int(rng.integers(0, 7)), rng.uniform(-900, 900)), 1
+                need -= n
+                word += [" ", ",", "\n", " , ", "\t\t"][int(rng.integers(0, 5))] + t
+            if rng.random() < 0.15:
+                word += "zM3 4" if rng.random() < 0.5 else "Z\nm.5.5"
+            out.append(word)
+            size += len(word)
+        s = " ".join(out)
+        s += " " * max(0, length - len(s)) if k % 3 else "Z"
+        strings.append(" " * int(rng.integers(0, 70)) * (k % 2) + s)
+    for k, odd in enumerate(["T1 2", "A1 1 0 0 1 5 5", "L1", "L1 2 3", "L1e9e", "x", "L1.2.", "é",
+                             "Z5", "ZL1 2", "L1 +2", "L0.1234567890123456789012 1", "e", "L--1 2"]):
+        strings.append(strings[k] + odd)
+        cut = len(strings[k]) // 2
+        strings.append(strings[k][:cut] + odd + strings[k][cut:])
+    strings.append("1 2 L 3 4")
+    strings.append("L 3 4")
+    batch, errs = S.parse_paths(strings)
+    for i, s in enumerate(strings):
+        rv, rp, re = O.parse_svg(s)
+        p = batch.path(i)
+        assert _err(errs[i]) == re.tolist(), (s, errs[i], re)
+        assert p.verbs.tolist() == rv.tolist(), s
+        assert p.points.shape == rp.shape, s
+        assert np.array_equal(p.points, rp, equal_nan=True), s
+    assert all(e is None for e in errs[:40])
+
+
 def test_round_trip_of_the_stroke_workload():
     """Full size: the 10,000-path stroke workload (and a closed variant) written as SVG
     path data with 9 significant digits parses back to the same verbs and bit-identical
