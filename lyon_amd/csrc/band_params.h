@@ -69,7 +69,7 @@ struct Params {
     uint32_t* b_rec_cap;  // room per band; scanned into b_rec_off (n_bands + 1)
     uint32_t* b_rec_off;
     uint32_t* b_nrec;
-    uint4* rec;           // (left edge, right edge, top event, bottom event)
+    uint4* rec;           // (left edge, right edge (band-local), top event, bottom event)
     // output
     uint32_t* r_nv;       // per record: vertices (0, 3 or 4), then triangles
     uint32_t* r_nt;

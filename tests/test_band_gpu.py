@@ -76,6 +76,43 @@ def test_corpus_coverage_and_area():
     assert checked > 100
 
 
+@pytest.mark.parametrize("spokes", [1, 2, 3, 4, 5, 8, 14, 31, 33, 70])
+def test_many_edges_meet_at_one_point(spokes):
+    """Thin triangles above and below one point (that many pairs of ends and of starts there,
+    around the numbers an event rebuilds at once), edges through it that end elsewhere, and
+    the rest of the scene on both sides: the covered region of the textbook winding number.
+    More than 32 positions at one event end with Internal."""
+    from lyon_amd.path import PathBuilder
+    b = PathBuilder()
+
+    def tri(*p):
+        b.begin(p[0])
+        for q in p[1:]:
+            b.line_to(q)
+        b.end(True)
+
+    for k in range(spokes):
+        x = 64.0 * (k - spokes / 2.0)
+        if k % 3 != 1:
+            tri((0.0, 0.0), (x - 9.0, -512.0), (x + 9.0 + k, -512.0))
+        if k % 3 != 2:
+            tri((0.0, 0.0), (x - 13.0, 512.0), (x + 7.0 + k, 512.0))
+    for k in range(min(spokes, 6)):  # a straight edge through the point
+        tri((-512.0 + 64.0 * k, -256.0), (512.0 - 64.0 * k, 256.0), (900.0, 300.0 + 8.0 * k))
+    for k in range(40):
+        tri((-900.0 + 3.0 * k, -300.0 + k), (-880.0 + 2.0 * k, 310.0), (-905.0 + 3.0 * k, 330.0))
+    path = b.build()
+    for rule in (0, 1):
+        if spokes > 16:
+            with pytest.raises(TessellationError) as e:
+                banded(path, rule)
+            assert e.value.code == 5
+            continue
+        v, i = banded(path, rule)
+        r = O.winding_compare(path, 0.1, rule, v, i, n=1024, eps=eps_for(path.points))
+        assert r["mismatch"] == 0 and r["overlap_a"] == 0, (rule, r)
+
+
 def test_walk_prefix_against_lyon():
     """A 65,536-vertex random walk (the large fill workload's generator), closed: the banded
     fill covers exactly the winding-number region and its area.  The restated lyon sweep's
