@@ -244,8 +244,8 @@ struct VWPar {
     uint8_t* pflags;
     float* src_t;
     uint32_t* src_id;
-    // edges with side lines: (slot, point) pairs in any order, four floats per slot
-    uint32_t* att_pair;
+    // edges with side lines (a path's at att_off): point (~0: unused slot), four floats
+    uint32_t* att_point;
     float* att_n;
     // per window
     uint32_t *win_att, *win_nv, *win_ni;
@@ -255,7 +255,7 @@ struct VWPar {
     uint32_t n_tails;
     uint32_t *slow_list, *cands, *dirty;
     uint32_t cand_cap, dirty_cap;
-    // [0] edges with side lines, [1] serial paths, [2] candidates, [3] windows to count
+    // [1] serial paths, [2] candidates, [3] windows to count
     // again, [4] a list overflowed
     uint32_t* ctr;
     const uint32_t *vtx_off, *idx_off;

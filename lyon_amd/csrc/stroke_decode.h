@@ -121,6 +121,49 @@ __device__ __forceinline__ void decode_verb(uint8_t verb, const float* pts, uint
     }
 }
 
+// lyon's serial t (t = t + step from 0) of a chunk's curve steps [b0, b0 + T_SPAN) at every
+// 16th step of the chunk: a lane per verb adds its curve's steps up, one addition per step (the
+// closed form once, where a curve starts far before b0), and a window's lanes then need 15
+// additions at most.  b0 is a multiple of 16; steps from b1 on are left out.
+static constexpr uint32_t T_SPAN = 4096;
+__device__ __forceinline__ void t_table(float* tab, const VRec& r, bool in, uint32_t b0,
+                                        uint32_t b1) {
+    const uint32_t kind = r.kind & 0xffu;
+    if (!in || (kind != K_QUAD && kind != K_CUBIC)) return;
+    if (b1 - b0 > T_SPAN) b1 = b0 + T_SPAN;
+#pragma unroll 1
+    for (int half = 0; half < 2; ++half) {
+        const uint32_t start = half ? r.off + r.nA : r.off, n = half ? r.nB : r.nA;
+        const float step = half ? r.sB : r.sA;
+        const uint32_t lo = ((start > b0 ? start : b0) + 15u) & ~15u;
+        const uint32_t hi = start + n < b1 ? start + n : b1;
+        if (lo >= hi) continue;
+        const uint32_t j = lo - start + 1u;
+        float t = 0.0f;
+        if (j <= 64u) {
+            for (uint32_t q = 0; q < j; ++q) t = t + step;
+        } else {
+            t = tchain(step, j);
+        }
+        for (uint32_t g = lo; g < hi; g += 16u) {
+            tab[(g - b0) >> 4] = t;
+#pragma unroll
+            for (int q = 0; q < 16; ++q) t = t + step;
+        }
+    }
+}
+// t of the chunk's step g, the j-th (from 1) of its curve, from a table of b0 on.
+__device__ __forceinline__ float t_at(const float* tab, uint32_t b0, uint32_t g, uint32_t j,
+                                      float step) {
+    const uint32_t ahead = g & 15u;
+    const bool listed = j > ahead;  // the curve holds the listed step before g
+    float t = listed ? tab[((g - b0) >> 4) & (T_SPAN / 16u - 1u)] : 0.0f;
+    const uint32_t more = listed ? ahead : j;
+#pragma unroll
+    for (uint32_t q = 0; q < 15u; ++q) t = q < more ? t + step : t;
+    return t;
+}
+
 __device__ __forceinline__ uint32_t verb_points(uint8_t v) {
     switch (v) {
         case LYG_VERB_BEGIN:

@@ -928,11 +928,14 @@ __global__ void __launch_bounds__(64) vw_plan_kernel(VWPar P) {
 
 // Wave per path: windows of 64 flattened points, one per lane; the kept ones are written
 // end to end with their running length.  Bound by that length's serial f32 sum (64 dependent
-// additions per window) and the t chain; the rest of a window is lane-parallel.
+// additions per window); the rest of a window is lane-parallel.  10,000 paths, 81 M points:
+// 7.6 ms with the windows' t chains in closed form and the edges with side lines listed through
+// one counter for all paths, 2.6 ms with t_table and a list per path.
 __global__ void __launch_bounds__(64) vw_points_kernel(VWPar P) {
     using namespace vw;
     __shared__ VRec recs[WAVE];
     __shared__ VX vxs[WAVE];
+    __shared__ float ts_tab[T_SPAN / 16];
     const int l = lane_id();
     const float nan = __builtin_nanf("");
     for (uint32_t path = blockIdx.x; path < P.in.n_paths; path += gridDim.x) {
@@ -990,18 +993,19 @@ __global__ void __launch_bounds__(64) vw_points_kernel(VWPar P) {
                 vxs[l] = x;
             }
             wave_sync();
-            // t chain of the curve piece the previous window ended in (key, steps, units)
-            uint32_t ch_key = 0xffffffffu, ch_j = 0;
-            uint64_t ch_T = 0;
             for (uint32_t w0 = 0; w0 < nsteps; w0 += WAVE) {
+                const uint32_t t0_step = w0 & ~(T_SPAN - 1u);
+                if (w0 == t0_step) {
+                    wave_sync();
+                    t_table(ts_tab, r, in, w0, nsteps);
+                    wave_sync();
+                }
                 const uint32_t g = w0 + (uint32_t)l;
                 const bool valid = g < nsteps;
                 vec2 pos = mk(nan, nan);
                 float hw = 0.0f, tw = 1.0f;
                 uint32_t id0 = 0, id1 = 0;
                 bool isB = false, isE = false, close = false, flat = false;
-                uint32_t my_key = 0xffffffffu, my_j = 0;
-                uint64_t my_T = 0;
                 if (valid) {
                     int lo = 0, hi = (int)nch - 1;  // last verb whose offset <= g
                     while (lo < hi) {
@@ -1029,23 +1033,8 @@ __global__ void __launch_bounds__(64) vw_points_kernel(VWPar P) {
                         if (j == (inA ? vr.nA : vr.nB)) {
                             pos = inA ? vr.toA : vr.toB;
                         } else {
-                            const float sstep = inA ? vr.sA : vr.sB;
-                            const uint32_t key = ((uint32_t)lo << 1) | (inA ? 0u : 1u);
-                            const bool cont = key == ch_key && ch_j < j;
-                            uint64_t T;
-                            if (!cont && j <= (uint32_t)WAVE) {
-                                t1 = 0.0f;
-                                for (uint32_t s = 0; s < j; ++s) t1 = t1 + sstep;
-                                T = tchain_units_of(sstep, t1);
-                            } else {
-                                T = tchain_units_from(tchain_mant(sstep), j, cont ? ch_j : 0u,
-                                                      cont ? ch_T : 0ull);
-                                t1 = tchain_value(sstep, T);
-                            }
+                            t1 = t_at(ts_tab, t0_step, g, j, inA ? vr.sA : vr.sB);
                             pos = horner(vr, !inA, inA && cubic, t1);
-                            my_key = key;
-                            my_j = j;
-                            my_T = T;
                         }
                         const bool split = !cubic && vx.ts > 0.0f;
                         const float t0 = split && !inA ? vx.ts : 0.0f;
@@ -1055,13 +1044,6 @@ __global__ void __launch_bounds__(64) vw_points_kernel(VWPar P) {
                         flat = t1 != 1.0f;
                         if (tw != 1.0f) id0 = vx.id0;
                     }
-                }
-                {
-                    const int lastl = (int)min((uint32_t)WAVE, nsteps - w0) - 1;
-                    ch_key = readlane_u(my_key, lastl);
-                    ch_j = readlane_u(my_j, lastl);
-                    ch_T = (uint64_t)readlane_u((uint32_t)my_T, lastl) |
-                           ((uint64_t)readlane_u((uint32_t)(my_T >> 32), lastl) << 32);
                 }
                 const uint64_t validm = ballot(valid), begm = ballot(isB), endm = ballot(isE);
                 const int nvalid = __builtin_popcountll(validm);
@@ -1168,15 +1150,8 @@ __global__ void __launch_bounds__(64) vw_points_kernel(VWPar P) {
                     const uint32_t tot = (uint32_t)__builtin_popcountll(attm);
                     if (n_att + tot > acap) {  // cannot happen: a curve's last point only
                         if (l == 0) mark_slow(P, path);
-                    } else {
-                        uint32_t g0 = 0;
-                        if (l == 0) g0 = atomicAdd(&P.ctr[0], tot);
-                        g0 = readlane_u(g0, 0);
-                        if (att) {
-                            const uint32_t k = g0 + (ord - n_att);
-                            P.att_pair[2ull * k] = abase + ord;
-                            P.att_pair[2ull * k + 1] = kbase + kidx;
-                        }
+                    } else if (att) {
+                        P.att_point[abase + ord] = kbase + kidx;
                     }
                     n_att += tot;
                 }
@@ -1216,12 +1191,13 @@ __global__ void __launch_bounds__(64) vw_points_kernel(VWPar P) {
     }
 }
 
-// Lane per edge with an endpoint at one end: the normals of its two side lines (attachments).
+// Lane per slot of an edge with an endpoint at one end: the normals of its two side lines (attachments).
 __global__ void __launch_bounds__(256) vw_att_kernel(VWPar P) {
-    const uint32_t n = P.ctr[0];
+    const uint32_t n = P.att_off[P.in.n_paths];
     const float PI = 3.14159265358979323846f;
-    for (uint32_t k = blockIdx.x * 256u + threadIdx.x; k < n; k += gridDim.x * 256u) {
-        const uint32_t slot = P.att_pair[2ull * k], i = P.att_pair[2ull * k + 1];
+    for (uint32_t slot = blockIdx.x * 256u + threadIdx.x; slot < n; slot += gridDim.x * 256u) {
+        const uint32_t i = P.att_point[slot];
+        if (i == 0xffffffffu) continue;
         const float4 p0 = reinterpret_cast<const float4*>(P.rec)[i - 1];
         const float4 p1 = reinterpret_cast<const float4*>(P.rec)[i];
         const vec2 e = sub(mk(p1.x, p1.y), mk(p0.x, p0.y));

@@ -94,7 +94,7 @@ int32_t vw_plan(lyg_ctx* c, const lyg::StrokeVWLaunch& L, uint32_t n, bool want_
     P.dirty_cap = 4u * P.cand_cap;
     const bool src = want_attrs;
     if (!ensure(c, c->vw_rec, 16 * raw) || !ensure(c, c->vw_flags, raw) ||
-        (src && !ensure(c, c->vw_src, 12 * raw)) || !ensure(c, c->vw_att, 24 * att) ||
+        (src && !ensure(c, c->vw_src, 12 * raw)) || !ensure(c, c->vw_att, 20 * att) ||
         !ensure(c, c->vw_win, 4 * (5 * win + 2)) ||
         !ensure(c, c->vw_tails, sizeof(lyg::VWTail) * tails) ||
         !ensure(c, c->vw_lists, 4ull * (2ull * P.cand_cap + P.dirty_cap))) {
@@ -108,7 +108,9 @@ int32_t vw_plan(lyg_ctx* c, const lyg::StrokeVWLaunch& L, uint32_t n, bool want_
         P.src_id = as<uint32_t>(c->vw_src) + raw;
     }
     P.att_n = as<float>(c->vw_att);
-    P.att_pair = as<uint32_t>(c->vw_att) + 4 * att;
+    P.att_point = as<uint32_t>(c->vw_att) + 4 * att;
+    if (!check(c, lyg_launch_fill_u32(P.att_point, (uint32_t)att, 0xffffffffu, s), "reset"))
+        return LYG_ERR_DEVICE;
     u = as<uint32_t>(c->vw_win);
     P.win_att = take(win);
     P.win_nv = take(win);

@@ -304,6 +304,20 @@ def to_svg(path):
     return " ".join(out)
 
 
+def counted_curves(b, counts, tol, rng, attrs=None):
+    """One sub-path of curves on builder b, cubics and quadratics in turn, that flatten to about
+    `counts` points each (Wang: n = sqrt(6 d / (8 tol)) for a second difference d)."""
+    b.begin((0.0, 0.0), *([] if attrs is None else [attrs()]))
+    for k, n in enumerate(counts):
+        d = float(n) ** 2 * 8.0 * tol / 6.0
+        x, y = rng.random(2) * 100.0
+        a = [] if attrs is None else [attrs()]
+        if k % 2:
+            b.quadratic_bezier_to((x + 1.5 * d, y), (x, y + 3.0), *a)
+        else:
+            b.cubic_bezier_to((x, y + d), (x - d, y), (x + 5.0, y - 2.0), *a)
+
+
 def random_svg(rng, n_cmds=12, arcs=True, corrupt=0.0):
     """Random SVG path data over every command (absolute and relative, implicit repeats,
     mixed separators, exponents, signs glued to the previous number), optionally with

@@ -12,6 +12,7 @@ same status."""
 import numpy as np
 import pytest
 
+from helpers import counted_curves
 from lyon_amd import (BuffersBuilder, LineCap, LineJoin, StrokeOptions, StrokeTessellator,
                       VertexBuffers)
 from lyon_amd import workloads
@@ -197,6 +198,26 @@ def test_sub_paths_around_the_window_size(join, closed):
         rv, ri = ref_vw(path, opts)
         same += np.array_equal(i, ri) and close_enough(v, rv, 300.0)
     assert same >= 0.97 * len(paths), same
+
+
+@pytest.mark.parametrize("counts", [[1, 2, 15, 16, 17, 18], [31, 33, 63, 65, 80], [4000, 90, 70],
+                                    [4080, 16, 50], [4095, 4097], [64, 9000, 20]])
+def test_curves_around_the_listed_steps(counts):
+    """Curves of as many points as the t of every 16th of 4,096 steps is listed for, starting
+    and ending around those numbers."""
+    rng = np.random.default_rng(counts[0])
+    tol = 1e-2
+    opts = StrokeOptions(line_width=1.0, line_join=LineJoin.Miter, tolerance=tol,
+                         variable_line_width=0)
+    for shift in (0, 1, 15):
+        b = PathBuilder(1)
+        counted_curves(b, [3] * shift + counts, tol, rng, lambda: [rng.uniform(0.5, 2.0)])
+        b.end(shift == 1)
+        path = b.build()
+        v, i = gpu_vw(path, opts)
+        rv, ri = ref_vw(path, opts)
+        assert np.array_equal(i, ri), shift
+        assert close_enough(v, rv, float(np.ptp(np.asarray(path.points), axis=0).max())), shift
 
 
 def test_batch_equals_plain_calls():
