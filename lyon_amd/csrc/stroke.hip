@@ -32,7 +32,6 @@ namespace lyg {
 static constexpr int WAVES_PER_BLOCK = 4;
 
 enum : uint32_t { F_BEGIN = 1u, F_END = 2u, F_CLOSE = 4u, F_FLAT = 8u };
-static constexpr uint32_t NO_CHAIN = 0xffffffffu;
 
 // What a lane publishes about the kept point before it (for the next lane's join).
 struct Pub {
@@ -180,6 +179,12 @@ struct WalkRange {
     uint32_t pt0;  // points consumed by the verbs before chunk k0
 };
 
+// A walk's LDS: a chunk's decoded verbs, and t_table of T_SPAN of its steps.
+struct WalkLds {
+    VRec recs[WAVE];
+    float t[T_SPAN / 16];
+};
+
 // Walks [R.k0, R.k1) of one path with the whole wave from the carry `c`, which it
 // updates; c.run_v / c.run_i count the vertices / triangles from the range's emitted
 // start.  EMIT: output to [v0, v_end) / [i0, i_end) of the output arrays.  `spec`: where
@@ -187,8 +192,8 @@ struct WalkRange {
 template <bool EMIT, bool RANGED = true>
 __device__ __forceinline__ void stroke_walk(const StrokeLaunch& L, uint32_t gpath, const WalkRange& R,
                             Carry& c, uint32_t path_v0, uint32_t path_v_end, uint32_t path_i0,
-                            uint32_t path_i_end, CarryRec* spec, VRec* recs, ArcJob* arc_jobs,
-                            uint32_t* arc_first, uint32_t* arc_c0) {
+                            uint32_t path_i_end, CarryRec* spec, WalkLds* lds,
+                            ArcJob* arc_jobs, uint32_t* arc_first, uint32_t* arc_c0) {
     const int l = lane_id();
     const uint32_t vb = L.in.verb_off[gpath], ve = L.in.verb_off[gpath + 1];
     const uint32_t pb = L.in.point_off[gpath], pe = L.in.point_off[gpath + 1];
@@ -198,6 +203,8 @@ __device__ __forceinline__ void stroke_walk(const StrokeLaunch& L, uint32_t gpat
     const lyg_stroke_options o = L.opts[L.opts_stride ? gpath : 0];
     const SParams P = make_params(o, L.nsub_thr);
     const float nan = __builtin_nanf("");
+    VRec* recs = lds->recs;
+    float* t_tab = lds->t;
     bool started = !RANGED || (R.k0 == R.ke && R.w0 == R.we);
 
     uint32_t pt_carry = RANGED ? R.pt0 : 0u;
@@ -229,11 +236,17 @@ __device__ __forceinline__ void stroke_walk(const StrokeLaunch& L, uint32_t gpat
         wave_sync();
 
         // ---- 2. windows of 64 steps ----------------------------------------------------
-        // t chain of the curve half the previous window ended in (key, steps, units)
-        uint32_t ch_key = NO_CHAIN, ch_j = 0;
-        uint64_t ch_T = 0;
-        for (uint32_t w0 = RANGED && kch == R.k0 ? R.w0 : 0u; w0 < nsteps; w0 += WAVE) {
+        const uint32_t w_first = RANGED && kch == R.k0 ? R.w0 : 0u;
+        uint32_t t_first = 0;  // the step t_tab starts at
+        for (uint32_t w0 = w_first; w0 < nsteps; w0 += WAVE) {
             if (RANGED && kch == R.k1 && w0 >= R.w1) break;
+            if (w0 == w_first || w0 - t_first == T_SPAN) {
+                t_first = w0;
+                wave_sync();
+                t_table(t_tab, r, (uint32_t)l < nch, w0,
+                        RANGED && kch == R.k1 && R.w1 < nsteps ? R.w1 : nsteps);
+                wave_sync();
+            }
             const bool silent = RANGED && (kch < R.ke || (kch == R.ke && w0 < R.we));
             if (!silent && !started) {
                 // the prologue ends: ids from here on count from the range's start
@@ -248,8 +261,6 @@ __device__ __forceinline__ void stroke_walk(const StrokeLaunch& L, uint32_t gpat
             const bool valid = g < nsteps;
             vec2 pos = mk(nan, nan);
             uint32_t flags = 0;
-            uint32_t my_key = NO_CHAIN, my_j = 0;  // the t chain this lane evaluated
-            uint64_t my_T = 0;
             if (valid) {
                 // last verb whose offset <= g
                 int lo = 0, hi = (int)nch - 1;
@@ -275,29 +286,9 @@ __device__ __forceinline__ void stroke_walk(const StrokeLaunch& L, uint32_t gpat
                     if (kk + 1 == (inA ? vr.nA : vr.nB)) {
                         pos = inA ? vr.toA : vr.toB;
                     } else {
-                        // t after kk + 1 steps, continuing the previous window's chain
-                        // when this curve half carries on from it
-                        const float sstep = inA ? vr.sA : vr.sB;
-                        const uint32_t key = ((uint32_t)lo << 1) | (inA ? 0u : 1u);
-                        const uint32_t j = kk + 1;
-                        const bool cont = key == ch_key && ch_j < j;
-                        float t;
-                        uint64_t T;
-                        if (!cont && j <= (uint32_t)WAVE) {
-                            // a curve half that starts in this window: lyon's serial sum
-                            t = 0.0f;
-                            for (uint32_t q = 0; q < j; ++q) t = t + sstep;
-                            T = tchain_units_of(sstep, t);
-                        } else {
-                            T = tchain_units_from(tchain_mant(sstep), j, cont ? ch_j : 0u,
-                                                  cont ? ch_T : 0ull);
-                            t = tchain_value(sstep, T);
-                        }
+                        const float t = t_at(t_tab, t_first, g, kk + 1, inA ? vr.sA : vr.sB);
                         pos = horner(vr, !inA, inA && cubic, t);
                         flags = F_FLAT;
-                        my_key = key;
-                        my_j = j;
-                        my_T = T;
                     }
                 }
             }
@@ -604,14 +595,6 @@ __device__ __forceinline__ void stroke_walk(const StrokeLaunch& L, uint32_t gpat
                     newcnt = c.sp_cnt + __builtin_popcountll(keptm);
                     newm = last_mnec;
                 }
-                // the t chain of the last step, for the next window
-                {
-                    const int src = lastv < 0 ? 0 : lastv;
-                    ch_key = lastv < 0 ? NO_CHAIN : readlane_u(my_key, src);
-                    ch_j = readlane_u(my_j, src);
-                    ch_T = (uint64_t)readlane_u((uint32_t)my_T, src) |
-                           ((uint64_t)readlane_u((uint32_t)(my_T >> 32), src) << 32);
-                }
                 if (lk >= 0) c.last_kept = lkp;
                 if (last_is_end) c.last_kept = mk(nan, nan);
                 // firsts of the (possibly new) current sub-path
@@ -649,7 +632,7 @@ __device__ __forceinline__ void stroke_walk(const StrokeLaunch& L, uint32_t gpat
 
 // Walks one whole path with the whole wave.  Returns (vertices, triangles).
 template <bool EMIT>
-__device__ void stroke_one_path(const StrokeLaunch& L, uint32_t gpath, VRec* recs,
+__device__ void stroke_one_path(const StrokeLaunch& L, uint32_t gpath, WalkLds* lds,
                                 ArcJob* arc_jobs, uint32_t* arc_first, uint32_t* arc_c0,
                                 uint32_t* out_nv, uint32_t* out_ni) {
     uint32_t path_v0 = 0, path_i0 = 0, path_v_end = 0, path_i_end = 0;
@@ -668,7 +651,7 @@ __device__ void stroke_one_path(const StrokeLaunch& L, uint32_t gpath, VRec* rec
     carry_init(c);
     const WalkRange R{0, 0, 0, 0, 0xffffffffu, 0, 0};
     stroke_walk<EMIT, false>(L, gpath, R, c, path_v0, path_v_end, path_i0, path_i_end, nullptr,
-                             recs, arc_jobs, arc_first, arc_c0);
+                             lds, arc_jobs, arc_first, arc_c0);
     *out_nv = c.run_v;
     *out_ni = c.run_i;
 }
@@ -677,7 +660,7 @@ __device__ void stroke_one_path(const StrokeLaunch& L, uint32_t gpath, VRec* rec
 // into its own staging room with item-local ids; stores its exact counts and, for parts,
 // the carries the check compares.
 template <bool EMIT>
-__device__ void stroke_item(const StrokeLaunch& L, uint32_t item, VRec* recs, ArcJob* arc_jobs,
+__device__ void stroke_item(const StrokeLaunch& L, uint32_t item, WalkLds* lds, ArcJob* arc_jobs,
                             uint32_t* arc_first, uint32_t* arc_c0) {
     const StrokeItem it = L.items[item];
     const WalkRange R{it.k0, it.w0, it.ke, it.we, it.k1, it.w1, it.pt0};
@@ -691,7 +674,7 @@ __device__ void stroke_item(const StrokeLaunch& L, uint32_t item, VRec* recs, Ar
     if (first) carry_init(c);
     else carry_mid_path(c, L.heads[it.path]);
     stroke_walk<EMIT>(L, it.path, R, c, it.v_off, it.v_off + it.v_room, it.i_off,
-                      it.i_off + it.i_room, first ? nullptr : L.item_spec + item, recs, arc_jobs,
+                      it.i_off + it.i_room, first ? nullptr : L.item_spec + item, lds, arc_jobs,
                       arc_first, arc_c0);
     if (lane_id() == 0) {
         L.items[item].nv = c.run_v;
@@ -713,16 +696,18 @@ __device__ __forceinline__ uint32_t next_path(uint32_t* counter) {
 // chain of shuffles, LDS reads and scans), so occupancy beats spill-free code.  Measured
 // on the 10,000-path stroke workload: count pass 11.4 ms at 1 wave/SIMD, 7.2 at 2, 6.0 at
 // 4; emit pass 16.0 ms at 1, 11.1 at 2, 15.7 at 4 (its larger state spills too much).
+// A window's t by t_table: 10,000 paths, 81 M points, the emit pass 5.38 -> 4.82 ms (each
+// window's lanes went through the closed form, integer divisions per binade, before).
 template <bool EMIT, bool ITEMS>
 __global__ void __launch_bounds__(WAVE* WAVES_PER_BLOCK)
     LYG_WAVES_PER_EU(EMIT ? 2 : 4) stroke_kernel(StrokeLaunch L) {
-    __shared__ VRec recs_all[WAVES_PER_BLOCK][WAVE];
+    __shared__ WalkLds lds_all[WAVES_PER_BLOCK];
     // the emit pass's cooperative arcs: two jobs per lane, first node and side split
     constexpr int AW = EMIT ? WAVES_PER_BLOCK : 1;
     __shared__ ArcJob arcs_all[AW][EMIT ? 2 * WAVE : 1];
     __shared__ uint32_t arc_first_all[AW][EMIT ? WAVE : 1], arc_c0_all[AW][EMIT ? WAVE : 1];
     const int w = threadIdx.x / WAVE;
-    VRec* recs = recs_all[w];
+    WalkLds* lds = &lds_all[w];
     ArcJob* arc_jobs = arcs_all[EMIT ? w : 0];
     uint32_t* arc_first = arc_first_all[EMIT ? w : 0];
     uint32_t* arc_c0 = arc_c0_all[EMIT ? w : 0];
@@ -735,7 +720,7 @@ __global__ void __launch_bounds__(WAVE* WAVES_PER_BLOCK)
                                                           (unsigned long long)L.cap_extra)
                           : L.n_items;
         while (pid < n_work) {
-            stroke_item<EMIT>(L, pid, recs, arc_jobs, arc_first, arc_c0);
+            stroke_item<EMIT>(L, pid, lds, arc_jobs, arc_first, arc_c0);
             pid = next_path(L.work_counter);
         }
         return;
@@ -744,7 +729,7 @@ __global__ void __launch_bounds__(WAVE* WAVES_PER_BLOCK)
     while (pid < n_list) {
         const uint32_t gp = L.path_list ? L.path_list[pid] : L.in.first_path + pid;
         uint32_t nv = 0, ni = 0;
-        stroke_one_path<EMIT>(L, gp, recs, arc_jobs, arc_first, arc_c0, &nv, &ni);
+        stroke_one_path<EMIT>(L, gp, lds, arc_jobs, arc_first, arc_c0, &nv, &ni);
         if (!EMIT || L.store_counts) {
             // every lane holds the totals; lane 0's store is the only one kept
             uint32_t* dst_v = L.path_nv + gp;
@@ -1106,13 +1091,13 @@ __global__ void __launch_bounds__(WAVE) stroke_cut_kernel(StrokeLaunch L, uint32
 // alone (a path whose first window does not keep three points is marked to be walked
 // again whole).
 __global__ void __launch_bounds__(WAVE) stroke_heads_kernel(StrokeLaunch L, uint32_t n_paths) {
-    __shared__ VRec recs[WAVE];
+    __shared__ WalkLds lds;
     for (uint32_t path = blockIdx.x; path < n_paths; path += gridDim.x) {
         if (L.heads[path].n_items < 2) continue;
         Carry c;
         carry_init(c);
         const WalkRange R{0, 0, 0, 0, 0, (uint32_t)WAVE, 0};
-        stroke_walk<false>(L, path, R, c, 0, 0, 0, 0, nullptr, recs, nullptr, nullptr, nullptr);
+        stroke_walk<false>(L, path, R, c, 0, 0, 0, 0, nullptr, &lds, nullptr, nullptr, nullptr);
         if (lane_id() == 0) {
             StrokeHeads* H = L.heads + path;
             if (c.sp_cnt >= 3 && !c.prev_end) {
@@ -1153,7 +1138,7 @@ __device__ __forceinline__ bool carry_match(const CarryRec& e, uint32_t nv_prev,
 // outgrew its staging room.
 __global__ void __launch_bounds__(WAVE) stroke_items_verify_kernel(StrokeLaunch L,
                                                                    uint32_t n_paths) {
-    __shared__ VRec recs[WAVE];
+    __shared__ WalkLds lds;
     const int l = lane_id();
     for (uint32_t path = blockIdx.x; path < n_paths; path += gridDim.x) {
         const uint32_t n = L.heads[path].n_items;
@@ -1190,7 +1175,7 @@ __global__ void __launch_bounds__(WAVE) stroke_items_verify_kernel(StrokeLaunch 
             Carry c;
             carry_init(c);
             const WalkRange R{0, 0, 0, 0, 0xffffffffu, 0, 0};
-            stroke_walk<false, false>(L, path, R, c, 0, 0, 0, 0, nullptr, recs, nullptr, nullptr,
+            stroke_walk<false, false>(L, path, R, c, 0, 0, 0, 0, nullptr, &lds, nullptr, nullptr,
                                       nullptr);
             vrun = c.run_v;
             irun = 3u * c.run_i;

@@ -7,7 +7,8 @@ import itertools
 import numpy as np
 import pytest
 
-from helpers import assert_same_geometry, bbox_diag, empty_caps_path, square_paths
+from helpers import (assert_same_geometry, bbox_diag, counted_curves, empty_caps_path,
+                     square_paths)
 from lyon_amd import (BuffersBuilder, LineCap, LineJoin, PathBuilder, StrokeOptions,
                       StrokeTessellator, VertexBuffers)
 from lyon_amd import workloads
@@ -50,6 +51,20 @@ ALL_OPTS = [StrokeOptions(line_width=w, line_join=j, start_cap=c, end_cap=c2, to
                 (4.0, LineJoin.Miter, LineCap.Butt, LineCap.Square, 0.05, 4.0),
                 (8.0, LineJoin.Round, LineCap.Square, LineCap.Round, 0.05, 2.0),
             ]]
+
+
+@pytest.mark.parametrize("counts", [[1, 2, 15, 16, 17, 18], [31, 33, 63, 65, 80], [4000, 90, 70],
+                                    [4080, 16, 50], [4095, 4097], [64, 9000, 20]])
+def test_curves_around_the_listed_steps(counts):
+    """Curves of as many points as the t of every 16th of 4,096 steps is listed for, starting
+    and ending around those numbers."""
+    rng = np.random.default_rng(counts[0])
+    opts = StrokeOptions(line_width=1.0, line_join=LineJoin.Miter, tolerance=1e-2)
+    for shift in (0, 1, 15):
+        b = PathBuilder()
+        counted_curves(b, [3] * shift + counts, opts.tolerance, rng)
+        b.end(shift == 1)
+        check(b.build(), opts, f"{counts} after {shift}")
 
 
 def test_square_kats():
