@@ -228,186 +228,155 @@ __global__ void fill_status_out_kernel(const uint32_t* st, uint32_t* out, uint32
                                   : v == 0xffffffffu ? (uint32_t)LYG_ERR_INTERNAL : v;
 }
 
-// Upper bound of the events of each path (one thread per path): flattened edges (the
-// swapped-curve Wang counts) plus one vertex event per edge, plus the closing edges; and the
-// sum of its segments' degrees, which a horizontal line crosses at most that often.
-__global__ void fill_bound_kernel(FillLaunch L, uint32_t n_paths, uint32_t* bound,
-                                  uint32_t* degree) {
-    uint32_t path = blockIdx.x * blockDim.x + threadIdx.x;
-    if (path >= n_paths) return;
-    const lyg_fill_options o = L.opts[L.opts_stride ? path : 0];
-    const uint32_t vb = L.in.verb_off[path], ve = L.in.verb_off[path + 1];
-    const uint32_t pb = L.in.point_off[path], pe = L.in.point_off[path + 1];
-    const float2* pts = reinterpret_cast<const float2*>(L.in.points) + pb;
-    const uint32_t npts = pe - pb;
-    auto ld = [&](uint32_t i) -> vec2 {
-        if (i >= npts) return mk(0.0f, 0.0f);
-        float2 q = pts[i];
-        return mk(q.x, q.y);
-    };
-    uint64_t e = 0, d = 0;
-    uint32_t p = 0;
-    vec2 cur = mk(0.0f, 0.0f);
-    float tol = o.tolerance > 0.0f ? o.tolerance : 1.0f;
-    for (uint32_t v = vb; v < ve; ++v) {
-        uint8_t verb = L.in.verbs[v];
-        if (verb == LYG_VERB_BEGIN) {
-            cur = ld(p++);
-        } else if (verb == LYG_VERB_LINE) {
-            cur = ld(p++);
-            e += 1;
-            d += 1;
-        } else if (verb == LYG_VERB_QUADRATIC) {
-            vec2 c = ld(p), t = ld(p + 1);
-            p += 2;
-            d += 2;
-            // the swapped curve can round one count differently: +1
-            e += seg_count(quad_wang(cur, c, t, tol)) + 1;
-            cur = t;
-        } else if (verb == LYG_VERB_CUBIC) {
-            vec2 c1 = ld(p), c2 = ld(p + 1), t = ld(p + 2);
-            p += 3;
-            d += 3;
-            e += seg_count(cubic_wang(cur, c1, c2, t, tol)) + 1;
-            cur = t;
-        } else {
-            if (verb == LYG_VERB_CLOSE) p++;
-            e += 1;
-            d += 1;
-        }
-    }
-    degree[path] = d > 0xffffffffull ? 0xffffffffu : (uint32_t)d;
-    uint64_t bnd = 2 * e + 16;
-    bound[path] = bnd > 0xffffffffull ? 0xffffffffu : (uint32_t)bnd;
-}
+// What sizes a path's first sweep, by a wave per path with a lane per verb:
+//   * an upper bound of its events: flattened edges (the swapped-curve Wang counts) plus one
+//     vertex event per edge, plus the closing edges;
+//   * the sum of its segments' degrees, which a horizontal line crosses at most that often;
+//   * an estimate of its self-intersections, which its output and its pending events grow with
+//     and the event bound does not see.  Two segments can only cross if their boxes (of the
+//     control points, padded by the tolerance: the flattened edges lie within) overlap; the
+//     estimate counts one crossing per overlapping pair of non-consecutive segments and one per
+//     cubic (its possible loop).  For polygons this is an upper bound (two line segments cross
+//     at most once); for curves it is a typical count rather than the worst case (a cubic pair
+//     may cross up to 9 times, most overlapping pairs do not cross at all), and a path that
+//     outgrows it is swept again with more room.  Paths with more than INTER_MAX_VERBS verbs
+//     get 0 (their first attempt is sized from the events).
+// CAP: the boxes one block's LDS holds.  The first launch takes every path, and raises `more`
+// for those with more verbs than its boxes, up to INTER_MAX_VERBS; the second (over > 0) counts
+// the pairs of those with more than `over`.  1,000 glyphs: 120 us when a thread walked a path,
+// once for the bound and once for boxes in memory, 13 us so.
+static constexpr uint32_t INTER_MAX_VERBS = 4096, INTER_FEW_VERBS = 1024;
 
-// ---- intersection estimate ---------------------------------------------------------------
-// A path's output and its pending-event heap grow with its self-intersections, which the
-// event bound does not see.  Sizing the first attempt from an estimate of them keeps
-// self-intersecting paths (stars) from running out of room and being swept again.
-//
-struct VBox {
-    float x0, y0, x1, y1;
-    uint32_t deg;
-};
-
-// fill_boxes_kernel: one record per verb of every path (thread per path, in verb order):
-// the bounding box of the segment's control points padded by the tolerance (the
-// flattened edges lie within it) and its degree (1 line or closing edge, 2 quadratic,
-// 3 cubic; 0 for Begin and empty closing edges).
-__global__ void fill_boxes_kernel(FillLaunch L, uint32_t n_paths, VBox* rec) {
-    uint32_t path = blockIdx.x * blockDim.x + threadIdx.x;
-    if (path >= n_paths) return;
-    const lyg_fill_options o = L.opts[L.opts_stride ? path : 0];
-    const uint32_t vb = L.in.verb_off[path], ve = L.in.verb_off[path + 1];
-    const uint32_t pb = L.in.point_off[path], pe = L.in.point_off[path + 1];
-    const float2* pts = reinterpret_cast<const float2*>(L.in.points) + pb;
-    const uint32_t npts = pe - pb;
-    auto ld = [&](uint32_t i) -> vec2 {
-        if (i >= npts) return mk(0.0f, 0.0f);
-        float2 q = pts[i];
-        return mk(q.x, q.y);
-    };
-    const float pad = o.tolerance > 0.0f ? o.tolerance : 0.0f;
-    auto box = [&](uint32_t deg, vec2 a, vec2 b, vec2 c, vec2 d) {
-        VBox r;
-        r.x0 = ffmin(ffmin(a.x, b.x), ffmin(c.x, d.x)) - pad;
-        r.y0 = ffmin(ffmin(a.y, b.y), ffmin(c.y, d.y)) - pad;
-        r.x1 = ffmax(ffmax(a.x, b.x), ffmax(c.x, d.x)) + pad;
-        r.y1 = ffmax(ffmax(a.y, b.y), ffmax(c.y, d.y)) + pad;
-        r.deg = deg;
-        return r;
-    };
-    uint32_t p = 0;
-    vec2 cur = mk(0.0f, 0.0f), start = cur;
-    for (uint32_t v = vb; v < ve; ++v) {
-        const uint8_t verb = L.in.verbs[v];
-        VBox r = box(0, cur, cur, cur, cur);
-        if (verb == LYG_VERB_BEGIN) {
-            cur = start = ld(p++);
-        } else if (verb == LYG_VERB_LINE) {
-            vec2 t = ld(p++);
-            r = box(1, cur, t, t, t);
-            cur = t;
-        } else if (verb == LYG_VERB_QUADRATIC) {
-            vec2 c = ld(p), t = ld(p + 1);
-            p += 2;
-            r = box(2, cur, c, t, t);
-            cur = t;
-        } else if (verb == LYG_VERB_CUBIC) {
-            vec2 c1 = ld(p), c2 = ld(p + 1), t = ld(p + 2);
-            p += 3;
-            r = box(3, cur, c1, c2, t);
-            cur = t;
-        } else {
-            if (verb == LYG_VERB_CLOSE) p++;
-            // every sub-path is closed by an edge back to its start (event_queue.rs:661-682)
-            if (!(cur.x == start.x && cur.y == start.y)) r = box(1, cur, start, start, start);
-            cur = start;
-        }
-        rec[v] = r;
-    }
-}
-
-// fill_inter_kernel: one wave per path.  Two segments can only cross if their boxes
-// overlap; the estimate counts one crossing per overlapping pair of non-consecutive
-// segments and one per cubic (its possible loop).  For polygons this is an upper bound
-// (two line segments cross at most once); for curves it is a typical count rather than
-// the worst case (a cubic pair may cross up to 9 times, most overlapping pairs do not
-// cross at all), and a path that outgrows it is swept again with more room.  Paths with
-// more than INTER_MAX_VERBS verbs get 0 (their first attempt is sized from the events).
-static constexpr uint32_t INTER_MAX_VERBS = 4096;
-__global__ void __launch_bounds__(WAVE) fill_inter_kernel(FillLaunch L, uint32_t n_paths,
-                                                         const VBox* rec, uint32_t* inter) {
+template <uint32_t CAP>
+__global__ void __launch_bounds__(WAVE) fill_measure_kernel(FillLaunch L, uint32_t over,
+                                                            uint32_t* bound, uint32_t* degree,
+                                                            uint32_t* inter, uint32_t* more) {
+    __shared__ float4 boxes[CAP];
     const uint32_t path = blockIdx.x;
-    if (path >= n_paths) return;
-    const uint32_t vb = L.in.verb_off[path], ve = L.in.verb_off[path + 1];
-    const uint32_t nv = ve - vb;
     const int l = lane_id();
-    uint32_t acc = 0;
-    if (nv <= INTER_MAX_VERBS) {
-        for (uint32_t i = (uint32_t)l; i < nv; i += WAVE) {
-            const VBox a = rec[vb + i];
-            if (a.deg == 0) continue;
-            if (a.deg == 3) acc += 1;
-            for (uint32_t j = i + 2; j < nv; ++j) {
-                const VBox b = rec[vb + j];
-                if (b.deg == 0) continue;
-                if (a.x0 > b.x1 || b.x0 > a.x1 || a.y0 > b.y1 || b.y0 > a.y1) continue;
-                acc += 1;
+    const uint32_t vb = L.in.verb_off[path], nv = L.in.verb_off[path + 1] - vb;
+    if (over && (nv <= over || nv > CAP)) return;
+    const lyg_fill_options o = L.opts[L.opts_stride ? path : 0];
+    const uint32_t pb = L.in.point_off[path], npts = L.in.point_off[path + 1] - pb;
+    const float2* pts = reinterpret_cast<const float2*>(L.in.points) + pb;
+    // the point before index i (0: none)
+    auto before = [&](uint32_t i) -> vec2 {
+        if (i == 0u || i > npts) return mk(0.0f, 0.0f);
+        const float2 q = pts[i - 1u];
+        return mk(q.x, q.y);
+    };
+    const float tol = o.tolerance > 0.0f ? o.tolerance : 1.0f;
+    const float pad = o.tolerance > 0.0f ? o.tolerance : 0.0f;
+    const bool pairs = nv <= CAP;
+    uint64_t edges = 0;
+    uint32_t deg = 0, acc = 0;
+    // points before the chunk; 1 + the index of the last point of a Begin, Line or curve and of
+    // the latest Begin; whether the verb before the chunk ends a sub-path
+    uint32_t pt = 0, c_cur = 0, c_beg = 0, c_end = 0;
+    for (uint32_t v0 = 0; v0 < nv; v0 += WAVE) {
+        const bool in = v0 + (uint32_t)l < nv;
+        const uint32_t verb = in ? (uint32_t)L.in.verbs[vb + v0 + l] : 0xffu;
+        const uint32_t np = verb == LYG_VERB_CUBIC ? 3u : verb == LYG_VERB_QUADRATIC ? 2u
+                          : verb <= LYG_VERB_CLOSE ? 1u : 0u;
+        const uint32_t upto = pt + incl_scan(np), first = upto - np;
+        const bool moves = verb <= LYG_VERB_BEGIN;  // Line, curves, Begin
+        uint32_t m = incl_max_u32(moves ? upto : 0u);
+        m = m > c_cur ? m : c_cur;
+        uint32_t beg = incl_max_u32(verb == LYG_VERB_BEGIN ? upto : 0u);
+        beg = beg > c_beg ? beg : c_beg;
+        const uint32_t is_end = in && !moves ? 1u : 0u;
+        const uint32_t cur_i = from_lane_before(m, c_cur);
+        const bool after_end = from_lane_before(is_end, c_end) != 0u;
+        const vec2 q1 = before(first + 1u), q2 = before(first + 2u), q3 = before(first + 3u);
+        uint32_t d = 0;
+        float4 bx = make_float4(INFINITY, INFINITY, -INFINITY, -INFINITY);
+        if (in && verb != LYG_VERB_BEGIN) {
+            if (over == 0u) {
+                const vec2 cur = before(cur_i);
+                // the swapped curve can round one count differently: +1
+                if (verb == LYG_VERB_QUADRATIC) {
+                    edges += (uint64_t)seg_count(quad_wang(cur, q1, q2, tol)) + 1u;
+                } else if (verb == LYG_VERB_CUBIC) {
+                    edges += (uint64_t)seg_count(cubic_wang(cur, q1, q2, q3, tol)) + 1u;
+                } else {
+                    edges += 1u;
+                }
+            }
+            // every sub-path is closed by an edge back to its start (event_queue.rs:661-682)
+            const vec2 start = before(beg);
+            const vec2 cur = after_end ? start : before(first);
+            const vec2 to = !moves ? start : verb == LYG_VERB_CUBIC ? q3
+                          : verb == LYG_VERB_QUADRATIC ? q2 : q1;
+            const vec2 c1 = verb == LYG_VERB_QUADRATIC || verb == LYG_VERB_CUBIC ? q1 : to;
+            const vec2 c2 = verb == LYG_VERB_CUBIC ? q2 : to;
+            d = verb == LYG_VERB_CUBIC ? 3u : verb == LYG_VERB_QUADRATIC ? 2u : 1u;
+            if (moves || !(cur.x == start.x && cur.y == start.y)) {
+                bx = make_float4(ffmin(ffmin(cur.x, c1.x), ffmin(c2.x, to.x)) - pad,
+                                 ffmin(ffmin(cur.y, c1.y), ffmin(c2.y, to.y)) - pad,
+                                 ffmax(ffmax(cur.x, c1.x), ffmax(c2.x, to.x)) + pad,
+                                 ffmax(ffmax(cur.y, c1.y), ffmax(c2.y, to.y)) + pad);
+                acc += verb == LYG_VERB_CUBIC ? 1u : 0u;
             }
         }
+        deg = deg + d < deg ? 0xffffffffu : deg + d;
+        if (pairs && in) boxes[v0 + l] = bx;
+        pt = readlane_u(upto, WAVE - 1);
+        c_cur = readlane_u(m, WAVE - 1);
+        c_beg = readlane_u(beg, WAVE - 1);
+        c_end = readlane_u(is_end, WAVE - 1);
     }
-    // wave sum: a lane sees at most 64 * 4096 pairs, so 32 bits hold it
-    uint32_t sum = incl_scan(acc);
-    sum = readlane_u(sum, WAVE - 1);
-    if (l == 0) inter[path] = sum > 0x7fffffffu ? 0x7fffffffu : sum;
+    wave_sync();
+    if (pairs) {
+        for (uint32_t i = (uint32_t)l; i < nv; i += WAVE) {
+            const float4 a = boxes[i];
+            for (uint32_t j = i + 2; j < nv; ++j) {
+                const float4 b = boxes[j];
+                acc += a.x > b.z || b.x > a.z || a.y > b.w || b.y > a.w ? 0u : 1u;
+            }
+        }
+        // a lane sees at most 64 * 4096 pairs, so 32 bits hold the sum
+        const uint32_t sum = readlane_u(incl_scan(acc), WAVE - 1);
+        if (l == 0) inter[path] = sum > 0x7fffffffu ? 0x7fffffffu : sum;
+    } else if (l == 0) {
+        inter[path] = 0u;
+        if (nv <= INTER_MAX_VERBS) *more = 1u;
+    }
+    if (over) return;
+    uint64_t all_edges = 0, all_deg = 0;
+    for (int i = 0; i < WAVE; ++i) {
+        all_edges += (uint64_t)readlane_u((uint32_t)(edges >> 32), i) << 32 |
+                     readlane_u((uint32_t)edges, i);
+        all_deg += readlane_u(deg, i);
+    }
+    if (l == 0) {
+        degree[path] = all_deg > 0xffffffffull ? 0xffffffffu : (uint32_t)all_deg;
+        const uint64_t bnd = 2 * all_edges + 16;
+        bound[path] = bnd > 0xffffffffull ? 0xffffffffu : (uint32_t)bnd;
+    }
 }
 
 }  // namespace lyg
 
 extern "C" {
 
-size_t lyg_fill_box_bytes() { return sizeof(lyg::VBox); }
-hipError_t lyg_launch_fill_inter(const lyg::FillLaunch* L, uint32_t n, void* boxes, uint32_t* inter,
-                                 hipStream_t s) {
+// bound, degree, inter: n each; more: set when some path's pairs are left to a second launch
+// (again), which is given the same arrays.
+hipError_t lyg_launch_fill_measure(const lyg::FillLaunch* L, uint32_t n, uint32_t* bound,
+                                   uint32_t* degree, uint32_t* inter, uint32_t* more, int again,
+                                   hipStream_t s) {
+    using namespace lyg;
     if (n == 0) return hipSuccess;
-    lyg::VBox* rec = static_cast<lyg::VBox*>(boxes);
-    hipLaunchKernelGGL(lyg::fill_boxes_kernel, dim3((n + 127) / 128), dim3(128), 0, s, *L, n, rec);
-    hipLaunchKernelGGL(lyg::fill_inter_kernel, dim3(n), dim3(lyg::WAVE), 0, s, *L, n,
-                       (const lyg::VBox*)rec, inter);
+    if (again)
+        hipLaunchKernelGGL(fill_measure_kernel<INTER_MAX_VERBS>, dim3(n), dim3(WAVE), 0, s, *L,
+                           INTER_FEW_VERBS, bound, degree, inter, more);
+    else
+        hipLaunchKernelGGL(fill_measure_kernel<INTER_FEW_VERBS>, dim3(n), dim3(WAVE), 0, s, *L, 0u,
+                           bound, degree, inter, more);
     return hipGetLastError();
 }
 size_t lyg_fill_work_bytes(const lyg::fillk::FillCaps* caps, size_t hot_bytes) {
     lyg::fillk::Work w;
     return lyg::fillk::carve(nullptr, nullptr, hot_bytes, *caps, w);
-}
-hipError_t lyg_launch_fill_bound(const lyg::FillLaunch* L, uint32_t n, uint32_t* bound,
-                                 uint32_t* degree, hipStream_t s) {
-    if (n == 0) return hipSuccess;
-    hipLaunchKernelGGL(lyg::fill_bound_kernel, dim3((n + 127) / 128), dim3(128), 0, s, *L, n,
-                       bound, degree);
-    return hipGetLastError();
 }
 // Resident blocks per CU of the sweep kernel for a launch shape (0 if it cannot launch).
 int lyg_fill_occupancy(uint32_t waves_per_block, uint32_t hot_bytes) {

@@ -1,7 +1,8 @@
 // Host side of the fill: sizing, launch rounds and compaction.
 //
 // A fill call runs in three steps on the context's stream:
-//   1. fill_bound_kernel writes an upper bound of every path's sweep events;
+//   1. fill_measure_kernel writes an upper bound of every path's sweep events and estimates of
+//      its active edges and self-intersections;
 //   2. rounds of sweeps: each path is swept by one wave into a staging area sized from its
 //      bound, in the first round with its active edges in registers (fill_reg.hip), later or
 //      beyond 1,024 of them over arrays (fill.hip).  Paths are grouped into size classes so
@@ -25,12 +26,10 @@ size_t lyg_fill_work_bytes(const lyg::fillk::FillCaps* caps, size_t hot_bytes);
 int lyg_fill_occupancy(uint32_t waves_per_block, uint32_t hot_bytes);
 int lyg_fill_reg_occupancy(uint32_t chunks, uint32_t rows);
 hipError_t lyg_launch_fill_reg(const lyg::FillLaunch* L, int grid, hipStream_t s);
-hipError_t lyg_launch_fill_bound(const lyg::FillLaunch* L, uint32_t n, uint32_t* bound,
-                                 uint32_t* degree, hipStream_t s);
+hipError_t lyg_launch_fill_measure(const lyg::FillLaunch* L, uint32_t n, uint32_t* bound,
+                                   uint32_t* degree, uint32_t* inter, uint32_t* more, int again,
+                                   hipStream_t s);
 hipError_t lyg_launch_fill_sweep(const lyg::FillLaunch* L, int grid, hipStream_t s);
-size_t lyg_fill_box_bytes();
-hipError_t lyg_launch_fill_inter(const lyg::FillLaunch* L, uint32_t n, void* boxes, uint32_t* inter,
-                                 hipStream_t s);
 hipError_t lyg_launch_fill_copy(const lyg::FillLaunch* L, hipStream_t s);
 hipError_t lyg_launch_fill_status_out(const uint32_t* st, uint32_t* out, uint32_t n,
                                       hipStream_t s);
@@ -386,38 +385,27 @@ struct FillResult {
     std::vector<uint32_t> round_len;  // paths swept in each round
 };
 
-// Step 1 and the intersection estimate, read back to the host: every path's event bound
-// and its estimated self-intersections.
-bool measure(lyg_ctx* c, const lyg::FillLaunch& L, hipStream_t s, std::vector<uint32_t>* bound_out,
-             std::vector<uint32_t>* degree_out, std::vector<uint32_t>* inter_out) {
+// Step 1, read back to the host: every path's event bound, degree and estimated
+// self-intersections.
+bool measure(lyg_ctx* c, const lyg::FillLaunch& L, hipStream_t s, std::vector<uint32_t>* bound,
+             std::vector<uint32_t>* degree, std::vector<uint32_t>* inter) {
     const uint32_t n = L.in.n_paths;
-    if (!ensure(c, c->f_bound, 8ull * n)) return false;
-    std::vector<uint32_t>& bound = *bound_out;
-    std::vector<uint32_t>& degree = *degree_out;
-    std::vector<uint32_t>& inter = *inter_out;
-    bound.assign(n, 0);
-    degree.assign(n, 0);
-    inter.assign(n, 0);
-    uint32_t n_verbs = 0;
-    uint32_t* d_bound = as<uint32_t>(c->f_bound);
-    if (!check(c, lyg_launch_fill_bound(&L, n, d_bound, d_bound + n, s), "fill bound") ||
-        !check(c, hipMemcpyAsync(bound.data(), d_bound, 4ull * n, hipMemcpyDeviceToHost, s),
-               "D2H") ||
-        !check(c, hipMemcpyAsync(degree.data(), d_bound + n, 4ull * n, hipMemcpyDeviceToHost, s),
-               "D2H") ||
-        !check(c, hipMemcpyAsync(&n_verbs, L.in.verb_off + n, 4, hipMemcpyDeviceToHost, s), "D2H") ||
-        !check(c, hipStreamSynchronize(s), "sync"))
-        return false;
-    // intersection estimate: one box record per verb, then a pair count per path
-    if (!ensure(c, c->f_inter, 4ull * n) ||
-        !ensure(c, c->f_boxes, lyg_fill_box_bytes() * ((size_t)n_verbs + 1)))
-        return false;
-    if (!check(c, lyg_launch_fill_inter(&L, n, c->f_boxes.p, as<uint32_t>(c->f_inter), s),
-               "fill inter") ||
-        !check(c, hipMemcpyAsync(inter.data(), c->f_inter.p, 4ull * n, hipMemcpyDeviceToHost, s),
-               "D2H") ||
-        !check(c, hipStreamSynchronize(s), "sync"))
-        return false;
+    const size_t bytes = 4ull * (3ull * n + 1u);
+    if (!ensure(c, c->f_bound, bytes)) return false;
+    uint32_t* d = as<uint32_t>(c->f_bound);  // bounds, degrees, intersections, more
+    std::vector<uint32_t> h(3ull * n + 1u);
+    for (int again = 0; again < 2; ++again) {
+        if ((!again && !check(c, lyg_launch_fill_u32(d + 3ull * n, 1, 0, s), "reset")) ||
+            !check(c, lyg_launch_fill_measure(&L, n, d, d + n, d + 2ull * n, d + 3ull * n, again, s),
+                   "fill measure") ||
+            !check(c, hipMemcpyAsync(h.data(), d, bytes, hipMemcpyDeviceToHost, s), "D2H") ||
+            !check(c, hipStreamSynchronize(s), "sync"))
+            return false;
+        if (!h[3ull * n]) break;
+    }
+    bound->assign(h.begin(), h.begin() + n);
+    degree->assign(h.begin() + n, h.begin() + 2ull * n);
+    inter->assign(h.begin() + 2ull * n, h.begin() + 3ull * n);
     return true;
 }
 
@@ -426,7 +414,7 @@ int32_t fill_sweep(lyg_ctx* c, const FillJob& J, uint32_t* vtx_off, uint32_t* id
                    FillResult* R) {
     const uint32_t n = J.in.n_paths;
     hipStream_t s = c->stream;
-    if (!ensure(c, c->f_bound, 4ull * n) || !ensure(c, c->f_status, 4ull * n) ||
+    if (!ensure(c, c->f_status, 4ull * n) ||
         !ensure(c, c->f_round, 4ull * n) || !ensure(c, c->f_hint, 4ull * n) ||
         !ensure(c, c->counts_v, 4ull * n) || !ensure(c, c->counts_i, 4ull * n))
         return LYG_ERR_DEVICE;

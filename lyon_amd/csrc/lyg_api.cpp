@@ -645,14 +645,12 @@ void lyg_ctx_destroy(lyg_ctx* c) {
     free_buf(c->f_work);
     free_buf(c->f_ops);
     free_buf(c->f_path_ops);
-    free_buf(c->f_inter);
     free_buf(c->nsub_thr);
     free_buf(c->scan_tiles);
     for (DevBuf* b : {&c->st_cap_v, &c->st_cap_i, &c->st_off_v, &c->st_off_i, &c->st_v, &c->st_i,
                       &c->st_fallback, &c->st_items, &c->st_heads, &c->st_spec, &c->st_end,
                       &c->st_parts, &c->st_parts_off})
         free_buf(*b);
-    free_buf(c->f_boxes);
     free_buf(c->f_counters);
     lyg_band_free(c);
     for (auto* v : {&c->f_stage_v, &c->f_stage_t, &c->f_stage_off, &c->f_list})

@@ -270,6 +270,43 @@ def test_active_edges_around_the_register_sets(shape, sizes):
                                   canon(np.asarray(ri, np.int64) + int(vo[k]))), sizes[k]
 
 
+@pytest.mark.parametrize("sizes", [(1, 2, 3, 62, 63, 64, 65), (1021, 1022, 1023, 1024),
+                                   (3, 4093, 4094, 4095, 4096)], ids=["few", "1024", "4096"])
+def test_paths_around_the_verbs_measured_at_once(sizes):
+    """Paths of as many verbs as are measured together (64 a turn, boxes of 1,024, of 4,096
+    again, none beyond), closed outlines that cross themselves here and there."""
+    from lyon_amd.batch import DeviceBatch, FillBatcher
+    from lyon_amd.path import PathBatch
+    rng = np.random.default_rng(sizes[0])
+    paths = []
+    for n in sizes:  # n + 1 verbs: Begin, lines and curves, Close
+        b = PathBuilder()
+        t = np.arange(n) * (2.0 * np.pi / max(n, 1))
+        r = 400.0 + 40.0 * np.sin(7.0 * t) + rng.random(n)
+        p = np.stack([r * np.cos(t), r * np.sin(2.0 * t)], 1)
+        b.begin(tuple(p[0]))
+        for k in range(1, n):
+            m = tuple((p[k - 1] + p[k]) * 0.5 + 0.5)
+            if k % 5 == 1:
+                b.quadratic_bezier_to(m, tuple(p[k]))
+            elif k % 5 == 2:
+                b.cubic_bezier_to(tuple(p[k - 1]), m, tuple(p[k]))
+            else:
+                b.line_to(tuple(p[k]))
+        b.end(True)
+        paths.append(b.build())
+    opts = workloads.fill_options(len(paths), tolerance=0.05)
+    res = FillBatcher().run(DeviceBatch(PathBatch.from_paths(paths), opts))
+    v, i, vo, io = res.all_vertices(), res.all_indices(), res.vertex_offsets, res.index_offsets
+    for k, p in enumerate(paths):
+        o = FillOptions(tolerance=0.05, fill_rule=FillRule(int(opts[k]["fill_rule"])))
+        st, rv, ri = ref_fill(p, o, int(vo[k]))
+        assert res.status[k] == st == 0
+        assert np.array_equal(v[vo[k]:vo[k + 1]].view(np.uint32),
+                              np.asarray(rv, np.float32).reshape(-1, 2).view(np.uint32)), sizes[k]
+        assert np.array_equal(canon(i[io[k]:io[k + 1]]), canon(ri)), sizes[k]
+
+
 def test_very_large_path():
     """fill_tests.rs:2140-2166: a path of 1,000,000 endpoints (two wiggling sides of a long
     band) fills without error; the same vertices and triangle count as the oracle and the
