@@ -315,8 +315,9 @@ def main():
                   "value": vtris / (vms / 1e3), "unit": "triangles/s",
                   "failed_paths": int(np.count_nonzero(vres.status)),
                   "note": "lyg_stroke_batch_vw over the stroke workload's paths and options, "
-                          "width factor per point U[0.5, 2]: one GPU lane per path (count "
-                          "pass, scans, emit pass); median of steps"}
+                          "width factor per point U[0.5, 2]: points of every path in "
+                          "parallel, joins in windows of 63 (count, scans, "
+                          "emit); median of steps"}
         log(f"  variable-width stroke: {vms:.2f} ms, {vtris} triangles")
         del vwb
     except Exception as e:  # reported, not fatal: the headline does not depend on it
