@@ -38,7 +38,7 @@ struct lyg_ctx {
     uint32_t fill_hot_bytes = 16 * 1024;
     uint32_t fill_lds_resident = 1;  // first round with the active edges in registers
     // fill: per-path arrays, per-wave working memory and per-round staging
-    DevBuf f_bound, f_status, f_round, f_hint, f_work, f_counters, f_ops,
+    DevBuf f_bound, f_status, f_round, f_hint, f_work, f_counters, f_ops, f_op_tris,
         f_path_ops;
     std::vector<DevBuf> f_stage_v, f_stage_t, f_stage_off, f_list;
     // stroke: staged single pass (emit into per-path staging room, then compact)

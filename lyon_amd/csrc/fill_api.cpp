@@ -176,7 +176,7 @@ int32_t plan_round(lyg_ctx* c, const std::vector<uint32_t>& todo,
                    const std::vector<uint32_t>& bound, const std::vector<uint32_t>& degree,
                    const std::vector<uint32_t>& inter, const std::vector<uint64_t>& need,
                    int round, uint64_t scale, bool graph, RoundPlan* P) {
-    // the register sweep's log takes 32 bytes per staged triangle
+    // the register sweep's log takes 52 bytes per staged triangle
     uint64_t all_v = 0, all_t = 0;
     for (uint32_t p : todo) {
         uint64_t v, t;
@@ -185,7 +185,7 @@ int32_t plan_round(lyg_ctx* c, const std::vector<uint32_t>& todo,
         all_t += t;
     }
     const uint32_t mode = c->fill_lds_resident;
-    const bool reg = round <= (mode == 1 ? 1 : 0) && 8 * all_v + 44 * all_t <= STAGE_BUDGET;
+    const bool reg = round <= (mode == 1 ? 1 : 0) && 8 * all_v + 64 * all_t <= STAGE_BUDGET;
     auto shape = [&](uint32_t p) { return Shape{bound[p], degree[p]}; };
     P->log_ops = reg ? all_t : 0;
     // order by launch: size class, then the form (the first round picks it per path, the
@@ -463,7 +463,8 @@ int32_t fill_sweep(lyg_ctx* c, const FillJob& J, uint32_t* vtx_off, uint32_t* id
             !ensure_at(c, c->f_stage_off, round, 8 * offs.size()) ||
             !ensure_at(c, c->f_stage_v, round, 8 * sv[m]) ||
             !ensure_at(c, c->f_stage_t, round, 12 * st[m]) ||
-            (P.log_ops && !ensure(c, c->f_ops, sizeof(lyg::FillOp) * P.log_ops)) ||
+            (P.log_ops && (!ensure(c, c->f_ops, sizeof(lyg::FillOp) * P.log_ops) ||
+                           !ensure(c, c->f_op_tris, sizeof(lyg::FillTri) * P.log_ops))) ||
             !ensure(c, c->f_path_ops, 4ull * n))
             return LYG_ERR_DEVICE;
         uint32_t* d_list = as<uint32_t>(c->f_list[round]);
@@ -482,6 +483,7 @@ int32_t fill_sweep(lyg_ctx* c, const FillJob& J, uint32_t* vtx_off, uint32_t* id
         L.stage_v = as<float>(c->f_stage_v[round]);
         L.stage_t = as<uint32_t>(c->f_stage_t[round]);
         L.ops = as<lyg::FillOp>(c->f_ops);
+        L.op_tris = as<lyg::FillTri>(c->f_op_tris);
         L.path_ops = as<uint32_t>(c->f_path_ops);
         const std::vector<Launch>& launches = P.launches;
         if (!ensure(c, c->f_work, P.work_bytes)) return LYG_ERR_NO_SPACE;
@@ -660,7 +662,7 @@ struct lygi::FillGraph {
     uint32_t n = 0;
     uint32_t vertex_offset = 0;
     uint64_t vertex_capacity = 0, index_capacity = 0;
-    DevBuf status, round, nv, ni, list, off, stage_v, stage_t, ops, path_ops, work, counters,
+    DevBuf status, round, nv, ni, list, off, stage_v, stage_t, ops, op_tris, path_ops, work, counters,
         totals, tiles;
     std::vector<hipGraph_t> graphs;
     hipGraphExec_t head = nullptr, tail = nullptr;
@@ -742,7 +744,8 @@ int32_t lygi::fill_graph_capture(lyg_ctx* c, const lyg_batch_in* in, const lyg_f
     const uint64_t* st = P.offs.data() + m + 1;
     if (!ensure(c, g->list, 4 * m) || !ensure(c, g->off, 8 * P.offs.size()) ||
         !ensure(c, g->stage_v, 8 * sv[m]) || !ensure(c, g->stage_t, 12 * st[m]) ||
-        (P.log_ops && !ensure(c, g->ops, sizeof(lyg::FillOp) * P.log_ops)) ||
+        (P.log_ops && (!ensure(c, g->ops, sizeof(lyg::FillOp) * P.log_ops) ||
+                       !ensure(c, g->op_tris, sizeof(lyg::FillTri) * P.log_ops))) ||
         !ensure(c, g->path_ops, 4ull * n))
         return LYG_ERR_DEVICE;
     if (!ensure(c, g->work, P.work_bytes)) return LYG_ERR_NO_SPACE;
@@ -756,6 +759,7 @@ int32_t lygi::fill_graph_capture(lyg_ctx* c, const lyg_batch_in* in, const lyg_f
     L.stage_v = as<float>(g->stage_v);
     L.stage_t = as<uint32_t>(g->stage_t);
     L.ops = as<lyg::FillOp>(g->ops);
+    L.op_tris = as<lyg::FillTri>(g->op_tris);
     L.path_ops = as<uint32_t>(g->path_ops);
     const size_t n_streams = std::min<size_t>(P.launches.size(), CLASS_STREAMS);
     if (!class_streams(c, n_streams, P.launches.size()) ||
@@ -892,7 +896,7 @@ void lygi::fill_graph_destroy(FillGraph* g) {
     if (g->fork) (void)hipEventDestroy(g->fork);
     for (hipEvent_t e : g->join) (void)hipEventDestroy(e);
     for (DevBuf* b : {&g->status, &g->round, &g->nv, &g->ni, &g->list, &g->off, &g->stage_v,
-                      &g->stage_t, &g->ops, &g->path_ops, &g->work, &g->counters, &g->totals, &g->tiles})
+                      &g->stage_t, &g->ops, &g->op_tris, &g->path_ops, &g->work, &g->counters, &g->totals, &g->tiles})
         free_buf(*b);
     delete g;
 }

@@ -14,8 +14,8 @@
 //     at one column only;
 //   * the monotone triangulation is left out of the chain: the sweep writes a log of span
 //     operations (begin, vertex on a side, end), linked per span, and lanes walk the spans
-//     afterwards, all at once: first counting each operation's triangles, then, after a scan
-//     in log order, writing them where the sweep would have.
+//     afterwards, all at once; after a scan of the operations' triangles in log order, they
+//     go where the sweep would have written them.
 // Vertices, triangles and their order are those of the sweep over arrays.
 //
 // A path stops with the retry status when it has more than 64 C active edges (or spans),
@@ -1034,8 +1034,9 @@ __device__ __forceinline__ void reg_sweep(const FillLaunch& L, uint32_t path, ui
 // AdvancedMonotoneTessellator over BasicMonotoneTessellator (monotone.rs:9-404) along one
 // span's operations, by one lane.  The operations are the nodes of the stack (link_stack) and
 // of the side lists (link_side; the link of a list's first node is kept in registers, as a
-// span's first vertex heads both).  EMIT false: each operation's triangle count; true: the
-// triangles at out + 3 * (the operation's scanned offset).
+// span's first vertex heads both).  Every triangle takes a vertex out, so a span has fewer of
+// them than operations: they wait in its operations' slots, with the counts per operation,
+// until the scan has placed them.
 struct TSide {
     vec2 ref, prev, last_pos;
     float cons_x;
@@ -1043,26 +1044,32 @@ struct TSide {
 };
 struct TSpan {
     FillOp* ops;
+    FillTri* tri;
     uint32_t top, pside;
     TSide side[2];
-    uint32_t cnt;
-    uint32_t* out;  // EMIT: the current operation's next triangle
+    uint32_t op, cnt;           // the current operation, its triangles so far
+    uint32_t slot, slot_next;   // where the next triangle goes, and the one after
 };
 __device__ __forceinline__ vec2 op_pos(const FillOp* ops, uint32_t i) {
     const float2 p = *reinterpret_cast<const float2*>(&ops[i].x);
     return mk(p.x, p.y);
 }
-template <bool EMIT>
+// A triangle waits in the slot of one of the span's operations, in their order: there are fewer
+// triangles than operations.
 __device__ __forceinline__ void t_tri(TSpan& t, uint32_t a, uint32_t b, uint32_t c) {
-    if (EMIT) {
-        t.out[3u * t.cnt + 0u] = a;
-        t.out[3u * t.cnt + 1u] = b;
-        t.out[3u * t.cnt + 2u] = c;
+    if (t.slot != DEAD) {
+        FillTri& d = t.tri[t.slot];
+        d.a = a;
+        d.b = b;
+        d.c = c;
+        d.op = t.op;
+        d.nth = t.cnt;
+        t.slot = t.slot_next;
+        if (t.slot != DEAD) t.slot_next = t.ops[t.slot].next;
     }
     ++t.cnt;
 }
 // BasicMonotoneTessellator::vertex (monotone.rs:60-107); n: the vertex's operation.
-template <bool EMIT>
 __device__ __forceinline__ void t_basic(TSpan& t, vec2 pos, uint32_t n, uint32_t side) {
     FillOp* ops = t.ops;
     const uint32_t id = ops[n].id;
@@ -1073,8 +1080,8 @@ __device__ __forceinline__ void t_basic(TSpan& t, vec2 pos, uint32_t n, uint32_t
         for (uint32_t a = ops[b].link_stack; a != DEAD;) {
             const vec2 pa = op_pos(ops, a);
             const uint32_t ia = ops[a].id, nx = ops[a].link_stack;
-            if (cross2(sub(pa, pb), sub(pos, pb)) >= 0.0f) t_tri<EMIT>(t, ia, ib, id);
-            else t_tri<EMIT>(t, ib, ia, id);
+            if (cross2(sub(pa, pb), sub(pos, pb)) >= 0.0f) t_tri(t, ia, ib, id);
+            else t_tri(t, ib, ia, id);
             pb = pa;
             ib = ia;
             a = nx;
@@ -1090,8 +1097,8 @@ __device__ __forceinline__ void t_basic(TSpan& t, vec2 pos, uint32_t n, uint32_t
             const vec2 na = side == 1u ? ph : pl, nb = side == 1u ? pl : ph;
             const float c = cross2(sub(pos, nb), sub(na, nb));
             if (!(c >= 0.0f)) break;
-            if (side == 1u) t_tri<EMIT>(t, il, ih, id);
-            else t_tri<EMIT>(t, ih, il, id);
+            if (side == 1u) t_tri(t, il, ih, id);
+            else t_tri(t, ih, il, id);
             lp = head;
             pl = ph;
             il = ih;
@@ -1105,7 +1112,7 @@ __device__ __forceinline__ void t_basic(TSpan& t, vec2 pos, uint32_t n, uint32_t
 }
 // flush_side (monotone.rs:356-398): true when the side's last vertex goes to the basic
 // tessellator.  Each level of the binary tree walks the list and drops every second node.
-template <bool EMIT, uint32_t SIDE>
+template <uint32_t SIDE>
 __device__ __forceinline__ bool t_flush(TSpan& t) {
     TSide& e = t.side[SIDE];
     FillOp* ops = t.ops;
@@ -1120,8 +1127,8 @@ __device__ __forceinline__ bool t_flush(TSpan& t) {
             const uint32_t b = a == head ? second : ops[a].link_side;
             const uint32_t l = ops[b].link_side;
             const uint32_t ib = ops[b].id, il = ops[l].id;
-            if (SIDE == 1u) t_tri<EMIT>(t, ib, ia, il);
-            else t_tri<EMIT>(t, ia, ib, il);
+            if (SIDE == 1u) t_tri(t, ib, ia, il);
+            else t_tri(t, ia, ib, il);
             if (a == head) second = l;
             else ops[a].link_side = l;
             a = l;
@@ -1129,8 +1136,8 @@ __device__ __forceinline__ bool t_flush(TSpan& t) {
         }
         if (imax * 2u * step + step < len) {
             const uint32_t c = a == head ? second : ops[a].link_side, ic = ops[c].id;
-            if (SIDE == 1u) t_tri<EMIT>(t, id0, ic, ia);
-            else t_tri<EMIT>(t, id0, ia, ic);
+            if (SIDE == 1u) t_tri(t, id0, ic, ia);
+            else t_tri(t, id0, ia, ic);
         }
     }
     e.head = e.tail;
@@ -1139,7 +1146,7 @@ __device__ __forceinline__ bool t_flush(TSpan& t) {
     e.ref = e.last_pos;
     return true;
 }
-template <bool EMIT, uint32_t SIDE>
+template <uint32_t SIDE>
 __device__ __forceinline__ void t_vertex(TSpan& t, vec2 pos, uint32_t n) {
     TSide& se = t.side[SIDE];
     TSide& op = t.side[1u - SIDE];
@@ -1160,13 +1167,13 @@ __device__ __forceinline__ void t_vertex(TSpan& t, vec2 pos, uint32_t n) {
     }
     if (outward || close) {
         if (pos_after(se.last_pos, op.last_pos)) {
-            if (t_flush<EMIT, 1u - SIDE>(t)) {
-                t_basic<EMIT>(t, op.last_pos, op.tail, 1u - SIDE);
+            if (t_flush<1u - SIDE>(t)) {
+                t_basic(t, op.last_pos, op.tail, 1u - SIDE);
                 se.cons_x = se.ref.x;
             }
         }
-        if (t_flush<EMIT, SIDE>(t)) {
-            t_basic<EMIT>(t, se.last_pos, se.tail, SIDE);
+        if (t_flush<SIDE>(t)) {
+            t_basic(t, se.last_pos, se.tail, SIDE);
             op.cons_x = op.ref.x;
         }
     }
@@ -1178,10 +1185,12 @@ __device__ __forceinline__ void t_vertex(TSpan& t, vec2 pos, uint32_t n) {
     se.prev = se.last_pos;
     se.last_pos = pos;
 }
-template <bool EMIT>
-__device__ void t_span(FillOp* ops, uint32_t first, uint32_t* out) {
+__device__ void t_span(FillOp* ops, FillTri* tri, uint32_t first) {
     TSpan t;
     t.ops = ops;
+    t.tri = tri;
+    t.slot = first;
+    t.slot_next = ops[first].next;
     t.top = first;
     t.pside = 0;
     const vec2 p0 = op_pos(ops, first);
@@ -1199,25 +1208,26 @@ __device__ void t_span(FillOp* ops, uint32_t first, uint32_t* out) {
         const float4 r = *reinterpret_cast<const float4*>(&ops[n]);
         const vec2 pos = mk(r.x, r.y);
         const uint32_t kind = f2u(r.w), next = ops[n].next;
+        t.op = n;
         t.cnt = 0;
-        if (EMIT) t.out = out + 3ull * ops[n].tris;
         if (kind == OP_LEFT) {
-            t_vertex<EMIT, 0u>(t, pos, n);
+            t_vertex<0u>(t, pos, n);
         } else if (kind == OP_RIGHT) {
-            t_vertex<EMIT, 1u>(t, pos, n);
+            t_vertex<1u>(t, pos, n);
         } else {
             // AdvancedMonotoneTessellator::end (monotone.rs:337-353)
-            const bool ha = t_flush<EMIT, 0u>(t);
-            const bool hb = t_flush<EMIT, 1u>(t);
+            const bool ha = t_flush<0u>(t);
+            const bool hb = t_flush<1u>(t);
             const bool b_first = hb && (!ha || pos_after(t.side[0].last_pos, t.side[1].last_pos));
-            if (b_first) t_basic<EMIT>(t, t.side[1].last_pos, t.side[1].tail, 1u);
-            if (ha) t_basic<EMIT>(t, t.side[0].last_pos, t.side[0].tail, 0u);
-            if (hb && !b_first) t_basic<EMIT>(t, t.side[1].last_pos, t.side[1].tail, 1u);
-            t_basic<EMIT>(t, pos, n, 1u - t.pside);
+            if (b_first) t_basic(t, t.side[1].last_pos, t.side[1].tail, 1u);
+            if (ha) t_basic(t, t.side[0].last_pos, t.side[0].tail, 0u);
+            if (hb && !b_first) t_basic(t, t.side[1].last_pos, t.side[1].tail, 1u);
+            t_basic(t, pos, n, 1u - t.pside);
         }
-        if (!EMIT) ops[n].tris = t.cnt;
+        ops[n].tris = t.cnt;
         n = next;
     }
+    for (uint32_t q = t.slot; q != DEAD; q = ops[q].next) tri[q].op = DEAD;
 }
 
 }  // namespace fillk
@@ -1252,18 +1262,38 @@ __global__ void __launch_bounds__(WAVE) fill_reg_kernel(FillLaunch L) {
 }
 
 // Lane per operation of a path (blockIdx.x: the path, blockIdx.y: a slice of its log); the
-// ones that begin a span walk it.
-template <bool EMIT>
+// ones that begin a span walk it, once: counting first and walking again for the triangles took
+// 1,000 glyphs 237 us, 161 us so, bound by the instructions along the longest span.
 __global__ void __launch_bounds__(256) fill_tess_kernel(FillLaunch L) {
     using namespace fillk;
     const uint32_t k = blockIdx.x;
     const uint32_t path = L.path_list[k];
     if (L.path_status[path] != 0u) return;
     FillOp* ops = L.ops + L.stage_t_off[k];
-    uint32_t* out = L.stage_t + 3ull * L.stage_t_off[k];
+    FillTri* tri = L.op_tris + L.stage_t_off[k];
     const uint32_t n = L.path_ops[path];
     for (uint32_t i = blockIdx.y * 256u + threadIdx.x; i < n; i += gridDim.y * 256u)
-        if (ops[i].kind == OP_BEGIN) t_span<EMIT>(ops, i, out);
+        if (ops[i].kind == OP_BEGIN) t_span(ops, tri, i);
+}
+
+// Lane per slot: the triangles to their places, in the operations' order.
+__global__ void __launch_bounds__(256) fill_tess_place_kernel(FillLaunch L) {
+    using namespace fillk;
+    const uint32_t k = blockIdx.x;
+    const uint32_t path = L.path_list[k];
+    if (L.path_status[path] != 0u) return;
+    const FillOp* ops = L.ops + L.stage_t_off[k];
+    const FillTri* tri = L.op_tris + L.stage_t_off[k];
+    uint32_t* out = L.stage_t + 3ull * L.stage_t_off[k];
+    const uint32_t n = L.path_ops[path];
+    for (uint32_t i = blockIdx.y * 256u + threadIdx.x; i < n; i += gridDim.y * 256u) {
+        const FillTri t = tri[i];
+        if (t.op == DEAD) continue;
+        uint32_t* d = out + 3ull * (ops[t.op].tris + t.nth);
+        d[0] = t.a;
+        d[1] = t.b;
+        d[2] = t.c;
+    }
 }
 
 // Wave per path: the operations' triangle counts become offsets in log order.
@@ -1334,9 +1364,9 @@ hipError_t lyg_launch_fill_reg(const lyg::FillLaunch* L, int grid, hipStream_t s
         return hipErrorInvalidValue;
     // enough blocks for a launch of few paths to spread over the GPU
     const uint32_t slices = L->n_list >= 512u ? 4u : L->n_list >= 32u ? 16u : 64u;
-    hipLaunchKernelGGL(lyg::fill_tess_kernel<false>, dim3(L->n_list, slices), dim3(256), 0, s, *L);
+    hipLaunchKernelGGL(lyg::fill_tess_kernel, dim3(L->n_list, slices), dim3(256), 0, s, *L);
     hipLaunchKernelGGL(lyg::fill_tess_scan_kernel, dim3(L->n_list), dim3(lyg::WAVE), 0, s, *L);
-    hipLaunchKernelGGL(lyg::fill_tess_kernel<true>, dim3(L->n_list, slices), dim3(256), 0, s, *L);
+    hipLaunchKernelGGL(lyg::fill_tess_place_kernel, dim3(L->n_list, slices), dim3(256), 0, s, *L);
     return hipGetLastError();
 }
 

@@ -644,6 +644,7 @@ void lyg_ctx_destroy(lyg_ctx* c) {
     free_buf(c->f_hint);
     free_buf(c->f_work);
     free_buf(c->f_ops);
+    free_buf(c->f_op_tris);
     free_buf(c->f_path_ops);
     free_buf(c->nsub_thr);
     free_buf(c->scan_tiles);

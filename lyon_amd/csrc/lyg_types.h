@@ -143,6 +143,11 @@ struct FillOp {
     uint32_t tris;                 // its triangles, then their offset in the path's
 };
 
+// A triangle of a span, until the operations' offsets are known: the nth of operation `op`.
+struct FillTri {
+    uint32_t a, b, c, op, nth;
+};
+
 struct FillLaunch {
     PathBatchDev in;
     const lyg_fill_options* opts;  // per path (opts_stride 1) or shared (stride 0)
@@ -172,6 +177,7 @@ struct FillLaunch {
     uint32_t reg_chunks, heap_rows;
     uint32_t act_limit, heap_limit;
     FillOp* ops;
+    FillTri* op_tris;              // as many
     uint32_t* path_ops;
     // copy pass
     const uint32_t* vtx_off;
