@@ -17,6 +17,9 @@ struct DevBuf {
 
 struct BandBufs;  // the banded fill's buffers (band_api.cpp)
 
+// The most launches of one fill round (size class x form); each has an event that joins it.
+static constexpr int FILL_MAX_LAUNCHES = 32;
+
 struct lyg_ctx {
     int device = 0;
     hipStream_t stream = nullptr;
@@ -58,7 +61,7 @@ struct lyg_ctx {
     DevBuf vw_path, vw_rec, vw_flags, vw_src, vw_att, vw_win, vw_tails, vw_lists;
     // fill: one stream per size class of a round, and the events that join them
     hipStream_t class_stream[8] = {};
-    hipEvent_t class_ev[25] = {};  // one per fill launch (size class x form) + 1
+    hipEvent_t class_ev[FILL_MAX_LAUNCHES + 1] = {};
     // banded fill: band size (edge starts per band) and the most bands of one path
     BandBufs* band = nullptr;
     uint32_t band_edges_per_band = 256;

@@ -14,6 +14,7 @@
 #include <algorithm>
 #include <chrono>
 #include <cstring>
+#include <iterator>
 #include <numeric>
 #include <vector>
 
@@ -56,6 +57,7 @@ constexpr int FORM_ARRAYS = 0;
 constexpr uint32_t REG_CHUNKS[N_FORMS] = {0, 2, 5, 16};
 constexpr uint32_t REG_MAX_ROWS = 44;  // pending events per column: 66 KiB of LDS
 constexpr int MAX_LAUNCHES = N_FORMS * MAX_CLASSES;
+static_assert(MAX_LAUNCHES <= FILL_MAX_LAUNCHES, "lyg_ctx::class_ev has an event per launch");
 constexpr int N_GRAPH_COUNTERS = 2 * MAX_LAUNCHES;  // a launch and the sweep after it
 constexpr size_t CLASS_STREAMS = 3;
 
@@ -126,7 +128,7 @@ int size_class(uint64_t bound) {
 // Streams (default priority) for running a round's size classes at once, and one event
 // per launch plus the start event.
 bool class_streams(lyg_ctx* c, size_t n, size_t n_launches) {
-    if (n > (size_t)MAX_CLASSES || n_launches > (size_t)MAX_LAUNCHES) return false;
+    if (n > std::size(c->class_stream) || n_launches >= std::size(c->class_ev)) return false;
     for (size_t i = 0; i < n; ++i)
         if (!c->class_stream[i] &&
             !check(c, hipStreamCreateWithFlags(&c->class_stream[i], hipStreamNonBlocking),
@@ -902,6 +904,25 @@ void lygi::fill_graph_destroy(FillGraph* g) {
 }
 
 extern "C" {
+
+// Not in lyg.h: the launches of the first round over paths of these measures, on the host
+// alone, and the events a context has to join launches with (one more than it can hold).
+int32_t lyg_fill_plan_launches(const uint32_t* bound, const uint32_t* degree,
+                               const uint32_t* inter, uint32_t n, uint32_t* launches,
+                               uint32_t* events) {
+    lyg_ctx c;
+    c.cu_count = 1;
+    std::vector<uint64_t> need(n);
+    std::vector<uint32_t> todo(n);
+    std::iota(todo.begin(), todo.end(), 0u);
+    for (uint32_t i = 0; i < n; ++i) need[i] = (uint64_t)bound[i] + 2ull * inter[i];
+    RoundPlan P;
+    const int32_t st = plan_round(&c, todo, {bound, bound + n}, {degree, degree + n},
+                                  {inter, inter + n}, need, 0, 1, false, &P);
+    *launches = (uint32_t)P.launches.size();
+    *events = (uint32_t)std::size(c.class_ev);
+    return st;
+}
 
 // FillTessellator::tessellate_path (fill.rs:628-641) into caller-owned host arrays.
 int32_t lyg_fill_path(lyg_ctx* c, const lyg_path_view* path, const lyg_fill_options* opts,

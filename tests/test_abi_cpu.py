@@ -66,3 +66,17 @@ def test_header_is_c_and_links():
         r = subprocess.run([exe], capture_output=True, text=True, timeout=60)
         assert r.returncode == 0, (r.returncode, r.stdout, r.stderr)
         assert r.stdout.strip()
+
+
+def test_fill_rounds_have_an_event_per_launch():
+    """A fill round launches once per size class and form; with a path of every pair that is as
+    many launches as the context has events for, and one event more starts the round."""
+    cases = [(100, degree, (4096 << 2 * k) // 8 if k else 0)
+             for k in range(8) for degree in (8, 300, 1000, 4000)]
+    bound, degree, inter = np.array(cases, np.uint32).T.copy()
+    launches, events = C.c_uint32(0), C.c_uint32(0)
+    p = lambda a: a.ctypes.data_as(C.c_void_p)
+    st = C.CDLL(_lib.LIB_PATH).lyg_fill_plan_launches(p(bound), p(degree), p(inter), len(cases),
+                                                      C.byref(launches), C.byref(events))
+    assert st == 0 and launches.value == 32
+    assert events.value >= launches.value + 1
