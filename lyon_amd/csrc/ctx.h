@@ -25,6 +25,7 @@ struct lyg_ctx {
     hipStream_t stream = nullptr;
     int cu_count = 256;
     std::string last_error;
+    size_t alloc_limit = 0;  // tests: refuse a device buffer beyond this many bytes (0: none)
     // grow-only device scratch
     DevBuf in_verbs, in_points, in_offs, in_opts, counts_v, counts_i, offs_v, offs_i, out_v,
         out_i, misc, arcs, flat_kinds, flat_ctrl, flat_runs, flat_poly, in_attrs, out_attrs;
@@ -110,6 +111,10 @@ inline bool ensure(lyg_ctx* c, DevBuf& b, size_t bytes) {
     size_t cap = std::max(bytes, (size_t)4096);
     if (bytes < ((size_t)256 << 20)) cap = std::max(cap, 2 * old_cap);
     cap = (cap + 4095) & ~(size_t)4095;
+    if (c->alloc_limit && bytes > c->alloc_limit) {
+        c->last_error = "hipMalloc: over the allocation limit";
+        return false;
+    }
     if (!check(c, hipMalloc(&b.p, cap), "hipMalloc")) return false;
     b.cap = cap;
     return true;

@@ -173,11 +173,11 @@ struct RoundPlan {
 
 // Plans round `round` over the paths `todo`, with `scale` times the first round's room.  A
 // captured graph has no second round: there every register launch is followed by a sweep over
-// arrays of the paths that outgrew it.
+// arrays of the paths that outgrew it.  registers false: every path goes over arrays (no log).
 int32_t plan_round(lyg_ctx* c, const std::vector<uint32_t>& todo,
                    const std::vector<uint32_t>& bound, const std::vector<uint32_t>& degree,
                    const std::vector<uint32_t>& inter, const std::vector<uint64_t>& need,
-                   int round, uint64_t scale, bool graph, RoundPlan* P) {
+                   int round, uint64_t scale, bool registers, bool graph, RoundPlan* P) {
     // the register sweep's log takes 52 bytes per staged triangle
     uint64_t all_v = 0, all_t = 0;
     for (uint32_t p : todo) {
@@ -187,7 +187,8 @@ int32_t plan_round(lyg_ctx* c, const std::vector<uint32_t>& todo,
         all_t += t;
     }
     const uint32_t mode = c->fill_lds_resident;
-    const bool reg = round <= (mode == 1 ? 1 : 0) && 8 * all_v + 64 * all_t <= STAGE_BUDGET;
+    const bool reg = registers && round <= (mode == 1 ? 1 : 0) &&
+                     8 * all_v + 64 * all_t <= STAGE_BUDGET;
     auto shape = [&](uint32_t p) { return Shape{bound[p], degree[p]}; };
     P->log_ops = reg ? all_t : 0;
     // order by launch: size class, then the form (the first round picks it per path, the
@@ -372,6 +373,14 @@ hipError_t launch_again(lyg_ctx* c, lyg::FillLaunch L, const Launch& ln, uint8_t
     return lyg_launch_fill_sweep(&L, (int)ln.again_blocks, s);
 }
 
+// The register sweep's log: what the sweep over arrays does without.
+bool ensure_log(lyg_ctx* c, const RoundPlan& P, uint32_t n, DevBuf& ops, DevBuf& op_tris,
+                DevBuf& path_ops) {
+    return !P.log_ops || (ensure(c, ops, sizeof(lyg::FillOp) * P.log_ops) &&
+                          ensure(c, op_tris, sizeof(lyg::FillTri) * P.log_ops) &&
+                          ensure(c, path_ops, 4ull * n));
+}
+
 struct FillJob {
     lyg::PathBatchDev in;
     const lyg_fill_options* opts;
@@ -452,23 +461,35 @@ int32_t fill_sweep(lyg_ctx* c, const FillJob& J, uint32_t* vtx_off, uint32_t* id
     }
     uint64_t scale = 1, next_scale = 4;
     int round = 0;
+    bool registers = true;
     for (; round < MAX_ROUNDS && !todo.empty(); ++round, scale = next_scale) {
         RoundPlan P;
-        const int32_t planned = plan_round(c, todo, bound, degree, inter, need, round, scale, false, &P);
+        const int32_t planned =
+            plan_round(c, todo, bound, degree, inter, need, round, scale, registers, false, &P);
         if (planned != LYG_OK) return planned;
         const std::vector<uint32_t>& list = P.list;
         const std::vector<uint64_t>& offs = P.offs;
         const size_t m = list.size();
         const uint64_t* sv = offs.data();
         const uint64_t* st = offs.data() + m + 1;
-        if (!ensure_at(c, c->f_list, round, 4 * m) ||
-            !ensure_at(c, c->f_stage_off, round, 8 * offs.size()) ||
-            !ensure_at(c, c->f_stage_v, round, 8 * sv[m]) ||
-            !ensure_at(c, c->f_stage_t, round, 12 * st[m]) ||
-            (P.log_ops && (!ensure(c, c->f_ops, sizeof(lyg::FillOp) * P.log_ops) ||
-                           !ensure(c, c->f_op_tris, sizeof(lyg::FillTri) * P.log_ops))) ||
-            !ensure(c, c->f_path_ops, 4ull * n))
-            return LYG_ERR_DEVICE;
+        const bool staged = ensure_at(c, c->f_list, round, 4 * m) &&
+                            ensure_at(c, c->f_stage_off, round, 8 * offs.size()) &&
+                            ensure_at(c, c->f_stage_v, round, 8 * sv[m]) &&
+                            ensure_at(c, c->f_stage_t, round, 12 * st[m]);
+        const bool worked = staged && ensure_log(c, P, n, c->f_ops, c->f_op_tris, c->f_path_ops) &&
+                            ensure(c, c->f_work, P.work_bytes);
+        if (!worked && registers) {
+            // no memory with a log (this round's, or an earlier call's): the sweep over arrays
+            // needs none
+            (void)hipGetLastError();
+            free_buf(c->f_ops);
+            free_buf(c->f_op_tris);
+            registers = false;
+            next_scale = scale;
+            --round;
+            continue;
+        }
+        if (!worked) return staged ? LYG_ERR_NO_SPACE : LYG_ERR_DEVICE;
         uint32_t* d_list = as<uint32_t>(c->f_list[round]);
         uint64_t* d_off = as<uint64_t>(c->f_stage_off[round]);
         if (!check(c, hipMemcpyAsync(d_list, list.data(), 4 * m, hipMemcpyHostToDevice, s), "H2D") ||
@@ -488,7 +509,6 @@ int32_t fill_sweep(lyg_ctx* c, const FillJob& J, uint32_t* vtx_off, uint32_t* id
         L.op_tris = as<lyg::FillTri>(c->f_op_tris);
         L.path_ops = as<uint32_t>(c->f_path_ops);
         const std::vector<Launch>& launches = P.launches;
-        if (!ensure(c, c->f_work, P.work_bytes)) return LYG_ERR_NO_SPACE;
         const auto t_round = std::chrono::steady_clock::now();
         if (c->timing && round == 0) (void)hipEventRecord(c->ev[2], s);
         const size_t n_streams = std::min<size_t>(launches.size(), CLASS_STREAMS);
@@ -739,18 +759,26 @@ int32_t lygi::fill_graph_capture(lyg_ctx* c, const lyg_batch_in* in, const lyg_f
         todo[i] = i;
     }
     RoundPlan P;
-    const int32_t planned = plan_round(c, todo, bound, degree, inter, need, 0, 1, true, &P);
-    if (planned != LYG_OK) return planned;
+    bool staged = false, worked = false;
+    for (bool registers : {true, false}) {
+        P = RoundPlan();
+        const int32_t planned =
+            plan_round(c, todo, bound, degree, inter, need, 0, 1, registers, true, &P);
+        if (planned != LYG_OK) return planned;
+        const size_t k = P.list.size();
+        staged = ensure(c, g->list, 4 * k) && ensure(c, g->off, 8 * P.offs.size()) &&
+                 ensure(c, g->stage_v, 8 * P.offs[k]) &&
+                 ensure(c, g->stage_t, 12 * P.offs[2 * k + 1]);
+        worked = staged && ensure_log(c, P, n, g->ops, g->op_tris, g->path_ops) &&
+                 ensure(c, g->work, P.work_bytes);
+        if (worked) break;
+        // no memory with a log: the sweep over arrays needs none
+        (void)hipGetLastError();
+        free_buf(g->ops);
+        free_buf(g->op_tris);
+    }
+    if (!worked) return staged ? LYG_ERR_NO_SPACE : LYG_ERR_DEVICE;
     const size_t m = P.list.size();
-    const uint64_t* sv = P.offs.data();
-    const uint64_t* st = P.offs.data() + m + 1;
-    if (!ensure(c, g->list, 4 * m) || !ensure(c, g->off, 8 * P.offs.size()) ||
-        !ensure(c, g->stage_v, 8 * sv[m]) || !ensure(c, g->stage_t, 12 * st[m]) ||
-        (P.log_ops && (!ensure(c, g->ops, sizeof(lyg::FillOp) * P.log_ops) ||
-                       !ensure(c, g->op_tris, sizeof(lyg::FillTri) * P.log_ops))) ||
-        !ensure(c, g->path_ops, 4ull * n))
-        return LYG_ERR_DEVICE;
-    if (!ensure(c, g->work, P.work_bytes)) return LYG_ERR_NO_SPACE;
     uint32_t* d_list = as<uint32_t>(g->list);
     uint64_t* d_off = as<uint64_t>(g->off);
     if (!check(c, hipMemcpyAsync(d_list, P.list.data(), 4 * m, hipMemcpyHostToDevice, s), "H2D") ||
@@ -905,6 +933,10 @@ void lygi::fill_graph_destroy(FillGraph* g) {
 
 extern "C" {
 
+// Not in lyg.h: makes the context refuse device buffers beyond `bytes` (0: none), as a GPU that
+// is out of memory does.
+void lyg_ctx_set_alloc_limit(lyg_ctx* c, uint64_t bytes) { c->alloc_limit = bytes; }
+
 // Not in lyg.h: the launches of the first round over paths of these measures, on the host
 // alone, and the events a context has to join launches with (one more than it can hold).
 int32_t lyg_fill_plan_launches(const uint32_t* bound, const uint32_t* degree,
@@ -918,7 +950,7 @@ int32_t lyg_fill_plan_launches(const uint32_t* bound, const uint32_t* degree,
     for (uint32_t i = 0; i < n; ++i) need[i] = (uint64_t)bound[i] + 2ull * inter[i];
     RoundPlan P;
     const int32_t st = plan_round(&c, todo, {bound, bound + n}, {degree, degree + n},
-                                  {inter, inter + n}, need, 0, 1, false, &P);
+                                  {inter, inter + n}, need, 0, 1, true, false, &P);
     *launches = (uint32_t)P.launches.size();
     *events = (uint32_t)std::size(c.class_ev);
     return st;

@@ -335,3 +335,44 @@ def test_very_large_path():
     assert len(vb.vertices) == len(rv) and len(vb.indices) == len(ri)
     c = O.coverage_compare(rv, ri, vb.vertices, vb.indices, n=256)
     assert c["mismatch"] == 0 and abs(c["area_a"] - c["area_b"]) <= 1e-6 * c["area_b"]
+
+
+def test_without_memory_for_the_span_log():
+    """Where the register sweep's log (52 bytes per staged triangle) cannot be allocated, the
+    paths are swept over arrays, which need none: an eager call and a captured one on a context
+    that refuses the log give the bytes of one that does not.  20,000 triangles stage 12
+    million: 388 MB of the log's larger array, 146 MB of triangles."""
+    import ctypes as C
+    import threading
+
+    from lyon_amd import _lib
+    from lyon_amd.batch import DeviceBatch, FillBatcher, FillGraph, _Ctx, synchronize
+    from lyon_amd.path import PathBatch
+    rng = np.random.default_rng(9)
+    n = 20000
+    batch = PathBatch.from_paths([polygon(t) for t in rng.uniform(0, 500, (n, 3, 2))])
+    db = DeviceBatch(batch, workloads.fill_options(n, tolerance=0.05))
+    lib = C.CDLL(_lib.LIB_PATH)
+    lib.lyg_ctx_set_alloc_limit.argtypes = [C.c_void_p, C.c_uint64]
+    lib.lyg_ctx_set_alloc_limit.restype = None
+    outs = {}
+
+    def fresh(limit):  # a context of its own
+        lib.lyg_ctx_set_alloc_limit(_Ctx.get(), limit)
+        res = FillBatcher().run(db)
+        said = _lib.lib().lyg_ctx_last_error(_Ctx.get()).decode()
+        synchronize()
+        g = FillGraph(db, int(res.n_vertices), int(res.n_indices))
+        g.launch()
+        outs[limit] = [said] + [(r.status.copy(), r.all_vertices().view(np.uint32).copy(),
+                                 r.all_indices().copy()) for r in (res, g.result())]
+
+    for limit in (0, 256 << 20):
+        t = threading.Thread(target=fresh, args=(limit,))
+        t.start()
+        t.join()
+    assert "limit" not in outs[0][0] and "limit" in outs[256 << 20][0]
+    first = outs[0][1]
+    assert not first[0].any() and len(first[1]) > 0
+    for other in outs[0][2:] + outs[256 << 20][1:]:
+        assert all(np.array_equal(a, b) for a, b in zip(first, other))
