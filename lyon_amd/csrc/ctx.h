@@ -40,6 +40,8 @@ struct lyg_ctx {
     // fill launch shape (set by the autotuner): waves per block, LDS bytes per wave
     uint32_t fill_waves_per_block = 2;
     uint32_t fill_hot_bytes = 16 * 1024;
+    uint32_t last_fill_rounds = 0;   // sweep rounds of the last eager fill, and its last one's
+    uint64_t last_fill_scale = 0;    // room as a multiple of the first's
     uint32_t fill_lds_resident = 1;  // first round with the active edges in registers
     // fill: per-path arrays, per-wave working memory and per-round staging
     DevBuf f_bound, f_status, f_round, f_hint, f_work, f_counters, f_ops, f_op_tris,

@@ -168,7 +168,7 @@ __global__ void __launch_bounds__(WAVE* FILL_MAX_WAVES_PER_BLOCK) fill_sweep_ker
     uint32_t k = readlane_u(atomicAdd(L.work_counter, lane_id() == 0 ? 1u : 0u), 0);
     while (k < L.n_list) {
         const uint32_t path = L.path_list ? L.path_list[k] : k;
-        if (L.only_retry && L.path_status[path] != fillk::ST_RETRY) {
+        if (L.only_retry && !fillk::is_retry(L.path_status[path])) {
             k = readlane_u(atomicAdd(L.work_counter, lane_id() == 0 ? 1u : 0u), 0);
             continue;
         }
@@ -224,8 +224,8 @@ __global__ void fill_status_out_kernel(const uint32_t* st, uint32_t* out, uint32
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     const uint32_t v = st[i];
-    out[i] = v == fillk::ST_RETRY ? (uint32_t)LYG_ERR_NO_SPACE
-                                  : v == 0xffffffffu ? (uint32_t)LYG_ERR_INTERNAL : v;
+    out[i] = fillk::is_retry(v) ? (uint32_t)LYG_ERR_NO_SPACE
+                                : v == 0xffffffffu ? (uint32_t)LYG_ERR_INTERNAL : v;
 }
 
 // What sizes a path's first sweep, by a wave per path with a lane per verb:

@@ -43,9 +43,12 @@ hipError_t lyg_launch_fill_u32(uint32_t* p, uint32_t n, uint32_t v, hipStream_t 
 
 namespace {
 
-constexpr uint32_t ST_RETRY = 100;
+using lyg::fillk::ST_RETRY;
+using lyg::fillk::ST_RETRY_ARRAYS;
+using lyg::fillk::REG_MAX_ROWS;
+using lyg::fillk::REG_MAX_SETS;
 constexpr uint32_t ST_UNSWEPT = 0xffffffffu;  // written before a round, replaced per path
-constexpr int MAX_ROUNDS = 5;
+constexpr int MAX_ROUNDS = 7;                        // two with registers, five with more room
 constexpr uint64_t MAX_PATH_EVENTS = 1ull << 27;     // larger paths: LYG_ERR_NO_SPACE
 constexpr size_t WORK_BUDGET = 16ull << 30;          // working memory of one round
 constexpr size_t STAGE_BUDGET = 64ull << 30;         // staging memory of one round
@@ -54,8 +57,7 @@ constexpr int MAX_CLASSES = 8;
 // or with its active edges in registers (2, 5 or 16 sets of 64).
 constexpr int N_FORMS = 4;
 constexpr int FORM_ARRAYS = 0;
-constexpr uint32_t REG_CHUNKS[N_FORMS] = {0, 2, 5, 16};
-constexpr uint32_t REG_MAX_ROWS = 44;  // pending events per column: 66 KiB of LDS
+constexpr uint32_t REG_CHUNKS[N_FORMS] = {0, 2, 5, REG_MAX_SETS};
 constexpr int MAX_LAUNCHES = N_FORMS * MAX_CLASSES;
 static_assert(MAX_LAUNCHES <= FILL_MAX_LAUNCHES, "lyg_ctx::class_ev has an event per launch");
 constexpr int N_GRAPH_COUNTERS = 2 * MAX_LAUNCHES;  // a launch and the sweep after it
@@ -171,13 +173,13 @@ struct RoundPlan {
     uint64_t log_ops = 0;        // operations the register sweep's log holds
 };
 
-// Plans round `round` over the paths `todo`, with `scale` times the first round's room.  A
-// captured graph has no second round: there every register launch is followed by a sweep over
+// Plans round `round` over the paths `todo`, with `scale` times the first round's room;
+// arrays[p]: the path has met a limit of every register launch.  A captured graph has no second round: there every register launch is followed by a sweep over
 // arrays of the paths that outgrew it.  registers false: every path goes over arrays (no log).
 int32_t plan_round(lyg_ctx* c, const std::vector<uint32_t>& todo,
                    const std::vector<uint32_t>& bound, const std::vector<uint32_t>& degree,
                    const std::vector<uint32_t>& inter, const std::vector<uint64_t>& need,
-                   int round, uint64_t scale, bool registers, bool graph, RoundPlan* P) {
+                   const std::vector<uint8_t>& arrays, int round, uint64_t scale, bool registers, bool graph, RoundPlan* P) {
     // the register sweep's log takes 52 bytes per staged triangle
     uint64_t all_v = 0, all_t = 0;
     for (uint32_t p : todo) {
@@ -190,18 +192,19 @@ int32_t plan_round(lyg_ctx* c, const std::vector<uint32_t>& todo,
     const bool reg = registers && round <= (mode == 1 ? 1 : 0) &&
                      8 * all_v + 64 * all_t <= STAGE_BUDGET;
     auto shape = [&](uint32_t p) { return Shape{bound[p], degree[p]}; };
-    P->log_ops = reg ? all_t : 0;
+    P->log_ops = 0;
     // order by launch: size class, then the form (the first round picks it per path, the
-    // second takes all the register sets, later ones sweep over arrays); then by path
+    // second takes all the register sets, later ones sweep over arrays, as do paths with more
+    // than a lane per edge at one point from then on); then by path
     std::vector<int> cls(todo.size());
     for (size_t k = 0; k < todo.size(); ++k) {
         const uint32_t p = todo[k];
-        const int form = !reg ? FORM_ARRAYS
+        const int form = !reg || arrays[p] ? FORM_ARRAYS
                          : round == 0 ? path_form(shape(p), mode)
-                         : mode && act_estimate(shape(p)) <= 64 * REG_CHUNKS[N_FORMS - 1]
-                             ? N_FORMS - 1
-                             : FORM_ARRAYS;
+                         : act_estimate(shape(p)) <= 64 * REG_MAX_SETS ? N_FORMS - 1
+                                                                       : FORM_ARRAYS;
         cls[k] = N_FORMS * size_class(need[p]) + form;
+        if (form != FORM_ARRAYS) P->log_ops = all_t;
     }
     std::vector<size_t> order(todo.size());
     std::iota(order.begin(), order.end(), 0);
@@ -445,7 +448,8 @@ int32_t fill_sweep(lyg_ctx* c, const FillJob& J, uint32_t* vtx_off, uint32_t* id
     std::vector<uint64_t> need(n);
     for (uint32_t i = 0; i < n; ++i) need[i] = (uint64_t)bound[i] + 2ull * inter[i];
     R->status.assign(n, 0);
-    // paths still to sweep, with their scale (4^round)
+    // paths still to sweep, and those that registers cannot hold
+    std::vector<uint8_t> arrays(n, 0);
     std::vector<uint32_t> todo;
     todo.reserve(n);
     for (uint32_t i = 0; i < n; ++i) {
@@ -459,13 +463,14 @@ int32_t fill_sweep(lyg_ctx* c, const FillJob& J, uint32_t* vtx_off, uint32_t* id
             !check(c, lyg_launch_fill_u32(L.path_round, n, 0xffffffffu, s), "zero"))
             return LYG_ERR_DEVICE;
     }
-    uint64_t scale = 1, next_scale = 4;
+    uint64_t scale = 1, next_scale = 1;
     int round = 0;
     bool registers = true;
     for (; round < MAX_ROUNDS && !todo.empty(); ++round, scale = next_scale) {
         RoundPlan P;
         const int32_t planned =
-            plan_round(c, todo, bound, degree, inter, need, round, scale, registers, false, &P);
+            plan_round(c, todo, bound, degree, inter, need, arrays, round, scale, registers,
+                       false, &P);
         if (planned != LYG_OK) return planned;
         const std::vector<uint32_t>& list = P.list;
         const std::vector<uint64_t>& offs = P.offs;
@@ -551,14 +556,19 @@ int32_t fill_sweep(lyg_ctx* c, const FillJob& J, uint32_t* vtx_off, uint32_t* id
             !check(c, hipStreamSynchronize(s), "sync"))
             return LYG_ERR_DEVICE;
         std::vector<uint32_t> next;
-        uint64_t grow = 4;  // next round's room: at least 4x, more if a path's hint asks
+        // next round's room: at least 4x if a path needs more, beyond that as their hints ask;
+        // the same for paths that only outgrew their registers (4x each time, a batch within
+        // the staging budget could end beyond it without needing the room)
+        uint64_t grow = 1;
         for (uint32_t p : list) {
             if (st_h[p] == ST_UNSWEPT) {  // no wave took the path: a launch error
                 c->last_error = "fill: a path was not swept";
                 return LYG_ERR_INTERNAL;
             }
-            if (st_h[p] == ST_RETRY) {
+            if (lyg::fillk::is_retry(st_h[p])) {
                 next.push_back(p);
+                if (st_h[p] == ST_RETRY) grow = std::max<uint64_t>(grow, 4);
+                if (st_h[p] == ST_RETRY_ARRAYS) arrays[p] = 1;
                 uint64_t v, t;
                 stage_caps(bound[p], inter[p], scale, &v, &t);
                 const uint64_t want = (uint64_t)hint_h[p] + hint_h[p] / 4;
@@ -575,9 +585,11 @@ int32_t fill_sweep(lyg_ctx* c, const FillJob& J, uint32_t* vtx_off, uint32_t* id
             fflush(stderr);
         }
         todo.swap(next);
+        c->last_fill_scale = scale;
         next_scale = scale * grow;
     }
     R->rounds = round;
+    c->last_fill_rounds = (uint32_t)round;
     for (uint32_t p : todo) R->status[p] = LYG_ERR_NO_SPACE;  // still out of room
     // step 3: offsets
     if (!check(c, lyg_launch_fill_u32(c->d_counters + 4, 1, 0, s), "reset") ||
@@ -763,7 +775,8 @@ int32_t lygi::fill_graph_capture(lyg_ctx* c, const lyg_batch_in* in, const lyg_f
     for (bool registers : {true, false}) {
         P = RoundPlan();
         const int32_t planned =
-            plan_round(c, todo, bound, degree, inter, need, 0, 1, registers, true, &P);
+            plan_round(c, todo, bound, degree, inter, need, std::vector<uint8_t>(n), 0, 1,
+                       registers, true, &P);
         if (planned != LYG_OK) return planned;
         const size_t k = P.list.size();
         staged = ensure(c, g->list, 4 * k) && ensure(c, g->off, 8 * P.offs.size()) &&
@@ -910,7 +923,7 @@ int32_t lygi::fill_graph_result(FillGraph* g, uint64_t* n_vertices, uint64_t* n_
     if (tot[0] > g->vertex_capacity || tot[1] > g->index_capacity) return LYG_ERR_CAPACITY;
     for (uint32_t v : st) {
         if (v == 0) continue;
-        if (v == ST_RETRY) return LYG_ERR_NO_SPACE;
+        if (lyg::fillk::is_retry(v)) return LYG_ERR_NO_SPACE;
         if (v == ST_UNSWEPT) return LYG_ERR_INTERNAL;
         return (int32_t)v;
     }
@@ -937,6 +950,12 @@ extern "C" {
 // is out of memory does.
 void lyg_ctx_set_alloc_limit(lyg_ctx* c, uint64_t bytes) { c->alloc_limit = bytes; }
 
+// Not in lyg.h: how the last eager fill went.
+void lyg_ctx_last_fill(const lyg_ctx* c, uint32_t* rounds, uint64_t* scale) {
+    *rounds = c->last_fill_rounds;
+    *scale = c->last_fill_scale;
+}
+
 // Not in lyg.h: the launches of the first round over paths of these measures, on the host
 // alone, and the events a context has to join launches with (one more than it can hold).
 int32_t lyg_fill_plan_launches(const uint32_t* bound, const uint32_t* degree,
@@ -950,7 +969,8 @@ int32_t lyg_fill_plan_launches(const uint32_t* bound, const uint32_t* degree,
     for (uint32_t i = 0; i < n; ++i) need[i] = (uint64_t)bound[i] + 2ull * inter[i];
     RoundPlan P;
     const int32_t st = plan_round(&c, todo, {bound, bound + n}, {degree, degree + n},
-                                  {inter, inter + n}, need, 0, 1, true, false, &P);
+                                  {inter, inter + n}, need, std::vector<uint8_t>(n), 0, 1, true,
+                                  false, &P);
     *launches = (uint32_t)P.launches.size();
     *events = (uint32_t)std::size(c.class_ev);
     return st;

@@ -30,7 +30,6 @@ enum : uint32_t {
     ST_POSITION_NAN = 3,
     ST_TOLERANCE_NAN = 4,
     ST_INTERNAL = 5,
-    ST_RETRY = 100,  // a scratch capacity was exceeded: rerun with more room
 };
 
 __device__ __forceinline__ int cmp_pos(vec2 a, vec2 b) {

@@ -18,8 +18,9 @@
 //     go where the sweep would have written them.
 // Vertices, triangles and their order are those of the sweep over arrays.
 //
-// A path stops with the retry status when it has more than 64 C active edges (or spans),
-// more than 64 edges below one event, or more pending intersections than its columns hold.
+// A path stops with a retry status when it has more than 64 C active edges (or spans) or more
+// pending intersections than its columns hold, which a launch of more may, or more than 64 edges
+// below one event (spans it ends, pushes), which is left to the sweep over arrays.
 #include <hip/hip_runtime.h>
 
 #include "fill_core.h"
@@ -160,6 +161,9 @@ __device__ __forceinline__ void reg_sweep(const FillLaunch& L, uint32_t path, ui
     FillOp* ops = L.ops + L.stage_t_off[k];
     const uint32_t op_cap = uni((uint32_t)(L.stage_t_off[k + 1] - L.stage_t_off[k]));
 
+    // the status of a path that outgrows the sets, or the columns
+    const uint32_t MORE_SETS = C < (int)REG_MAX_SETS ? ST_RETRY_SETS : ST_RETRY_ARRAYS;
+    const uint32_t MORE_ROWS = H.rows < REG_MAX_ROWS ? ST_RETRY_SETS : ST_RETRY_ARRAYS;
     uint32_t status = ST_OK;
     auto fail = [&](uint32_t st) { status = uni(status == ST_OK ? st : status); };
     // active edges (fill.rs:153-170): winding (low 16 bits) | merge, first vertex id
@@ -208,7 +212,7 @@ __device__ __forceinline__ void reg_sweep(const FillLaunch& L, uint32_t path, ui
     uint32_t cv = 0;
     auto add_below = [&](vec2 to, int32_t w) {
         if (n_below >= (uint32_t)WAVE) {
-            fail(ST_RETRY);
+            fail(ST_RETRY_ARRAYS);
             return;
         }
         const float key = slope(sub(to, cp));
@@ -221,7 +225,7 @@ __device__ __forceinline__ void reg_sweep(const FillLaunch& L, uint32_t path, ui
     };
     auto push_later = [&](vec2 pos, vec2 to, int32_t w, bool edge) {
         if (n_push >= (uint32_t)WAVE) {
-            fail(ST_RETRY);
+            fail(ST_RETRY_ARRAYS);
             return;
         }
         const bool me = ul == n_push;
@@ -234,7 +238,7 @@ __device__ __forceinline__ void reg_sweep(const FillLaunch& L, uint32_t path, ui
     };
     auto span_op = [&](uint32_t kind, int32_t idx, vec2 pos, uint32_t id) {
         if (n_acts >= (uint32_t)WAVE) {
-            fail(ST_RETRY);
+            fail(ST_RETRY_ARRAYS);
             return;
         }
         const bool me = ul == n_acts;
@@ -280,7 +284,7 @@ __device__ __forceinline__ void reg_sweep(const FillLaunch& L, uint32_t path, ui
                         break;
                     }
                     if (n_spans + 1u > 64u * (uint32_t)C) {
-                        fail(ST_RETRY);
+                        fail(MORE_SETS);
                         break;
                     }
                 }
@@ -629,7 +633,7 @@ __device__ __forceinline__ void reg_sweep(const FillLaunch& L, uint32_t path, ui
                         first = false;
                     }
                     if (n_end > (uint32_t)WAVE || n_split > (uint32_t)WAVE) {
-                        fail(ST_RETRY);
+                        fail(ST_RETRY_ARRAYS);
                         break;
                     }
                 }
@@ -928,7 +932,7 @@ __device__ __forceinline__ void reg_sweep(const FillLaunch& L, uint32_t path, ui
             const uint32_t a = above_start, removed = above_end - a, added = n_below;
             const uint32_t n_new = n_act - removed + added;
             if (n_new > act_cap) {
-                fail(ST_RETRY);
+                fail(MORE_SETS);
                 break;
             }
             if (added > removed) {
@@ -980,7 +984,7 @@ __device__ __forceinline__ void reg_sweep(const FillLaunch& L, uint32_t path, ui
         // ---- the event's pushes (EventQueue::insert_sorted, event_queue.rs:188-250) ----
         for (uint32_t q = 0; q < n_push; ++q) {
             if (heap_n >= heap_cap) {
-                fail(ST_RETRY);
+                fail(MORE_ROWS);
                 break;
             }
             const vec2 pos = readlane_v(mk(q_px, q_py), (int)q);
@@ -992,7 +996,7 @@ __device__ __forceinline__ void reg_sweep(const FillLaunch& L, uint32_t path, ui
                 m = ballot(h_cnt <= level);
             }
             if (level >= H.rows) {
-                fail(ST_RETRY);
+                fail(MORE_ROWS);
                 break;
             }
             const uint32_t hi = fkey(pos.y), lo = fkey(pos.x);
@@ -1023,7 +1027,7 @@ __device__ __forceinline__ void reg_sweep(const FillLaunch& L, uint32_t path, ui
     *out_status = status;
     *out_nv = nv;
     *out_ops = n_ops;
-    if (status == ST_RETRY) {
+    if (is_retry(status)) {
         const uint64_t est = (uint64_t)nv * (uint64_t)(n_static ? n_static : 1u) /
                              (uint64_t)(cur ? cur : 1u);
         *out_hint = est > 0xffffffffull ? 0xffffffffu : (uint32_t)est;
@@ -1255,7 +1259,7 @@ __global__ void __launch_bounds__(WAVE) fill_reg_kernel(FillLaunch L) {
             L.path_ni[path] = 0u;  // until the triangles are counted
             L.path_ops[path] = n_ops;
             L.path_round[path] = L.round;
-            if (L.path_hint) L.path_hint[path] = st == ST_RETRY ? hint : 0u;
+            if (L.path_hint) L.path_hint[path] = is_retry(st) ? hint : 0u;
         }
         k = readlane_u(atomicAdd(L.work_counter, lane_id() == 0 ? 1u : 0u), 0);
     }

@@ -132,6 +132,13 @@ namespace fillk {
 struct FillCaps {
     uint32_t ev, heap, act, span, node, below;
 };
+// A path's sweep that has to be done again (statuses of the sweep's own): with more room; with
+// more register sets or columns of pending events than its launch had; over arrays, as it met a
+// limit of every register launch.
+enum : uint32_t { ST_RETRY = 100, ST_RETRY_SETS = 101, ST_RETRY_ARRAYS = 102 };
+static constexpr uint32_t REG_MAX_SETS = 16;  // register sets of 64 active edges
+static constexpr uint32_t REG_MAX_ROWS = 44;  // pending events per column: 66 KiB of LDS
+constexpr bool is_retry(uint32_t status) { return status - ST_RETRY < 3u; }
 }  // namespace fillk
 
 // A span operation of the register sweep's log (fill_reg.hip).

@@ -376,3 +376,20 @@ def test_without_memory_for_the_span_log():
     assert not first[0].any() and len(first[1]) > 0
     for other in outs[0][2:] + outs[256 << 20][1:]:
         assert all(np.array_equal(a, b) for a, b in zip(first, other))
+
+
+@pytest.mark.parametrize("shape,size,rounds", [
+    (fan, 62, 1), (fan, 126, 2),             # more than 64 edges below one event: over arrays next
+    (zigzag, 126, 1), (zigzag, 1900, 1),     # estimated right
+    (zigzag, 1020, 1)], ids=["fan62", "fan126", "zigzag126", "zigzag1900", "zigzag1020"])
+def test_rounds_of_paths_that_outgrow_the_registers(shape, size, rounds):
+    """A path that meets a limit of every register launch is swept over arrays in the next
+    round, with the room it had (it needed no more)."""
+    import ctypes as C
+
+    from lyon_amd import _lib
+    from lyon_amd.batch import _Ctx
+    st, _, _ = gpu_fill(shape(size), FillOptions(tolerance=0.05))
+    n, scale = C.c_uint32(0), C.c_uint64(0)
+    C.CDLL(_lib.LIB_PATH).lyg_ctx_last_fill(C.c_void_p(_Ctx.get()), C.byref(n), C.byref(scale))
+    assert st == 0 and (n.value, scale.value) == (rounds, 1)
