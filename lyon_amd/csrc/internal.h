@@ -24,8 +24,8 @@ struct BatchSpec {
     uint32_t* idx_off;       // device, n + 1
 };
 
-// How a batched stroke cuts its long paths: parts of `windows` windows (0: whole paths), or of
-// as many more as make max_parts parts of a path (0: any number).
+// How a batched stroke cuts its long paths: parts of `windows` windows (0: whole paths), after
+// a path's first max_parts (0: none) of 64.
 struct Cutting {
     uint32_t windows, max_parts;
 };

@@ -869,12 +869,13 @@ __device__ __forceinline__ void item_room(uint64_t steps, uint64_t verbs, uint64
 }
 
 // The cutting of one path into items.  A path of one sub-path with at least
-// 2 * split_windows windows is cut into parts of split_windows windows (part j starts at
-// window j * split_windows of the path; its prologue is the window before it), or of as many
-// more as make max_parts parts of it (0: any number); every other path is one item.  PLAN: counts the parts beyond the first and the staging room
-// of all of them (*extra, *rv, *ri).  Otherwise: writes the items, item 0 at index
-// `path`, parts 1.. from extra_first, staging rooms from v_base / i_base on (the rooms
-// are recomputed exactly as planned).  One wave.
+// 2 * split_windows windows is cut into parts of split_windows windows, the ones after the
+// first max_parts (0: none) of COARSE_WINDOWS (a part's prologue is the window before it);
+// every other path is one item.  PLAN: counts the parts beyond the first and the staging room of all of them
+// (*extra, *rv, *ri).  Otherwise: writes the items, item 0 at index `path`, parts 1.. from
+// extra_first, staging rooms from v_base / i_base on (the rooms are recomputed exactly as
+// planned).  One wave.
+static constexpr uint32_t COARSE_WINDOWS = 64;  // a prologue then costs 1/64 of its part
 template <bool PLAN>
 __device__ void cut_path(const StrokeLaunch& L, uint32_t path, uint32_t split_windows,
                          uint32_t max_parts, float room_scale, uint32_t* extra, uint32_t* rv, uint32_t* ri,
@@ -896,18 +897,6 @@ __device__ void cut_path(const StrokeLaunch& L, uint32_t path, uint32_t split_wi
         A = arc_count(arc_subdivisions(2.0f * 3.14159265358979323846f, hw, tol));
     // parts of split_windows windows; with PLAN the eligibility is decided at the end
     const bool cut = PLAN ? split_windows > 0 : n_extra_planned > 0;
-    if (cut && max_parts) {
-        uint64_t all = 0;
-        uint32_t pts_before = 0;
-        for (uint32_t v0 = 0; v0 < nverbs; v0 += WAVE) {
-            uint8_t mv;
-            uint32_t off, cnt;
-            all += (chunk_steps(verbs, nverbs, v0, pts, npts, &pts_before, tol, &mv, &off, &cnt) +
-                    WAVE - 1) / WAVE;
-        }
-        const uint64_t most = (all + max_parts - 1) / max_parts;
-        if (most > split_windows) split_windows = (uint32_t)min<uint64_t>(most, 1u << 30);
-    }
     uint64_t steps = 0, windows = 0, sum_v = 0, sum_i = 0;
     uint32_t n_begin = 0, n_end = 0, pt_carry = 0, open_j = 0;
     bool end_last = false;
@@ -921,6 +910,8 @@ __device__ void cut_path(const StrokeLaunch& L, uint32_t path, uint32_t split_wi
     StrokeItem cur{};
     cur.path = path;
     cur.flags = ITEM_FIRST | ITEM_SPLIT;
+    const uint32_t fine = max_parts ? max_parts : ~0u;  // parts of split_windows
+    const uint32_t coarse = split_windows > COARSE_WINDOWS ? split_windows : COARSE_WINDOWS;
     uint64_t next_cut = split_windows;  // the window the next part starts at
     uint64_t cur_steps = 0, cur_verbs = 0;
     auto close_item = [&]() {
@@ -955,7 +946,7 @@ __device__ void cut_path(const StrokeLaunch& L, uint32_t path, uint32_t split_wi
             if (!cut) continue;
             const uint32_t nw = (ns + WAVE - 1) / WAVE;
             uint32_t part_s = 0;  // first step of the open part in this chunk
-            for (; next_cut < windows + nw; next_cut += split_windows) {
+            for (; next_cut < windows + nw; next_cut += open_j < fine ? split_windows : coarse) {
                 // the open part ends here; the next starts with its prologue
                 const uint32_t w = (uint32_t)(next_cut - windows), s0 = w * WAVE;
                 cur_steps += s0 - part_s;

@@ -95,6 +95,39 @@ def test_cutting_by_the_number_of_paths(n):
         assert np.array_equal(np.asarray(i), np.asarray(ri))
 
 
+@pytest.mark.parametrize("n,lines", [(3000, 400000), (7000, 128000), (40000, 128000)])
+def test_one_long_path_among_many_short_ones(n, lines):
+    """A context whose cutting was never set cuts a long path into parts of at most 64 windows
+    of 64 points, however many short paths come with it, and the bytes are those of the whole
+    walk."""
+    import threading
+
+    from lyon_amd.batch import DeviceBatch, StrokeBatcher, stroke_split_stats
+    rng = np.random.default_rng(n)
+    b = PathBuilder()
+    b.begin((0.0, 0.0))
+    for x, y in rng.uniform(0, 2048, (lines, 2)):
+        b.line_to((x, y))
+    b.end(False)
+    short = workloads.stroke_batch(n, 1, 4, 2048.0, seed=n)
+    batch = PathBatch.from_paths([short.path(i) for i in range(n)] + [b.build()])
+    opts = workloads.stroke_options(n + 1, tolerance=0.05, seed=n)
+    ref = run(DeviceBatch(batch, opts), 0)
+    got = []
+
+    def fresh():  # a context of its own
+        r = StrokeBatcher().run(DeviceBatch(batch, opts))
+        got.append(((r.vertex_offsets.copy(), r.index_offsets.copy(),
+                     r.all_vertices().view(np.uint32).copy(), r.all_indices().copy()),
+                    stroke_split_stats()["items"]))
+
+    t = threading.Thread(target=fresh)
+    t.start()
+    t.join()
+    same(ref, got[0][0], f"{n} paths and one of {lines} lines")
+    assert got[0][1] >= n + lines // 4096, got[0][1]
+
+
 def test_split_with_short_paths_mixed_in():
     """The 10,000-path batched stroke workload's first 2,000 paths (8-256 segments), most
     of them too short to split, with a few long ones."""
