@@ -68,6 +68,20 @@ def test_autotune_keeps_results():
     assert same(snapshot(fb.run(fdb, check=False)), fref)
 
 
+@pytest.mark.parametrize("n,windows", [(512, (0, 2, 4, 8, 16, 32, 64, 128)),
+                                       (513, (0, 16, 32, 64, 128))])
+def test_autotune_offers_fine_parts_to_few_paths(n, windows):
+    """Parts of less than 16 windows are chosen for at most 512 paths: the short paths of this
+    batch, whose every cutting takes the same time, are tuned to one of the offered numbers."""
+    batch = workloads.stroke_batch(n, 1, 2, 512.0, seed=8)
+    db = DeviceBatch(batch, workloads.stroke_options(n, seed=8))
+    b = StrokeBatcher()
+    ref = snapshot(b.run(db))
+    for _ in range(4):
+        assert autotune(b, db)["split_windows"] in windows
+    assert same(snapshot(b.run(db)), ref)
+
+
 def test_autotune_band_size_keeps_the_region():
     """The banded fill's band size changes its triangles, never the region: after the
     autotuner picks one, every path covers the same area (relative 1e-6 of the exact
