@@ -231,7 +231,10 @@ __global__ void fill_status_out_kernel(const uint32_t* st, uint32_t* out, uint32
 // What sizes a path's first sweep, by a wave per path with a lane per verb:
 //   * an upper bound of its events: flattened edges (the swapped-curve Wang counts) plus one
 //     vertex event per edge, plus the closing edges;
-//   * the sum of its segments' degrees, which a horizontal line crosses at most that often;
+//   * the sum of its segments' degrees, which a horizontal line crosses at most that often (the
+//     host takes half of them for active edges: combs of more than 1,024 verbs, where that
+//     decides between registers and arrays, are counted, or they outgrow the registers and
+//     are swept twice: a comb of 1,500 edges 47 ms, 34 ms so);
 //   * an estimate of its self-intersections, which its output and its pending events grow with
 //     and the event bound does not see.  Two segments can only cross if their boxes (of the
 //     control points, padded by the tolerance: the flattened edges lie within) overlap; the
@@ -246,6 +249,49 @@ __global__ void fill_status_out_kernel(const uint32_t* st, uint32_t* out, uint32
 // the pairs of those with more than `over`.  1,000 glyphs: 120 us when a thread walked a path,
 // once for the bound and once for boxes in memory, 13 us so.
 static constexpr uint32_t INTER_MAX_VERBS = 4096, INTER_FEW_VERBS = 1024;
+
+// The most segments that cross one sweep line, by their boxes (padded by `pad`), to within those
+// that begin or end in the same 1,024th of the path's extent.
+static constexpr uint32_t CROSS_BINS = 1024;
+__device__ __forceinline__ uint32_t segments_crossed(const float4* boxes, uint32_t nv, float pad,
+                                                     bool horizontal, int32_t* bins) {
+    const uint32_t l = (uint32_t)lane_id();
+    auto top = [&](const float4& b) { return (horizontal ? b.x : b.y) + pad; };
+    auto bottom = [&](const float4& b) { return (horizontal ? b.z : b.w) - pad; };
+    float lo = INFINITY, hi = -INFINITY;
+    for (uint32_t i = l; i < nv; i += WAVE) {
+        lo = ffmin(lo, top(boxes[i]));
+        hi = ffmax(hi, bottom(boxes[i]));
+    }
+    for (int d = 1; d < WAVE; d <<= 1) {
+        lo = ffmin(lo, u2f(shfl_u(f2u(lo), (int)l ^ d)));
+        hi = ffmax(hi, u2f(shfl_u(f2u(hi), (int)l ^ d)));
+    }
+    for (uint32_t i = l; i < CROSS_BINS; i += WAVE) bins[i] = 0;
+    wave_sync();
+    const float scale = (float)CROSS_BINS / (hi - lo);
+    auto bin = [&](float y) {
+        const float k = (y - lo) * scale;
+        return k >= 1.0f ? (k < (float)CROSS_BINS ? (uint32_t)k : CROSS_BINS - 1u) : 0u;
+    };
+    for (uint32_t i = l; i < nv; i += WAVE) {
+        const float t = top(boxes[i]), b = bottom(boxes[i]);
+        if (!(t <= b)) continue;
+        atomicAdd(&bins[bin(t)], 1);
+        const uint32_t after = bin(b) + 1u;
+        if (after < CROSS_BINS) atomicAdd(&bins[after], -1);
+    }
+    wave_sync();
+    constexpr uint32_t PER = CROSS_BINS / WAVE;
+    int32_t sum = 0, most = 0;
+    for (uint32_t k = 0; k < PER; ++k) {
+        sum += bins[l * PER + k];
+        most = sum > most ? sum : most;
+    }
+    const int32_t before = (int32_t)incl_scan((uint32_t)sum) - sum;
+    const int32_t here = before + most;  // (before alone is the last bin's of the lane before)
+    return readlane_u(incl_max_u32(here > 0 ? (uint32_t)here : 0u), WAVE - 1);
+}
 
 template <uint32_t CAP>
 __global__ void __launch_bounds__(WAVE) fill_measure_kernel(FillLaunch L, uint32_t over,
@@ -341,7 +387,15 @@ __global__ void __launch_bounds__(WAVE) fill_measure_kernel(FillLaunch L, uint32
         inter[path] = 0u;
         if (nv <= INTER_MAX_VERBS) *more = 1u;
     }
-    if (over) return;
+    if (over) {
+        // the host's estimate is 9/16 of the degree and 16
+        __shared__ int32_t bins[CROSS_BINS];
+        const uint32_t most = segments_crossed(
+            boxes, nv, pad, o.sweep_orientation == LYG_ORIENT_HORIZONTAL, bins);
+        const uint32_t least = most > 16u ? (most - 16u) * 16u / 9u + 2u : 0u;
+        if (l == 0 && least > degree[path]) degree[path] = least;
+        return;
+    }
     uint64_t all_edges = 0, all_deg = 0;
     for (int i = 0; i < WAVE; ++i) {
         all_edges += (uint64_t)readlane_u((uint32_t)(edges >> 32), i) << 32 |

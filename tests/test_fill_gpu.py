@@ -380,16 +380,24 @@ def test_without_memory_for_the_span_log():
 
 @pytest.mark.parametrize("shape,size,rounds", [
     (fan, 62, 1), (fan, 126, 2),             # more than 64 edges below one event: over arrays next
-    (zigzag, 126, 1), (zigzag, 1900, 1),     # estimated right
-    (zigzag, 1020, 1)], ids=["fan62", "fan126", "zigzag126", "zigzag1900", "zigzag1020"])
+    (zigzag, 126, 1), (zigzag, 1900, 1),     # estimated right; below, counted
+    (zigzag, 1020, 1), (zigzag, 1100, 1), (zigzag, 1500, 1), (zigzag, 1790, 1)],
+    ids=["fan62", "fan126", "zigzag126", "zigzag1900", "zigzag1020", "zigzag1100", "zigzag1500",
+         "zigzag1790"])
 def test_rounds_of_paths_that_outgrow_the_registers(shape, size, rounds):
     """A path that meets a limit of every register launch is swept over arrays in the next
-    round, with the room it had (it needed no more)."""
+    round, with the room it had (it needed no more).  A comb's edges are all active at once,
+    twice what half the degrees say: where that is beyond the registers it is known before, in
+    both orientations."""
     import ctypes as C
 
     from lyon_amd import _lib
     from lyon_amd.batch import _Ctx
-    st, _, _ = gpu_fill(shape(size), FillOptions(tolerance=0.05))
-    n, scale = C.c_uint32(0), C.c_uint64(0)
-    C.CDLL(_lib.LIB_PATH).lyg_ctx_last_fill(C.c_void_p(_Ctx.get()), C.byref(n), C.byref(scale))
-    assert st == 0 and (n.value, scale.value) == (rounds, 1)
+    up, side = shape(size), shape(size)
+    side.points = np.stack([side.points[:, 1], -side.points[:, 0]], axis=1)
+    for path, way in ((up, Orientation.Vertical), (side, Orientation.Horizontal)):
+        st, _, _ = gpu_fill(path, FillOptions(tolerance=0.05, sweep_orientation=way))
+        n, scale = C.c_uint32(0), C.c_uint64(0)
+        C.CDLL(_lib.LIB_PATH).lyg_ctx_last_fill(C.c_void_p(_Ctx.get()), C.byref(n),
+                                                C.byref(scale))
+        assert st == 0 and (n.value, scale.value) == (rounds, 1)
