@@ -323,9 +323,7 @@ struct SvgLaunch {
     uint32_t* n_errors;        // [0] strings with an error, [1] staging rooms overflowed
     uint8_t* verbs;            // staging rooms (see svg_parse_kernel)
     float* points;
-    // strings left to the serial parser (null: every string) and their number
-    uint32_t* serial;
-    uint32_t* n_serial;
+    uint32_t by_wave;          // a wave per string first; counts_v: SVG_LEFT for the serial parser
     // compaction
     const uint32_t* off_v;
     const uint32_t* off_p;

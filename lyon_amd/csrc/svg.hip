@@ -704,6 +704,7 @@ __device__ void parse_svg(const uint8_t* s, uint32_t a, uint32_t b, int nattr, i
 constexpr uint32_t SVG_CHARS = 1024;  // characters looked at together
 constexpr uint32_t SVG_AHEAD = 64;    // and beyond, for a number that ends there
 constexpr int SVG_WAVES = 4;
+constexpr uint32_t SVG_LEFT = 0xffffffffu;  // verbs of a string left to the serial parser
 
 struct SvgText {
     uint8_t text[SVG_CHARS + SVG_AHEAD];
@@ -979,7 +980,7 @@ __global__ void __launch_bounds__(WAVE* SVG_WAVES) svg_wave_kernel(SvgLaunch L) 
                                reinterpret_cast<uint32_t*>(vals) + len, O);
     if (lane_id() != 0) return;
     if (!done) {
-        L.serial[atomicAdd(L.n_serial, 1u)] = i;
+        L.counts_v[i] = SVG_LEFT;
         return;
     }
     L.counts_v[i] = O.nv;
@@ -989,16 +990,27 @@ __global__ void __launch_bounds__(WAVE* SVG_WAVES) svg_wave_kernel(SvgLaunch L) 
         for (int k = 0; k < 4; ++k) L.errors[4ull * i + k] = 0;
 }
 
-// The serial parser, a lane per string.
+// The serial parser, a lane per string; of the strings left by the wave parser, the block's
+// first lanes take those among its 256 (a list of them all through one counter cost 45 us when
+// all of 4,096 strings were left).
 // Parses string i into its staging room: verbs at text_off[i] + 2 i (room: its bytes + 2),
 // points at 2 text_off[i] + 2 i (room: twice its bytes + 2).  Every command consumes at
 // least one character and makes at most one verb and two points per character (an arc's
 // eight quadratics need eleven), plus the End of the last sub-path; a string whose output
 // would not fit anyway raises the overflow counter instead of writing past its room.
 __global__ void __launch_bounds__(256) svg_parse_kernel(SvgLaunch L) {
+    __shared__ uint32_t left[256], n_left;
     uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (L.serial ? *L.n_serial : L.n)) return;
-    if (L.serial) i = L.serial[i];
+    if (L.by_wave) {
+        if (threadIdx.x == 0) n_left = 0;
+        __syncthreads();
+        if (i < L.n && L.counts_v[i] == SVG_LEFT) left[atomicAdd(&n_left, 1u)] = i;
+        __syncthreads();
+        if (threadIdx.x >= n_left) return;
+        i = left[threadIdx.x];
+    } else if (i >= L.n) {
+        return;
+    }
     const uint32_t a = L.text_off[i], b = L.text_off[i + 1];
     PErr E;
     Out<true> O{L.verbs + a + 2ull * i, reinterpret_cast<float2*>(L.points) + 2ull * a + 2ull * i,
@@ -1039,7 +1051,7 @@ extern "C" {
 
 hipError_t lyg_launch_svg_parse(const lyg::SvgLaunch* L, hipStream_t s) {
     if (L->n == 0) return hipSuccess;
-    if (L->serial)
+    if (L->by_wave)
         hipLaunchKernelGGL(lyg::svg_wave_kernel, dim3((L->n - 1) / lyg::SVG_WAVES + 1),
                            dim3(lyg::WAVE * lyg::SVG_WAVES), 0, s, *L);
     hipLaunchKernelGGL(lyg::svg_parse_kernel, dim3((L->n + 255) / 256), dim3(256), 0, s, *L);

@@ -57,11 +57,7 @@ int32_t lyg_parse_svg_paths(lyg_ctx* c, const uint8_t* text, const uint32_t* tex
     L.verbs = as<uint8_t>(c->st_i);
     L.points = as<float>(c->st_v);
     // the wave parser knows neither attributes nor a stop character
-    if (num_attributes == 0 && stop_at < 0) {
-        if (!ensure(c, c->st_fallback, 4ull * n)) return LYG_ERR_DEVICE;
-        L.serial = as<uint32_t>(c->st_fallback);
-        L.n_serial = c->d_counters + 7;
-    }
+    L.by_wave = num_attributes == 0 && stop_at < 0;
     if (!check(c, lyg_launch_fill_u32(c->d_counters, 8, 0, s), "reset") ||
         !check(c, lyg_launch_svg_parse(&L, s), "svg parse") ||
         !check(c, ctx_scan(c, L.counts_v, n, verb_offsets, c->d_totals, c->d_counters + 4, s), "scan") ||
