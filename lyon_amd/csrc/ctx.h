@@ -61,6 +61,8 @@ struct lyg_ctx {
     DevBuf st_items, st_heads, st_spec, st_end, st_parts, st_parts_off;
     // variable-width stroke: per-path plan, kept points, their flags and vertex sources, side
     // lines, windows, sub-path ends, candidate lists
+    bool vw_serial = false;  // tests: no parallel form
+    uint32_t last_vw_serial = 0, last_vw_recounted = 0;
     DevBuf vw_path, vw_rec, vw_flags, vw_src, vw_att, vw_win, vw_tails, vw_lists;
     // fill: one stream per size class of a round, and the events that join them
     hipStream_t class_stream[8] = {};

@@ -1353,9 +1353,19 @@ __global__ void __launch_bounds__(256) vw_window_kernel(VWPar P, uint32_t list, 
     }
 }
 
-// Thread per candidate of the count pass: settles which joins fold back.  A skip only
-// changes what the next points see before them, so the first candidate of a group (none in
-// the 8 points before it) walks on until 8 joins in a row are not skipped.
+// A candidate that is the first of its group: none in the 8 points before it on its curve.
+__device__ __forceinline__ bool skip_leader(const uint8_t* fl, uint32_t i) {
+    for (uint32_t b = 1; b <= 8u && b <= i && (fl[i - b] & vw::PF_FLAT); ++b)
+        if (fl[i - b] & vw::PF_CAND) return false;
+    return true;
+}
+
+// Thread per candidate of the count pass: settles which joins fold back.  A skip only changes
+// what the next points see before them, and nothing beyond the curve's end, which is never
+// skipped (whether a join after it folds back depends on points from there on).  So the first
+// candidate of a group walks on along its curve until 8 joins in a row are neither skipped nor
+// candidates.  Skips that the count could not see may bring it to the next group, whose own
+// thread has then read flags from before them: the path is left to the serial kernel.
 __global__ void __launch_bounds__(64) vw_skip_kernel(VWPar P) {
     using namespace vw;
     const uint32_t n = min(P.ctr[2], P.cand_cap);
@@ -1364,30 +1374,26 @@ __global__ void __launch_bounds__(64) vw_skip_kernel(VWPar P) {
         if (P.path_mode[path] != 0u) continue;
         const PC c = path_ctx(P, path);
         uint8_t* fl = P.pflags + P.raw_off[path];
-        bool leader = true;
-        for (uint32_t b = 1; b <= 8u && b <= i; ++b) {
-            const uint32_t f = fl[i - b];
-            if (f & PF_CAND) leader = false;
-            if (f & PF_FIRST) break;
-        }
-        if (!leader) continue;
-        uint32_t clean = 0;
-        for (uint32_t x = i; clean < 8u && x + 1u < c.kn && !(fl[x + 1u] & PF_FIRST); ++x) {
+        if (!skip_leader(fl, i)) continue;
+        uint32_t clean = 0, x = i;
+        for (; clean < 8u && x + 1u < c.kn && (fl[x] & PF_FLAT) && !(fl[x + 1u] & PF_FIRST); ++x) {
+            const bool cand = (fl[x] & PF_CAND) != 0;
+            if (cand && x != i && skip_leader(fl, x)) {
+                mark_slow(P, path);
+                break;
+            }
             JInfo J;
             uint32_t q;
             bool pfirst;
             join_at(c, x, att_ord(c, x), J, q, pfirst);
-            if (q + 1u != x && (fl[x] & PF_FLAT) && (fl[x + 1u] & PF_FLAT)) {
+            if (q + 1u != x && (fl[x + 1u] & PF_FLAT)) {
                 // the running lengths were written as if the point before had stayed
                 const vec2 a = pos_of(c.rec[x - 1u]), j = pos_of(c.rec[x]);
                 const bool naive = dot(sub(j, a), sub(pos_of(c.rec[x + 1u]), j)) > 0.0f;
                 if (naive != J.fast) mark_slow(P, path);
             }
-            if (!J.weird) {
-                ++clean;
-                continue;
-            }
-            clean = 0;
+            clean = cand || J.weird ? 0u : clean + 1u;
+            if (!J.weird) continue;
             fl[x] = (uint8_t)(fl[x] | PF_SKIP);
             for (uint32_t y = x; y <= x + 2u && y < c.kn; ++y) {
                 if (y != x && y / WIN == (y - 1u) / WIN) continue;

@@ -164,7 +164,7 @@ int32_t stroke_vw_run(lyg_ctx* c, lyg::StrokeVWLaunch& L, bool want_attrs, uint3
     L.err = c->d_counters + 5;
     lyg::VWPar P{};
     VWShape sh{};
-    int32_t st = vw_plan(c, L, n, want_attrs, &P, &sh);
+    int32_t st = c->vw_serial ? (int32_t)LYG_ERR_NO_SPACE : vw_plan(c, L, n, want_attrs, &P, &sh);
     if (st == LYG_OK) st = vw_count(c, P, sh);
     if (st == LYG_ERR_DEVICE) return st;
     bool par = st == LYG_OK;
@@ -182,7 +182,8 @@ int32_t stroke_vw_run(lyg_ctx* c, lyg::StrokeVWLaunch& L, bool want_attrs, uint3
         grid = par ? (int)std::min(n, slots)
                    : (int)std::min<uint32_t>((n + L.paths_per_wave - 1) / L.paths_per_wave,
                                              1u << 20);
-        h[3] = 0;
+        h[3] = h[4] = 0;  // serial paths, candidates, windows counted again, a list overflowed
+        uint32_t* went = reinterpret_cast<uint32_t*>(h + 3);
         if (!check(c, lyg_launch_fill_u32(c->d_counters + 4, 2, 0, s), "reset") ||
             !check(c, lyg_launch_stroke_vw(&L, 0, grid, s), "stroke vw count") ||
             !check(c, ctx_scan(c, L.path_nv, n, vtx_off, c->d_totals + 0, c->d_counters + 4, s),
@@ -192,14 +193,16 @@ int32_t stroke_vw_run(lyg_ctx* c, lyg::StrokeVWLaunch& L, bool want_attrs, uint3
             !check(c, hipMemcpyAsync(h, c->d_totals, 16, hipMemcpyDeviceToHost, s), "D2H") ||
             !check(c, hipMemcpyAsync(h + 2, c->d_counters + 4, 4, hipMemcpyDeviceToHost, s),
                    "D2H") ||
-            (par && !check(c, hipMemcpyAsync(h + 3, P.ctr + 4, 4, hipMemcpyDeviceToHost, s),
+            (par && !check(c, hipMemcpyAsync(went, P.ctr + 1, 16, hipMemcpyDeviceToHost, s),
                            "D2H")) ||
             !check(c, hipMemcpyAsync(status->data(), L.path_status, 4ull * n,
                                      hipMemcpyDeviceToHost, s),
                    "D2H") ||
             !check(c, hipStreamSynchronize(s), "sync"))
             return LYG_ERR_DEVICE;
-        if (!(uint32_t)h[3]) break;
+        c->last_vw_serial = par && !went[3] ? went[0] : n;
+        c->last_vw_recounted = went[2];
+        if (!went[3]) break;
         par = false;  // more joins that may fold back than the lists hold
     }
     *tv = h[0];
@@ -245,6 +248,14 @@ int32_t first_failure(const std::vector<uint32_t>& st) {
 }  // namespace
 
 extern "C" {
+
+// Not in lyg.h: sends every path to the serial kernel (the two forms give the same bytes); how
+// the last call went: paths walked by it, and windows counted again for joins that fold back.
+void lyg_ctx_set_vw_serial(lyg_ctx* c, int enabled) { c->vw_serial = enabled != 0; }
+void lyg_ctx_last_vw(const lyg_ctx* c, uint32_t* serial, uint32_t* recounted) {
+    *serial = c->last_vw_serial;
+    *recounted = c->last_vw_recounted;
+}
 
 // StrokeTessellator::tessellate_path with StrokeOptions::variable_line_width
 // (stroke.rs:653-767) for a batch in device memory.

@@ -278,3 +278,113 @@ def test_vertex_attributes_match_the_oracle():
         same_rows += np.array_equal(ga.view(np.uint32), ra.view(np.uint32))
     print(f"{matched} paths matched, {same_rows} with the same attribute rows", flush=True)
     assert matched >= 0.97 * n and same_rows >= 0.97 * matched
+
+
+def forms(paths, opts, attrs=None):
+    """The batch by the parallel form and by the serial kernel (one lane per path): equal
+    offsets, statuses, and bytes of vertices, indices and vertex attributes.  Returns the paths
+    that the first run left to the serial kernel and the windows it counted again."""
+    import ctypes as C
+
+    from lyon_amd import _lib
+    from lyon_amd.batch import _Ctx
+    from lyon_amd.path import PathBatch
+    lib = C.CDLL(_lib.LIB_PATH)
+    ctx = C.c_void_p(_Ctx.get())
+    batch = paths if isinstance(paths, PathBatch) else PathBatch.from_paths(paths)
+    if attrs is None:
+        attrs = np.concatenate([p.attributes for p in paths])
+    db = DeviceBatch(batch, opts)
+    outs, serial, again = [], C.c_uint32(0), C.c_uint32(0)
+    for enabled in (0, 1):
+        b = StrokeVWBatcher(attrs, vertex_attributes=True)
+        lib.lyg_ctx_set_vw_serial(ctx, enabled)
+        try:
+            res = b.run(db, vertex_offset=5)
+        finally:
+            lib.lyg_ctx_set_vw_serial(ctx, 0)
+        if not enabled:
+            lib.lyg_ctx_last_vw(ctx, C.byref(serial), C.byref(again))
+        synchronize()
+        rows = b.vertex_attributes.download(np.uint32, b.n_attributes * res.n_vertices)
+        outs.append((res.status.copy(), res.vertex_offsets.copy(), res.index_offsets.copy(),
+                     res.all_vertices().view(np.uint32).copy(), res.all_indices().copy(), rows))
+    for a, b, what in zip(*outs, ("statuses", "vertex offsets", "index offsets", "vertices",
+                                  "indices", "vertex attributes")):
+        assert a.shape == b.shape, what
+        if not np.array_equal(a, b):
+            at = int(np.nonzero((a != b).reshape(len(a), -1).any(1))[0][0])
+            raise AssertionError((what, at))
+    assert not outs[0][0].any()
+    return serial.value, again.value
+
+
+def vw_options(n, rng, width, tol):
+    o = workloads.stroke_options(n, tolerance=tol, seed=int(rng.integers(1 << 30)))
+    o["line_width"] = width
+    o["line_join"] = rng.choice([0, 2, 3], n)  # no MiterClip: those paths are always serial
+    o["start_cap"] = o["end_cap"] = rng.integers(0, 3, n)
+    return o
+
+
+@pytest.mark.parametrize("seed", [5, 6])
+def test_the_two_forms_agree(seed):
+    n = 400
+    batch, opts, widths = random_batch(n, seed)
+    attrs = np.stack([widths, np.arange(len(widths), dtype=np.float32)], axis=1)
+    serial, _ = forms(batch, opts, attrs)
+    assert serial < n
+
+
+@pytest.mark.parametrize("closed", [False, True])
+def test_many_skipped_joins_in_a_row(closed):
+    """Curves of a few to hundreds of points whose first joins are skipped, one or dozens in a
+    row, across window borders and up to the curve's end."""
+    rng = np.random.default_rng(60 + closed)
+    paths = []
+    for lead in list(range(67)) * 3:
+        b = PathBuilder(1)
+        at = np.zeros(2)
+        b.begin(tuple(at), [1.0])
+        for _ in range(lead):
+            at = at + rng.uniform((1, -3), (4, 3))
+            b.line_to(tuple(at), [rng.uniform(0.5, 1)])
+        for _ in range(int(rng.integers(1, 5))):
+            size = 10 ** rng.uniform(0.3, 2)
+            at = at + rng.uniform(2, 30, 2)
+            b.line_to(tuple(at), [rng.uniform(0.5, 2) * size])
+            q = [tuple(at + rng.uniform(-size, size, 2)) for _ in range(2)]
+            at = at + rng.uniform(-size, size, 2)
+            if rng.random() < 0.3:
+                b.quadratic_bezier_to(q[0], tuple(at), [rng.uniform(0.01, 2)])
+            else:
+                b.cubic_bezier_to(*q, tuple(at), [rng.uniform(0.01, 2)])
+            for _ in range(int(rng.integers(0, 3))):
+                at = at + rng.uniform(-3, 3, 2)
+                b.line_to(tuple(at), [rng.uniform(0.2, 2)])
+        b.end(closed)
+        paths.append(b.build())
+    serial, again = forms(paths, vw_options(len(paths), rng, 2.0, 0.02))
+    print(f"{serial} of {len(paths)} paths serial, {again} windows counted again", flush=True)
+    assert again > len(paths) and serial < len(paths) // 2
+
+
+def test_skips_where_rounding_makes_them():
+    """Far from the origin the points of a curve lie on a coarse grid and any of its joins may
+    seem to fold back, in groups close together: whichever thread settles them, the bytes are
+    the serial kernel's."""
+    rng = np.random.default_rng(50)
+    paths = []
+    for k in range(300):
+        far = 10 ** rng.uniform(4, 6.5)
+        b = PathBuilder(1)
+        b.begin((far, far), [rng.uniform(1, 50)])
+        for _ in range(6):
+            q = [tuple(far + rng.uniform(0, 40, 2)) for _ in range(3)]
+            b.cubic_bezier_to(*q, [rng.uniform(0.1, 50)])
+        b.end(k % 2 == 0)
+        paths.append(b.build())
+    for tol in (0.1, 1e-3):
+        serial, again = forms(paths, vw_options(len(paths), rng, 2.0, tol))
+        print(f"{serial} of {len(paths)} paths serial, {again} windows again", flush=True)
+        assert again > 0
