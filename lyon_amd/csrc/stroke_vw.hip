@@ -1227,7 +1227,11 @@ __global__ void __launch_bounds__(256) vw_window_kernel(VWPar P, uint32_t list, 
         uint32_t path = 0, wend = 0;  // the path of the windows before `wend`
         bool run = false;
         PC c;
-        for (uint32_t k = c0; k < min(n_win, c0 + chunk); ++k) {
+        const uint32_t c1 = min(n_win, c0 + chunk);
+        // EMIT: where the next window has to start, and whether one did not
+        uint32_t next_v = EMIT ? P.win_voff[c0] : 0u, next_t = EMIT ? P.win_ioff[c0] : 0u;
+        uint32_t differ = 0;
+        for (uint32_t k = c0; k < c1; ++k) {
             const uint32_t w = list ? P.dirty[k] : k;
             if (w >= wend || list) {
                 path = wave_search_last_le(P.win_off, P.in.n_paths + 1u, w);
@@ -1239,6 +1243,10 @@ __global__ void __launch_bounds__(256) vw_window_kernel(VWPar P, uint32_t list, 
             const uint32_t start = (w - wb) * WIN;
             if (!run || start >= c.kn) {
                 if (!EMIT && l == 0) P.win_nv[w] = P.win_ni[w] = 0u;
+                if (EMIT && !run) {  // a path left to the serial kernel after it was counted
+                    next_v = P.win_voff[w + 1u];
+                    next_t = P.win_ioff[w + 1u];
+                }
                 continue;
             }
             uint32_t i = start + (uint32_t)l - 1u, back = 0;
@@ -1300,9 +1308,14 @@ __global__ void __launch_bounds__(256) vw_window_kernel(VWPar P, uint32_t list, 
                 nv = l > 0 ? tail->nv : 0u;
                 nt = l > 0 ? tail->nt : 0u;
             }
-            const uint32_t v_at = P.win_voff[w] - P.win_voff[wb];
-            const uint32_t t_at = P.win_ioff[w] - P.win_ioff[wb];
-            const uint32_t vx = incl_scan(nv) - nv, tx = incl_scan(nt) - nt;
+            const uint32_t w_v = P.win_voff[w], w_t = P.win_ioff[w];
+            const uint32_t v_at = w_v - P.win_voff[wb];
+            const uint32_t t_at = w_t - P.win_ioff[wb];
+            differ |= (w_v ^ next_v) | (w_t ^ next_t);
+            const uint32_t vi = incl_scan(nv), ti = incl_scan(nt);
+            const uint32_t vx = vi - nv, tx = ti - nt;
+            next_v = w_v + readlane_u(vi, WAVE - 1);
+            next_t = w_t + readlane_u(ti, WAVE - 1);
             const uint32_t my_v = l == 0 ? v_at - nv0 : v_at + vx;
             const uint32_t pv = shfl_u(my_v, lq < 0 ? 0 : lq);
             const uint32_t v0 = P.vtx_off[path], id_base = P.vertex_offset + v0;
@@ -1350,6 +1363,9 @@ __global__ void __launch_bounds__(256) vw_window_kernel(VWPar P, uint32_t list, 
                 }
             }
         }
+        // the count saw other joins than these
+        if (EMIT && (differ | (P.win_voff[c1] ^ next_v) | (P.win_ioff[c1] ^ next_t)) != 0u && l == 0)
+            atomicOr(P.err, 4u);
     }
 }
 
@@ -1366,6 +1382,10 @@ __device__ __forceinline__ bool skip_leader(const uint8_t* fl, uint32_t i) {
 // candidate of a group walks on along its curve until 8 joins in a row are neither skipped nor
 // candidates.  Skips that the count could not see may bring it to the next group, whose own
 // thread has then read flags from before them: the path is left to the serial kernel.
+//
+// A skip changes the counts of up to four buffered points after it, and past the curve's end
+// those of the end's join and of the point after that: all windows of the walk are counted
+// again, and that of the two points after a walk to the end.
 __global__ void __launch_bounds__(64) vw_skip_kernel(VWPar P) {
     using namespace vw;
     const uint32_t n = min(P.ctr[2], P.cand_cap);
@@ -1393,14 +1413,13 @@ __global__ void __launch_bounds__(64) vw_skip_kernel(VWPar P) {
                 if (naive != J.fast) mark_slow(P, path);
             }
             clean = cand || J.weird ? 0u : clean + 1u;
-            if (!J.weird) continue;
-            fl[x] = (uint8_t)(fl[x] | PF_SKIP);
-            for (uint32_t y = x; y <= x + 2u && y < c.kn; ++y) {
-                if (y != x && y / WIN == (y - 1u) / WIN) continue;
-                const uint32_t s = atomicAdd(&P.ctr[3], 1u);
-                if (s < P.dirty_cap) P.dirty[s] = P.win_off[path] + y / WIN;
-                else atomicOr(&P.ctr[4], 1u);
-            }
+            if (J.weird) fl[x] = (uint8_t)(fl[x] | PF_SKIP);
+        }
+        const uint32_t last = min(x + 2u, c.kn - 1u);
+        for (uint32_t w = i / WIN; w <= last / WIN; ++w) {
+            const uint32_t s = atomicAdd(&P.ctr[3], 1u);
+            if (s < P.dirty_cap) P.dirty[s] = P.win_off[path] + w;
+            else atomicOr(&P.ctr[4], 1u);
         }
     }
 }

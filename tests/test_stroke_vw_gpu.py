@@ -336,6 +336,55 @@ def test_the_two_forms_agree(seed):
     assert serial < n
 
 
+def turns(rng, at, heading, lengths, most):
+    """Points one after the other from `at`, each at a turn of up to `most`; the last heading."""
+    out = []
+    for length in lengths:
+        heading += rng.uniform(-most, most)
+        at = at + length * np.array([np.cos(heading), np.sin(heading)])
+        out.append(at)
+    return out, heading
+
+
+@pytest.mark.parametrize("lead", [0, 1, 55, 56, 57, 58, 59, 60, 61, 62])
+def test_skipped_joins_around_the_window_size(lead):
+    """Where a curve's width falls faster than it advances, its first join folds back and is
+    skipped, and what up to four points after it emit may change with it, past the curve's end
+    too: of these random curves of three points, about 1 in 300 changes the triangles of the edge
+    after it.  Behind `lead` points of lines, so that the skip and what it reaches lie on both
+    sides of the 63rd join."""
+    rng = np.random.default_rng(40 + lead)
+    paths, tol = [], []
+    for _ in range(2500):
+        b = PathBuilder(1)
+        b.begin((0.0, 0.0), [1.0])
+        at, heading = np.zeros(2), 0.0
+        for _ in range(lead):
+            at = at + rng.uniform((1, -2), (3, 2))
+            b.line_to(tuple(at), [rng.uniform(0.5, 1)])
+        at = at + rng.uniform((5, -9), (20, 9))
+        steps = 10 ** rng.uniform(-0.5, 0.5, 3)
+        (x, y, e), heading = turns(rng, at, rng.uniform(-np.pi, np.pi), steps, 1.2)
+        w = 10 ** rng.uniform(-0.3, 1.3)
+        b.line_to(tuple(at), [w])
+        c1 = (-5 * at + 18 * x - 9 * y + 2 * e) / 6  # through x and y at t = 1/3 and 2/3
+        c2 = (2 * at - 9 * x + 18 * y - 5 * e) / 6
+        w = max(0.05, w - 3 * steps[0] * rng.uniform(0.3, 1))
+        b.cubic_bezier_to(tuple(c1), tuple(c2), tuple(e), [w])
+        for q in turns(rng, e, heading, 10 ** rng.uniform(-0.7, 1, 4), np.pi)[0]:
+            b.line_to(tuple(q), [w * rng.uniform(0.2, 2)])
+        b.end(False)
+        paths.append(b.build())
+        second = max(np.hypot(*(at - 2 * c1 + c2)), np.hypot(*(c1 - 2 * c2 + e)))
+        tol.append(6 * second / (8 * 6.25))  # Wang: n = sqrt(6 second / (8 tol)) = 2.5, so 3
+    opts = vw_options(len(paths), rng, 2.0, 0.1)
+    opts["tolerance"] = tol
+    opts["line_join"][::2] = int(LineJoin.Miter)
+    serial, again = forms(paths, opts)
+    print(f"{serial} of {len(paths)} paths serial, {again} windows counted again", flush=True)
+    assert again > len(paths) // 10 and serial < len(paths) // 10
+
+
 @pytest.mark.parametrize("closed", [False, True])
 def test_many_skipped_joins_in_a_row(closed):
     """Curves of a few to hundreds of points whose first joins are skipped, one or dozens in a
