@@ -90,7 +90,9 @@ int32_t vw_plan(lyg_ctx* c, const lyg::StrokeVWLaunch& L, uint32_t n, bool want_
         return LYG_ERR_NO_SPACE;
     P.n_windows = (uint32_t)win;
     P.n_tails = (uint32_t)tails;
-    P.cand_cap = (uint32_t)std::max<uint64_t>(4096, win);
+    // candidates for skipped joins: but for rounding, each is a curve's first point, and a curve
+    // has an edge with side lines at both ends
+    P.cand_cap = (uint32_t)std::max<uint64_t>({4096, win, att / 2});
     P.dirty_cap = 4u * P.cand_cap;
     const bool src = want_attrs;
     if (!ensure(c, c->vw_rec, 16 * raw) || !ensure(c, c->vw_flags, raw) ||

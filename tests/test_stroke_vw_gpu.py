@@ -418,6 +418,25 @@ def test_many_skipped_joins_in_a_row(closed):
     assert again > len(paths) and serial < len(paths) // 2
 
 
+def test_more_skipped_joins_than_windows():
+    """Short paths whose every curve starts with a skipped join: more of them than windows, and
+    none of the paths is left to the serial kernel."""
+    rng = np.random.default_rng(70)
+    paths = []
+    for _ in range(2000):
+        b = PathBuilder(1)
+        at = rng.uniform(0, 100, 2)
+        b.begin(tuple(at), [8.0])
+        for _ in range(6):
+            b.cubic_bezier_to(*[tuple(at + (3.0 * k, 0.4 * (k % 3))) for k in (1, 2, 3)], [2.0])
+            at = at + (9.0, 3.0)
+            b.line_to(tuple(at), [8.0])
+        b.end(False)
+        paths.append(b.build())
+    serial, again = forms(paths, vw_options(len(paths), rng, 2.0, 0.02))
+    assert serial == 0 and again >= len(paths)
+
+
 def test_skips_where_rounding_makes_them():
     """Far from the origin the points of a curve lie on a coarse grid and any of its joins may
     seem to fold back, in groups close together: whichever thread settles them, the bytes are
