@@ -52,7 +52,10 @@ int32_t vw_plan(lyg_ctx* c, const lyg::StrokeVWLaunch& L, uint32_t n, bool want_
     P.path_nv = L.path_nv;
     P.path_ni = L.path_ni;
     P.err = L.err;
-    if (!ensure(c, c->vw_path, 4ull * (11ull * n + 4) + 64)) return LYG_ERR_DEVICE;
+    if (!ensure(c, c->vw_path, 4ull * (11ull * n + 4) + 64)) {
+        (void)hipGetLastError();
+        return LYG_ERR_NO_SPACE;
+    }
     uint32_t* u = as<uint32_t>(c->vw_path);
     auto take = [&](size_t k) {
         uint32_t* p = u;

@@ -319,6 +319,47 @@ def forms(paths, opts, attrs=None):
     return serial.value, again.value
 
 
+@pytest.mark.parametrize("limit", [0, 2 << 20, 5 << 20])
+def test_without_memory_for_the_parallel_form(limit):
+    """Where one of the parallel form's buffers cannot be allocated (4.4 MB per-path counts, 6.4
+    MB of points) the serial kernel takes the batch."""
+    import ctypes as C
+    import threading
+
+    from lyon_amd import _lib
+    from lyon_amd.batch import _Ctx
+    from lyon_amd.path import PathBatch
+    n = 100000
+    rng = np.random.default_rng(3)
+    pts = rng.uniform(0, 50, (4 * n, 2)).astype(np.float32)
+    batch = PathBatch(np.tile(np.array([3, 0, 0, 0, 5], np.uint8), n), pts,
+                      np.arange(n + 1, dtype=np.uint32) * 5, np.arange(n + 1, dtype=np.uint32) * 4)
+    widths = rng.uniform(0.5, 1.5, 4 * n).astype(np.float32)
+    opts = vw_options(n, rng, 1.0, 0.1)
+    opts["line_join"] = int(LineJoin.Miter)
+    db = DeviceBatch(batch, opts)
+    ref = StrokeVWBatcher(widths).run(db)
+    want = ref.all_vertices().view(np.uint32).copy(), ref.all_indices().copy()
+    lib = C.CDLL(_lib.LIB_PATH)
+    lib.lyg_ctx_set_alloc_limit.argtypes = [C.c_void_p, C.c_uint64]
+    lib.lyg_ctx_set_alloc_limit.restype = None
+    got = []
+
+    def fresh():  # a context of its own
+        lib.lyg_ctx_set_alloc_limit(_Ctx.get(), limit)
+        r = StrokeVWBatcher(widths).run(db)
+        n_serial, again = C.c_uint32(0), C.c_uint32(0)
+        lib.lyg_ctx_last_vw(C.c_void_p(_Ctx.get()), C.byref(n_serial), C.byref(again))
+        got.append((n_serial.value, r.all_vertices().view(np.uint32).copy(),
+                    r.all_indices().copy()))
+
+    t = threading.Thread(target=fresh)
+    t.start()
+    t.join()
+    assert got and got[0][0] == (n if limit else 0)
+    assert np.array_equal(got[0][1], want[0]) and np.array_equal(got[0][2], want[1])
+
+
 def vw_options(n, rng, width, tol):
     o = workloads.stroke_options(n, tolerance=tol, seed=int(rng.integers(1 << 30)))
     o["line_width"] = width
