@@ -198,6 +198,10 @@ def test_sub_paths_around_the_window_size(join, closed):
         rv, ri = ref_vw(path, opts)
         same += np.array_equal(i, ri) and close_enough(v, rv, 300.0)
     assert same >= 0.97 * len(paths), same
+    o = vw_options(len(paths), rng, 2.0, 0.05)
+    o["line_join"] = int(join)
+    serial, _ = forms(paths, o)
+    assert serial == len(paths) if join == LineJoin.MiterClip else serial < len(paths) // 4
 
 
 @pytest.mark.parametrize("counts", [[1, 2, 15, 16, 17, 18], [31, 33, 63, 65, 80], [4000, 90, 70],
