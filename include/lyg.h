@@ -414,9 +414,10 @@ int32_t lyg_ctx_set_stroke_split(lyg_ctx* ctx, uint32_t windows_per_part);
  * give the same output.  enabled > 1 divides the first form's capacities by that factor, so
  * that paths outgrow them and take the fallback (for tests). */
 int32_t lyg_ctx_set_fill_lds_resident(lyg_ctx* ctx, int enabled);
-/* Of the last split batched stroke on this context: the items walked (whole paths and
- * parts) and the paths walked again whole because a part's prologue did not rebuild the
- * state or a part outgrew its room (no lyon counterpart). */
+/* Of the last stroke on this context that was cut into parts (a batch, or a plain call on a
+ * path of 512 points or more): the items walked (whole paths and parts) and the paths walked
+ * again whole because a part's prologue did not rebuild the state or a part outgrew its room
+ * (no lyon counterpart). */
 int32_t lyg_ctx_stroke_split_stats(lyg_ctx* ctx, uint64_t* items, uint32_t* walked_again);
 int32_t lyg_autotune_stroke(lyg_ctx* ctx, const lyg_batch_in* in, const lyg_stroke_options* opts,
                             uint32_t n_opts, lyg_batch_out* out, lyg_tuning* chosen);

@@ -310,7 +310,7 @@ struct ValidateLaunch {
     float* areas;
 };
 
-// SVG path data parse (svg.hip): one lane per string.
+// SVG path data parse (svg.hip): a wave per string, or a lane.
 struct SvgLaunch {
     const uint8_t* text;
     const uint32_t* text_off;  // n + 1

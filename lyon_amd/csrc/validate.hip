@@ -9,8 +9,8 @@
 //     the flattened points of each, counting the crossings left of the query; the count is
 //     an integer, so the sum is exact in any order.
 //   * approximate signed areas (approximate_signed_area, crates/algorithms/src/area.rs:7-54):
-//     lyon's serial f32 sum of cross products in event order; one wave per path computes the
-//     terms 64 at a time and adds them in order.
+//     lyon's serial f32 sum of cross products in event order; one wave per path computes up to
+//     1,024 terms at once and adds them in order, the running value going from lane to lane.
 //
 // Paths are as lyon's builders make them: every sub-path opens with Begin, so the current
 // point of a verb is the last point consumed before it (path.rs:843-909).  Curves are

@@ -159,10 +159,10 @@ def test_batch_matches_plain_calls():
 
 
 def test_lds_resident_form_and_fallback():
-    """The batched fill gives the same bytes whether its first round keeps each path's hot
-    arrays in LDS (the default), starts them in LDS and moves them to global memory as
-    they grow, or keeps them in LDS at an eighth of the estimated capacities (so that many
-    paths outgrow them and are swept again in the global form); paths of every size of the
+    """The batched fill gives the same bytes whether its first round keeps each path's active
+    edges in registers (the default), sweeps over arrays that start in LDS and move to global
+    memory as they grow, or keeps them in registers at an eighth of the estimated capacities (so
+    that many paths outgrow them and are swept again over arrays); paths of every size of the
     fill workload, the 513-point stars included."""
     from lyon_amd.batch import DeviceBatch, FillBatcher, set_fill_lds_resident, synchronize
     n = 512
@@ -188,10 +188,10 @@ def test_lds_resident_form_and_fallback():
 
 
 def test_many_launches_in_one_round():
-    """Paths in many size classes and placement forms (fill-workload stars and cubic loops,
-    closed random walks of 2,000 to 60,000 vertices) give a round more launches than there
-    used to be work counters: every path is swept (status 0) and the bytes equal those of
-    the migrating form, launched the old way."""
+    """Paths in many size classes and forms (fill-workload stars and cubic loops, closed random
+    walks of 2,000 to 60,000 vertices) give a round about ten launches (a host-side test plans
+    all 32): every path is swept (status 0) and the bytes equal those of the sweep over
+    arrays."""
     from lyon_amd.batch import DeviceBatch, FillBatcher, set_fill_lds_resident, synchronize
     from lyon_amd.path import PathBatch
     base = workloads.fill_batch(1024, seed=2)
