@@ -704,6 +704,10 @@ __device__ void parse_svg(const uint8_t* s, uint32_t a, uint32_t b, int nattr, i
 constexpr uint32_t SVG_CHARS = 1024;  // characters looked at together
 constexpr uint32_t SVG_AHEAD = 64;    // and beyond, for a number that ends there
 constexpr int SVG_WAVES = 4;
+// Up to here a string that its wave leaves is parsed by a lane of that wave, one launch less;
+// beyond, many of them fill lanes better in a launch of their own.  us a call of 1 / 64 / 1,024
+// / 4,096 strings with an arc: 329 375 546 1,127 by their waves, 369 384 560 1,050 in a launch.
+constexpr uint32_t SVG_FEW = 1024;
 constexpr uint32_t SVG_LEFT = 0xffffffffu;  // verbs of a string left to the serial parser
 
 struct SvgText {
@@ -964,53 +968,12 @@ __device__ bool wave_svg(const uint8_t* s, uint32_t len, SvgText& T, float* vals
 
 }  // namespace
 
-// A wave per string; the staging rooms as svg_parse_kernel's.  The upper half of a string's
-// points room (twice as many as its characters; a point takes at least one) holds its numbers
-// and command words meanwhile.
-__global__ void __launch_bounds__(WAVE* SVG_WAVES) svg_wave_kernel(SvgLaunch L) {
-    __shared__ SvgText texts[SVG_WAVES];
-    const uint32_t w = readlane_u(threadIdx.x / WAVE, 0);
-    const uint32_t i = blockIdx.x * SVG_WAVES + w;
-    if (i >= L.n) return;
-    const uint32_t a = L.text_off[i], len = L.text_off[i + 1] - a;
-    float2* pts = reinterpret_cast<float2*>(L.points) + 2ull * a + 2ull * i;
-    float* vals = reinterpret_cast<float*>(pts + len + 2u);
-    Out<true> O{L.verbs + a + 2ull * i, pts, 0, 0, mk(0.0f, 0.0f), len + 2, 2 * len + 2};
-    const bool done = wave_svg(L.text + a, len, texts[w], vals,
-                               reinterpret_cast<uint32_t*>(vals) + len, O);
-    if (lane_id() != 0) return;
-    if (!done) {
-        L.counts_v[i] = SVG_LEFT;
-        return;
-    }
-    L.counts_v[i] = O.nv;
-    L.counts_p[i] = O.np;
-    if (O.nv > O.cap_v || O.np > len + 2u) atomicAdd(L.n_errors + 1, 1u);
-    if (L.errors)
-        for (int k = 0; k < 4; ++k) L.errors[4ull * i + k] = 0;
-}
-
-// The serial parser, a lane per string; of the strings left by the wave parser, the block's
-// first lanes take those among its 256 (a list of them all through one counter cost 45 us when
-// all of 4,096 strings were left).
 // Parses string i into its staging room: verbs at text_off[i] + 2 i (room: its bytes + 2),
 // points at 2 text_off[i] + 2 i (room: twice its bytes + 2).  Every command consumes at
 // least one character and makes at most one verb and two points per character (an arc's
 // eight quadratics need eleven), plus the End of the last sub-path; a string whose output
 // would not fit anyway raises the overflow counter instead of writing past its room.
-__global__ void __launch_bounds__(256) svg_parse_kernel(SvgLaunch L) {
-    __shared__ uint32_t left[256], n_left;
-    uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (L.by_wave) {
-        if (threadIdx.x == 0) n_left = 0;
-        __syncthreads();
-        if (i < L.n && L.counts_v[i] == SVG_LEFT) left[atomicAdd(&n_left, 1u)] = i;
-        __syncthreads();
-        if (threadIdx.x >= n_left) return;
-        i = left[threadIdx.x];
-    } else if (i >= L.n) {
-        return;
-    }
+__device__ __forceinline__ void serial_string(const SvgLaunch& L, uint32_t i) {
     const uint32_t a = L.text_off[i], b = L.text_off[i + 1];
     PErr E;
     Out<true> O{L.verbs + a + 2ull * i, reinterpret_cast<float2*>(L.points) + 2ull * a + 2ull * i,
@@ -1027,6 +990,56 @@ __global__ void __launch_bounds__(256) svg_parse_kernel(SvgLaunch L) {
         e[3] = (int32_t)E.ch;
     }
     if (E.kind != LYG_SVG_OK) atomicAdd(L.n_errors, 1u);
+}
+
+// A wave per string; the staging rooms as serial_string's.  The upper half of a string's
+// points room (twice as many as its characters; a point takes at least one) holds its numbers
+// and command words meanwhile.  SERIAL: a lane of the wave goes through a string that the wave
+// leaves, else svg_parse_kernel does.
+template <bool SERIAL>
+__global__ void __launch_bounds__(WAVE* SVG_WAVES) svg_wave_kernel(SvgLaunch L) {
+    __shared__ SvgText texts[SVG_WAVES];
+    const uint32_t w = readlane_u(threadIdx.x / WAVE, 0);
+    const uint32_t i = blockIdx.x * SVG_WAVES + w;
+    if (i >= L.n) return;
+    const uint32_t a = L.text_off[i], len = L.text_off[i + 1] - a;
+    float2* pts = reinterpret_cast<float2*>(L.points) + 2ull * a + 2ull * i;
+    float* vals = reinterpret_cast<float*>(pts + len + 2u);
+    Out<true> O{L.verbs + a + 2ull * i, pts, 0, 0, mk(0.0f, 0.0f), len + 2, 2 * len + 2};
+    const bool done = wave_svg(L.text + a, len, texts[w], vals,
+                               reinterpret_cast<uint32_t*>(vals) + len, O);
+    // what the wave wrote of a string it leaves comes before what the lane writes there
+    if (SERIAL && !done) __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
+    if (lane_id() != 0) return;
+    if (!done) {
+        if (SERIAL) serial_string(L, i);
+        else L.counts_v[i] = SVG_LEFT;
+        return;
+    }
+    L.counts_v[i] = O.nv;
+    L.counts_p[i] = O.np;
+    if (O.nv > O.cap_v || O.np > len + 2u) atomicAdd(L.n_errors + 1, 1u);
+    if (L.errors)
+        for (int k = 0; k < 4; ++k) L.errors[4ull * i + k] = 0;
+}
+
+// The serial parser, a lane per string; of the strings left by the wave parser, the block's
+// first lanes take those among its 256 (a list of them all through one counter cost 45 us when
+// all of 4,096 strings were left).
+__global__ void __launch_bounds__(256) svg_parse_kernel(SvgLaunch L) {
+    __shared__ uint32_t left[256], n_left;
+    uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (L.by_wave) {
+        if (threadIdx.x == 0) n_left = 0;
+        __syncthreads();
+        if (i < L.n && L.counts_v[i] == SVG_LEFT) left[atomicAdd(&n_left, 1u)] = i;
+        __syncthreads();
+        if (threadIdx.x >= n_left) return;
+        i = left[threadIdx.x];
+    } else if (i >= L.n) {
+        return;
+    }
+    serial_string(L, i);
 }
 
 // Copies every string's verbs and points from its staging room to its place in the batch:
@@ -1050,11 +1063,17 @@ __global__ void __launch_bounds__(256) svg_compact_kernel(SvgLaunch L, uint8_t* 
 extern "C" {
 
 hipError_t lyg_launch_svg_parse(const lyg::SvgLaunch* L, hipStream_t s) {
+    using namespace lyg;
     if (L->n == 0) return hipSuccess;
-    if (L->by_wave)
-        hipLaunchKernelGGL(lyg::svg_wave_kernel, dim3((L->n - 1) / lyg::SVG_WAVES + 1),
-                           dim3(lyg::WAVE * lyg::SVG_WAVES), 0, s, *L);
-    hipLaunchKernelGGL(lyg::svg_parse_kernel, dim3((L->n + 255) / 256), dim3(256), 0, s, *L);
+    if (L->by_wave) {
+        const dim3 grid((L->n - 1) / SVG_WAVES + 1), block(WAVE * SVG_WAVES);
+        if (L->n <= SVG_FEW) {
+            hipLaunchKernelGGL(svg_wave_kernel<true>, grid, block, 0, s, *L);
+            return hipGetLastError();
+        }
+        hipLaunchKernelGGL(svg_wave_kernel<false>, grid, block, 0, s, *L);
+    }
+    hipLaunchKernelGGL(svg_parse_kernel, dim3((L->n + 255) / 256), dim3(256), 0, s, *L);
     return hipGetLastError();
 }
 

@@ -152,6 +152,23 @@ def test_random_svg_matches_oracle(arcs):
     assert 0 < n_err < len(strings)
 
 
+@pytest.mark.parametrize("n", [1, 3, 5, 1023, 1024, 1025])
+def test_batch_sizes_around_a_launch_for_what_the_waves_leave(n):
+    """Up to 1,024 strings, one that its wave leaves is parsed by a lane of that wave, beyond by
+    a launch of their own: the same verbs, points and errors as in a batch of 1,500."""
+    rng = np.random.default_rng(23)
+    strings = [random_svg(rng, int(rng.integers(1, 40)), arcs=k % 3 == 0, corrupt=0.1)
+               for k in range(1500)]
+    ref, ref_errs = S.parse_paths(strings)
+    for first in (0, 1500 - n):
+        part, errs = S.parse_paths(strings[first:first + n])
+        for k in range(n):
+            a, b = part.path(k), ref.path(first + k)
+            assert _err(errs[k]) == _err(ref_errs[first + k])
+            assert np.array_equal(a.verbs, b.verbs)
+            assert np.array_equal(a.points, b.points, equal_nan=True)
+
+
 @pytest.mark.parametrize("length", [1, 63, 64, 65, 1000, 1023, 1024, 1025, 2048, 5000])
 def test_strings_around_what_a_wave_looks_at(length):
     """Well-formed strings (no arcs, no smooth quadratics, so that a wave parses each) whose
