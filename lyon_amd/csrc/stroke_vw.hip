@@ -527,16 +527,17 @@ __device__ __forceinline__ void curve_piece(Stroker& S, const VRec& r, bool b, b
 }  // namespace vw
 
 
-// One lane per path, the first L.paths_per_wave lanes of each one-wave block taking paths
-// (grid-stride): few paths per wave spread the serial walks over every SIMD and keep the
+// One lane per path, the first L.paths_per_wave lanes (of a list: as many as the grid needs) of
+// each one-wave block taking paths (grid-stride): few paths per wave spread the serial walks over every SIMD and keep the
 // lanes of a wave from waiting on each other's branches.  Counting (EMIT false) or writing
 // at the scanned offsets.
 template <bool EMIT>
 __global__ void __launch_bounds__(64) stroke_vw_kernel(StrokeVWLaunch L) {
     using namespace vw;
-    const uint32_t ppw = L.paths_per_wave;
-    if (threadIdx.x >= ppw) return;
     const uint32_t n_walk = L.list ? *L.n_list : L.in.n_paths;
+    uint32_t ppw = L.paths_per_wave;
+    if (L.list) ppw = min((uint32_t)WAVE, max(1u, (n_walk + gridDim.x - 1u) / gridDim.x));
+    if (threadIdx.x >= ppw) return;
     for (uint32_t k = blockIdx.x * ppw + threadIdx.x; k < n_walk; k += gridDim.x * ppw) {
         const uint32_t path = L.list ? L.list[k] : k;
         const lyg_stroke_options o = L.opts[L.opts_stride ? path : 0];
@@ -676,7 +677,7 @@ struct VX {  // per verb of a chunk: line_width * width factor at both ends, spl
 };
 
 __device__ __forceinline__ void mark_slow(const VWPar& P, uint32_t path) {
-    if (atomicExch(&P.path_mode[path], 1u) == 0u) P.slow_list[atomicAdd(&P.ctr[1], 1u)] = path;
+    P.path_mode[path] = 1u;
 }
 
 // One path's kept points.
@@ -916,12 +917,8 @@ __global__ void __launch_bounds__(64) vw_plan_kernel(VWPar P) {
             P.win_n[path] = run ? (uint32_t)((raw + WIN - 1) / WIN) : 0u;
             P.tail_n[path] = run ? ends : 0u;
             P.att_cap_n[path] = run ? 2u * corners : 0u;
-            P.path_mode[path] = run ? 0u : 2u;
+            P.path_mode[path] = run ? 0u : bad ? 1u : 2u;
             P.path_status[path] = bad || !space ? 0u : (uint32_t)LYG_ERR_NO_SPACE;
-            if (bad) {
-                P.path_mode[path] = 1u;
-                P.slow_list[atomicAdd(&P.ctr[1], 1u)] = path;
-            }
         }
     }
 }
@@ -1570,10 +1567,20 @@ __global__ void __launch_bounds__(64) vw_tail_kernel(VWPar P) {
     }
 }
 
-// Per path: its counts from its windows' offsets.
+// Per path: its counts from its windows' offsets, or its place in the list of those that the
+// serial kernel counts (a counter's addition per wave: one per path took 360 us of 30,000).
 __global__ void __launch_bounds__(256) vw_totals_kernel(VWPar P) {
-    for (uint32_t p = blockIdx.x * 256u + threadIdx.x; p < P.in.n_paths; p += gridDim.x * 256u) {
-        if (P.path_mode[p] == 1u) continue;  // the serial count follows
+    const uint32_t n = P.in.n_paths;
+    for (uint32_t p0 = blockIdx.x * 256u; p0 < n; p0 += gridDim.x * 256u) {
+        const uint32_t p = p0 + threadIdx.x;
+        const bool serial = p < n && P.path_mode[p] == 1u;
+        const uint64_t m = ballot(serial);
+        if (m) {
+            const uint32_t at =
+                readlane_u(atomicAdd(&P.ctr[1], lane_id() == 0 ? (uint32_t)__popcll(m) : 0u), 0);
+            if (serial) P.slow_list[at + (uint32_t)__popcll(m & mask_lt(lane_id()))] = p;
+        }
+        if (p >= n || serial) continue;
         const uint32_t a = P.win_off[p], b = P.win_off[p + 1];
         P.path_nv[p] = P.win_voff[b] - P.win_voff[a];
         P.path_ni[p] = 3u * (P.win_ioff[b] - P.win_ioff[a]);

@@ -173,8 +173,8 @@ int32_t stroke_vw_run(lyg_ctx* c, lyg::StrokeVWLaunch& L, bool want_attrs, uint3
     if (st == LYG_OK) st = vw_count(c, P, sh);
     if (st == LYG_ERR_DEVICE) return st;
     bool par = st == LYG_OK;
-    // The serial kernel over all paths: about six resident waves per SIMD (four SIMDs per
-    // CU), each with as few paths as fill them; over the paths left to it: one path a wave.
+    // The serial kernel, over all paths or those left to it: about six resident waves per SIMD
+    // (four SIMDs per CU), each with as few paths as fill them.
     const uint32_t slots = (uint32_t)std::max(1, c->cu_count) * 4u * 6u;
     int grid = 0;
     uint64_t* h = reinterpret_cast<uint64_t*>(c->h_pinned);
@@ -182,8 +182,8 @@ int32_t stroke_vw_run(lyg_ctx* c, lyg::StrokeVWLaunch& L, bool want_attrs, uint3
     for (;;) {
         L.list = par ? P.slow_list : nullptr;
         L.n_list = par ? P.ctr + 1 : nullptr;
-        L.paths_per_wave =
-            par ? 1u : std::min<uint32_t>(64u, std::max<uint32_t>(1u, (n + slots - 1) / slots));
+        L.paths_per_wave =  // of a list: by its length, in the kernel
+            std::min<uint32_t>(64u, std::max<uint32_t>(1u, (n + slots - 1) / slots));
         grid = par ? (int)std::min(n, slots)
                    : (int)std::min<uint32_t>((n + L.paths_per_wave - 1) / L.paths_per_wave,
                                              1u << 20);
