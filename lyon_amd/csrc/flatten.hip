@@ -370,9 +370,8 @@ __global__ void arc_to_quads_kernel(const float* arcs, uint32_t n, uint32_t* cou
 // ---- exclusive scan of u32 counts into n+1 offsets (single workgroup) -----------------
 // 1024 threads, each owning a contiguous slice; totals are carried in 64-bit and an
 // overflow of the 32-bit offsets is reported through `overflow`.
-__global__ void __launch_bounds__(1024) scan_offsets_kernel(const uint32_t* counts, uint32_t n,
-                                                            uint32_t* offsets, uint64_t* total,
-                                                            uint32_t* overflow) {
+__device__ __forceinline__ void scan_block(const uint32_t* counts, uint32_t n, uint32_t* offsets,
+                                           uint64_t* total, uint32_t* overflow) {
     __shared__ uint64_t part[1024];
     const uint32_t t = threadIdx.x;
     const uint32_t per = (n + 1023) / 1024;
@@ -400,6 +399,16 @@ __global__ void __launch_bounds__(1024) scan_offsets_kernel(const uint32_t* coun
         *total = part[1023];
     }
     if (ovf) atomicOr(overflow, 1u);
+}
+__global__ void __launch_bounds__(1024) scan_offsets_kernel(const uint32_t* counts, uint32_t n,
+                                                            uint32_t* offsets, uint64_t* total,
+                                                            uint32_t* overflow) {
+    scan_block(counts, n, offsets, total, overflow);
+}
+// Several scans at once, a block each.
+__global__ void __launch_bounds__(1024) scan_several_kernel(ScanJobs J) {
+    const ScanJob& j = J.job[blockIdx.x];
+    scan_block(j.counts, j.n, j.offsets, j.total, J.overflow);
 }
 
 // Large scans (n > SCAN_SMALL, lyg_launch_scan_tiles): three launches.  Tiles of SCAN_TILE counts (256 threads x
@@ -570,6 +579,10 @@ hipError_t lyg_launch_scan(const uint32_t* counts, uint32_t n, uint32_t* offsets
                            uint32_t* overflow, hipStream_t s) {
     hipLaunchKernelGGL(lyg::scan_offsets_kernel, dim3(1), dim3(1024), 0, s, counts, n, offsets,
                        total, overflow);
+    return hipGetLastError();
+}
+hipError_t lyg_launch_scan_several(const lyg::ScanJobs* J, hipStream_t s) {
+    hipLaunchKernelGGL(lyg::scan_several_kernel, dim3(J->n_jobs), dim3(1024), 0, s, *J);
     return hipGetLastError();
 }
 // Bytes of the `tiles` scratch lyg_launch_scan_tiles needs for n counts.

@@ -126,6 +126,19 @@ struct StrokeCompact {
     uint32_t* err;
 };
 
+// Exclusive scans launched together (scan_several_kernel).
+struct ScanJob {
+    const uint32_t* counts;
+    uint32_t n;
+    uint32_t* offsets;  // n + 1
+    uint64_t* total;
+};
+struct ScanJobs {
+    ScanJob job[4];
+    uint32_t n_jobs;
+    uint32_t* overflow;
+};
+
 namespace fillk {
 // Capacities of one wave's fill working arrays (events, heap, active edges, spans,
 // monotone nodes, pending edges).
@@ -269,8 +282,9 @@ struct VWPar {
     uint32_t *slow_list, *cands, *dirty;
     uint32_t cand_cap, dirty_cap;
     // [1] serial paths, [2] candidates, [3] windows to count
-    // again, [4] a list overflowed
+    // again, [4] a list overflowed, [5] some path has more than `few` points
     uint32_t* ctr;
+    uint32_t few;
     const uint32_t *vtx_off, *idx_off;
     float* out_vertices;
     uint32_t* out_indices;

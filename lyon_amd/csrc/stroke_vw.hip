@@ -918,6 +918,7 @@ __global__ void __launch_bounds__(64) vw_plan_kernel(VWPar P) {
             P.tail_n[path] = run ? ends : 0u;
             P.att_cap_n[path] = run ? 2u * corners : 0u;
             P.path_mode[path] = run ? 0u : bad ? 1u : 2u;
+            if (raw > P.few) P.ctr[5] = 1u;
             P.path_status[path] = bad || !space ? 0u : (uint32_t)LYG_ERR_NO_SPACE;
         }
     }

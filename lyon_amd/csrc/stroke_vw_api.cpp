@@ -17,12 +17,29 @@ hipError_t lyg_launch_vw_count(const lyg::VWPar* P, int grid_paths, int grid_win
 hipError_t lyg_launch_vw_totals(const lyg::VWPar* P, hipStream_t s);
 hipError_t lyg_launch_vw_emit(const lyg::VWPar* P, int grid_win, uint32_t chunk, hipStream_t s);
 hipError_t lyg_launch_fill_u32(uint32_t* p, uint32_t n, uint32_t v, hipStream_t s);
+hipError_t lyg_launch_scan_several(const lyg::ScanJobs* J, hipStream_t s);
 }
 
 namespace {
 
 bool valid_opts(const lyg_stroke_options& o) {
     return o.start_cap <= 2 && o.end_cap <= 2 && o.line_join <= 3;
+}
+
+// Scans of up to 32,768 counts each in one launch, a block each; longer ones one by one.
+bool scans(lyg_ctx* c, std::initializer_list<lyg::ScanJob> jobs, uint32_t* overflow) {
+    lyg::ScanJobs J{};
+    J.overflow = overflow;
+    bool small = true;
+    for (const lyg::ScanJob& j : jobs) {
+        J.job[J.n_jobs++] = j;
+        small = small && j.n <= 32768;
+    }
+    if (small) return check(c, lyg_launch_scan_several(&J, c->stream), "scans");
+    for (const lyg::ScanJob& j : jobs)
+        if (!check(c, ctx_scan(c, j.counts, j.n, j.offsets, j.total, overflow, c->stream), "scan"))
+            return false;
+    return true;
 }
 
 // Launch shape of the window kernels.
@@ -35,8 +52,17 @@ struct VWShape {
 // bytes per flattened point, the output takes about 40).
 constexpr uint64_t VW_MAX_POINTS = 1ull << 30;
 
+// Paths of no more points are sooner walked by a lane each (13 us a point) than by the parallel
+// form's launches, while every path has a wave: plain calls of 1 / 3 / 10 lines 168 187 279 us
+// against 220 to 250.
+constexpr uint32_t VW_FEW = 5;
+
+// About six resident waves per SIMD (four SIMDs per CU) of the serial kernel.
+uint32_t serial_slots(const lyg_ctx* c) { return (uint32_t)std::max(1, c->cu_count) * 4u * 6u; }
+
 // The plan and the parallel form's memory.  LYG_ERR_NO_SPACE: the batch goes to the serial
-// kernel (too many points, or no device memory for them).
+// kernel (too many points, or no device memory for them; no path for the parallel form; few
+// short paths).
 int32_t vw_plan(lyg_ctx* c, const lyg::StrokeVWLaunch& L, uint32_t n, bool want_attrs,
                 lyg::VWPar* out, VWShape* sh) {
     hipStream_t s = c->stream;
@@ -62,6 +88,7 @@ int32_t vw_plan(lyg_ctx* c, const lyg::StrokeVWLaunch& L, uint32_t n, bool want_
         u += k;
         return p;
     };
+    P.few = VW_FEW;
     P.ctr = take(16);
     P.raw_n = take(n);
     P.win_n = take(n);
@@ -76,18 +103,21 @@ int32_t vw_plan(lyg_ctx* c, const lyg::StrokeVWLaunch& L, uint32_t n, bool want_
     P.win_off = off[1];
     P.tail_off = off[2];
     P.att_off = off[3];
-    const uint32_t* cnt[4] = {P.raw_n, P.win_n, P.tail_n, P.att_cap_n};
     sh->grid_paths = (int)std::min<uint32_t>(n, (uint32_t)std::max(1, c->cu_count) * 32u);
     if (!check(c, lyg_launch_fill_u32(P.ctr, 16, 0, s), "reset") ||
-        !check(c, lyg_launch_vw_plan(&P, sh->grid_paths, s), "stroke vw plan"))
+        !check(c, lyg_launch_vw_plan(&P, sh->grid_paths, s), "stroke vw plan") ||
+        !scans(c, {{P.raw_n, n, off[0], c->d_totals + 2}, {P.win_n, n, off[1], c->d_totals + 3},
+                   {P.tail_n, n, off[2], c->d_totals + 4},
+                   {P.att_cap_n, n, off[3], c->d_totals + 5}}, P.ctr + 8))
         return LYG_ERR_DEVICE;
-    for (int k = 0; k < 4; ++k)
-        if (!check(c, ctx_scan(c, cnt[k], n, off[k], c->d_totals + 2 + k, P.ctr + 8, s), "scan"))
-            return LYG_ERR_DEVICE;
     uint64_t* h = reinterpret_cast<uint64_t*>(c->h_pinned);
+    h[4] = 1;
     if (!check(c, hipMemcpyAsync(h, c->d_totals + 2, 32, hipMemcpyDeviceToHost, s), "D2H") ||
+        (n <= serial_slots(c) &&
+         !check(c, hipMemcpyAsync(h + 4, P.ctr + 5, 4, hipMemcpyDeviceToHost, s), "D2H")) ||
         !check(c, hipStreamSynchronize(s), "sync"))
         return LYG_ERR_DEVICE;
+    if (h[0] == 0 || (uint32_t)h[4] == 0) return LYG_ERR_NO_SPACE;
     const uint64_t raw = h[0], win = h[1], tails = h[2], att = h[3];
     if (raw > VW_MAX_POINTS || tails > VW_MAX_POINTS || att > VW_MAX_POINTS)
         return LYG_ERR_NO_SPACE;
@@ -143,19 +173,19 @@ int32_t vw_count(lyg_ctx* c, lyg::VWPar& P, const VWShape& sh) {
     uint32_t* wi = const_cast<uint32_t*>(P.win_ioff);
     if (!check(c, lyg_launch_vw_count(&P, sh.grid_paths, sh.grid, sh.chunk, s),
                "stroke vw count") ||
-        !check(c, ctx_scan(c, P.win_nv, P.n_windows, wv, c->d_totals + 6, P.ctr + 8, s), "scan") ||
-        !check(c, ctx_scan(c, P.win_ni, P.n_windows, wi, c->d_totals + 7, P.ctr + 8, s), "scan") ||
+        !scans(c, {{P.win_nv, P.n_windows, wv, c->d_totals + 6},
+                   {P.win_ni, P.n_windows, wi, c->d_totals + 7}}, P.ctr + 8) ||
         !check(c, lyg_launch_vw_totals(&P, s), "stroke vw totals"))
         return LYG_ERR_DEVICE;
     return LYG_OK;
 }
 
-// Runs the batch `L` (inputs, options, widths set); offsets go to vtx_off / idx_off (n + 1
+// Runs the batch `L` (inputs, options, widths set), `serial`: without the plan; offsets go to vtx_off / idx_off (n + 1
 // each), per-path statuses to c->f_status; want_attrs: vertex attributes will be asked for
 // (L.out_attrs is set by then); `alloc` sets the output arrays once the totals
 // are known.
-int32_t stroke_vw_run(lyg_ctx* c, lyg::StrokeVWLaunch& L, bool want_attrs, uint32_t* vtx_off,
-                      uint32_t* idx_off, uint32_t vertex_offset, const lygi::OutAlloc& alloc,
+int32_t stroke_vw_run(lyg_ctx* c, lyg::StrokeVWLaunch& L, bool serial, bool want_attrs,
+                      uint32_t* vtx_off, uint32_t* idx_off, uint32_t vertex_offset, const lygi::OutAlloc& alloc,
                       uint64_t* tv, uint64_t* ti, std::vector<uint32_t>* status) {
     const uint32_t n = L.in.n_paths;
     hipStream_t s = c->stream;
@@ -169,13 +199,13 @@ int32_t stroke_vw_run(lyg_ctx* c, lyg::StrokeVWLaunch& L, bool want_attrs, uint3
     L.err = c->d_counters + 5;
     lyg::VWPar P{};
     VWShape sh{};
-    int32_t st = c->vw_serial ? (int32_t)LYG_ERR_NO_SPACE : vw_plan(c, L, n, want_attrs, &P, &sh);
+    int32_t st = serial || c->vw_serial ? (int32_t)LYG_ERR_NO_SPACE
+                                        : vw_plan(c, L, n, want_attrs, &P, &sh);
     if (st == LYG_OK) st = vw_count(c, P, sh);
     if (st == LYG_ERR_DEVICE) return st;
     bool par = st == LYG_OK;
-    // The serial kernel, over all paths or those left to it: about six resident waves per SIMD
-    // (four SIMDs per CU), each with as few paths as fill them.
-    const uint32_t slots = (uint32_t)std::max(1, c->cu_count) * 4u * 6u;
+    // the serial kernel, over all paths or those left to it: its waves take as few as fill them
+    const uint32_t slots = serial_slots(c);
     int grid = 0;
     uint64_t* h = reinterpret_cast<uint64_t*>(c->h_pinned);
     status->assign(n, 0);
@@ -191,10 +221,8 @@ int32_t stroke_vw_run(lyg_ctx* c, lyg::StrokeVWLaunch& L, bool want_attrs, uint3
         uint32_t* went = reinterpret_cast<uint32_t*>(h + 3);
         if (!check(c, lyg_launch_fill_u32(c->d_counters + 4, 2, 0, s), "reset") ||
             !check(c, lyg_launch_stroke_vw(&L, 0, grid, s), "stroke vw count") ||
-            !check(c, ctx_scan(c, L.path_nv, n, vtx_off, c->d_totals + 0, c->d_counters + 4, s),
-                   "scan") ||
-            !check(c, ctx_scan(c, L.path_ni, n, idx_off, c->d_totals + 1, c->d_counters + 4, s),
-                   "scan") ||
+            !scans(c, {{L.path_nv, n, vtx_off, c->d_totals + 0},
+                       {L.path_ni, n, idx_off, c->d_totals + 1}}, c->d_counters + 4) ||
             !check(c, hipMemcpyAsync(h, c->d_totals, 16, hipMemcpyDeviceToHost, s), "D2H") ||
             !check(c, hipMemcpyAsync(h + 2, c->d_counters + 4, 4, hipMemcpyDeviceToHost, s),
                    "D2H") ||
@@ -292,7 +320,8 @@ int32_t lyg_stroke_batch_vw(lyg_ctx* c, const lyg_batch_in* in, const float* att
     uint64_t tv = 0, ti = 0;
     std::vector<uint32_t> status;
     int32_t st = stroke_vw_run(
-        c, L, out_attributes != nullptr, out->path_vertex_offsets, out->path_index_offsets, out->vertex_offset,
+        c, L, false, out_attributes != nullptr, out->path_vertex_offsets, out->path_index_offsets,
+        out->vertex_offset,
         [&](uint64_t nv, uint64_t ni, float** v, uint32_t** i) -> int32_t {
             if (nv > out->vertex_capacity || ni > out->index_capacity) return LYG_ERR_CAPACITY;
             *v = out->vertices;
@@ -359,8 +388,16 @@ int32_t lyg_stroke_path_vw(lyg_ctx* c, const lyg_path_view* path, const float* a
     L.n_attrs = n_attributes;
     uint64_t tv = 0, ti = 0;
     std::vector<uint32_t> status;
+    // a clipped miter join, or a few lines
+    const bool serial =
+        opts->line_join == LYG_JOIN_MITER_CLIP ||
+        (path->n_points <= VW_FEW &&
+         std::none_of(path->verbs, path->verbs + path->n_verbs, [](uint8_t v) {
+             return v == LYG_VERB_QUADRATIC || v == LYG_VERB_CUBIC;
+         }));
     int32_t st = stroke_vw_run(
-        c, L, out_attributes != nullptr, as<uint32_t>(c->offs_v), as<uint32_t>(c->offs_i), out->vertex_offset,
+        c, L, serial, out_attributes != nullptr, as<uint32_t>(c->offs_v), as<uint32_t>(c->offs_i),
+        out->vertex_offset,
         [&](uint64_t nv, uint64_t ni, float** v, uint32_t** i) -> int32_t {
             if (nv > out->vertex_capacity || ni > out->index_capacity) {
                 out->n_vertices = (uint32_t)nv;

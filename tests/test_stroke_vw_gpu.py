@@ -381,6 +381,35 @@ def test_the_two_forms_agree(seed):
     assert serial < n
 
 
+@pytest.mark.parametrize("points,all_serial", [((1, 2, 3, 4, 5), True), ((2, 5, 6), False),
+                                               ((6, 7), False)])
+@pytest.mark.parametrize("join", [LineJoin.Miter, LineJoin.MiterClip])
+def test_short_paths_around_where_the_parallel_form_starts(points, all_serial, join):
+    """Batches of a few paths of at most five points, or of clipped miters alone, are walked by
+    the serial kernel; one path of six points brings the parallel form.  Plain calls of the same
+    paths match the oracle."""
+    rng = np.random.default_rng(len(points))
+    paths = []
+    for k in points * 4:
+        b = PathBuilder(1)
+        pts = rng.uniform(0, 50, (k, 2)).round(1)
+        b.begin(tuple(pts[0]), [rng.uniform(0.5, 2)])
+        for q in pts[1:]:
+            b.line_to(tuple(q), [rng.uniform(0.5, 2)])
+        b.end(len(paths) % 2 == 0)
+        paths.append(b.build())
+    o = vw_options(len(paths), rng, 1.0, 0.1)
+    o["line_join"] = int(join)
+    serial, _ = forms(paths, o)
+    assert serial == (len(paths) if all_serial or join == LineJoin.MiterClip else 0)
+    for path in paths:
+        opts = StrokeOptions(line_width=1.0, line_join=join, start_cap=LineCap.Round,
+                             end_cap=LineCap.Square, tolerance=0.1, variable_line_width=0)
+        v, i = gpu_vw(path, opts)
+        rv, ri = ref_vw(path, opts)
+        assert np.array_equal(i, ri) and close_enough(v, rv, 50.0)
+
+
 def turns(rng, at, heading, lengths, most):
     """Points one after the other from `at`, each at a turn of up to `most`; the last heading."""
     out = []
