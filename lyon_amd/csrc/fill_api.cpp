@@ -174,12 +174,14 @@ struct RoundPlan {
 };
 
 // Plans round `round` over the paths `todo`, with `scale` times the first round's room;
-// arrays[p]: the path has met a limit of every register launch.  A captured graph has no second round: there every register launch is followed by a sweep over
-// arrays of the paths that outgrew it.  registers false: every path goes over arrays (no log).
+// arrays[p]: the path has met a limit of every register launch; registers false: every path
+// goes over arrays (no log).  A captured graph has no second round: there every register launch
+// is followed by a sweep over arrays of the paths that outgrew it.
 int32_t plan_round(lyg_ctx* c, const std::vector<uint32_t>& todo,
                    const std::vector<uint32_t>& bound, const std::vector<uint32_t>& degree,
                    const std::vector<uint32_t>& inter, const std::vector<uint64_t>& need,
-                   const std::vector<uint8_t>& arrays, int round, uint64_t scale, bool registers, bool graph, RoundPlan* P) {
+                   const std::vector<uint8_t>& arrays, int round, uint64_t scale, bool registers,
+                   bool graph, RoundPlan* P) {
     // the register sweep's log takes 52 bytes per staged triangle
     uint64_t all_v = 0, all_t = 0;
     for (uint32_t p : todo) {
